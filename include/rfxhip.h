@@ -217,8 +217,19 @@ int rfxh_kernel_time_ms(rfxh_plan* plan, int which, double* avg_ms, int64_t* cou
  * param = x segments, 0 = automatic; at most 1024 material ids and 4 DFT
  * planes, no flux monitors, NTFF boxes or dispersion; an odd last step of
  * a run takes the two-pass kernels; rfxh_kernel_time_ms which = 0 is then
- * the two-step sweep).  Kernels 1-3, 7 and 8 need the second field set.
- * Variants compute the same step; they differ in speed only.  The
+ * the two-step sweep); 9: the resident step, a whole run in one
+ * launch with the state in registers (param = 0; in place, either field
+ * set; grids cut into at most one block per compute unit, about a million
+ * cells, no dispersion or per-component eps, at most 32 planes, monitors
+ * and NTFF faces in all and 256 point operations a block).  It is the
+ * default of every plan that fits; runs of fewer than 4 steps, timed runs
+ * and runs on a stream under capture take the two-pass step instead.  Its
+ * first run allocates its workspace (up to 100 MB, kept by the plan).  Such
+ * launches run one at a time on a device, in the order of the calls; while
+ * another process holds the device for them, runs take the two-pass step.
+ * Kernels 1-3, 7 and 8 need the second field set.
+ * Variants compute the same step; they differ in speed only (9 is 4 and 0
+ * bit for bit).  The
  * project's autotuner (rfx_amd/autotune.py) times them on the actual
  * problem.  No counterpart in the reference (its XLA lowering has no
  * kernel choice). */

@@ -54,7 +54,7 @@ def variants(dr):
         out += [(kern, order) for order in (1, 0)]
     nx = dr.prob.shape[0]
     if len(dr.sets) == 2:
-        out += [(1, 1), (1, 0)]
+        out += [(9, 0), (1, 1), (1, 0)]
         # the wave-march and temporal-blocked steps stage the material table
         # in LDS (at most 1024 ids)
         small = len(dr.flags) <= 1024
@@ -73,6 +73,8 @@ ORDERED = {0: "two-pass", 1: "fused", 4: "col2", 5: "col4", 6: "col3"}
 def variant_name(v) -> str:
     """two-pass-flat, col2-bands, col3-flat, fused-flat, march14-16, wmarch-8, ..."""
     k, prm = v
+    if k == 9:
+        return "resident"
     if k == 8:
         return "tb2" if prm == 0 else f"tb2-{prm}"
     if k == 7:
@@ -84,6 +86,8 @@ def variant_name(v) -> str:
 
 
 def parse_variant(name: str):
+    if name == "resident":
+        return (9, 0)
     if name.startswith("tb2"):
         _, _, seg = name.partition("-")
         return (8, int(seg) if seg else 0)
@@ -128,7 +132,7 @@ def autotune(dr, trial_steps: int = 32, repeats: int = 2, cache_file: str | None
     steps = max(1, min(int(trial_steps), dr.n_steps))
     stream = torch.cuda.current_stream(dr.device)
     timings = {}
-    for v in variants(dr):
+    for v in dict.fromkeys([(9, 0)] + variants(dr)):
         try:
             set_variant(dr, *v)
         except _lib.RfxHipError:

@@ -30,6 +30,9 @@
 // hipGraph of a chunk of steps is replayed for every chunk.
 
 #include <hip/hip_runtime.h>
+#include <sys/socket.h>
+#include <sys/un.h>
+#include <unistd.h>
 
 #include <algorithm>
 #include <cmath>
@@ -2233,6 +2236,8 @@ __global__ __launch_bounds__(256) void k_flux_flush(FluxParams q) {
   flux_fold(q, (int)blockIdx.y, pidx, npts, lo, last, false, 0.f);
 }
 
+#include "resident.h"
+
 // ---------------------------------------------------------------------------
 // Near-to-far-field transform: one thread per (direction, frequency).  The
 // face cells stream through LDS in chunks of kFFBlock, each staged once per
@@ -3607,6 +3612,22 @@ __global__ void k_advance2(long long* step) {
 
 }  // namespace
 
+// The resident step of a plan: how the grid is cut into blocks, and its
+// workspace (allocated by the first run that takes it, kept until the plan
+// ends).
+struct ResPlan {
+  bool ok = false;
+  int nx = 0, ty = 0, tz = 0, ntx = 0, nty = 0, ntz = 0, threads = 0;
+  long long chunk = 0;            // steps of one launch
+  int dev = -1;                   // the device its workspace is on (-1: none yet)
+  u64* box = nullptr;
+  unsigned* stop = nullptr;
+  ResSnap* snaps = nullptr;
+  KParams* kp = nullptr;          // device copy of the plan's parameters
+  std::vector<float*> rings;      // staging ring of each DFT plane, then of each flux entry
+  unsigned tag = 0;               // tags handed out so far
+};
+
 struct rfxh_plan {
   KParams kp;
   // Debye / Lorentz polarisation state (caller-owned) and per-material pole coefficients
@@ -3627,6 +3648,8 @@ struct rfxh_plan {
   bool tb = false;              // two steps per sweep (temporal-blocked march), ping-pong
   int tb_seg = 0;               // its x segments (0: automatic)
   int tb_ops_max = 0;           // most point operations in one of its tile columns
+  ResPlan rp;                   // the resident step's blocks (rp.ok: the plan can take it)
+  bool res = false;             // runs take the resident step where they can
   float* psi_base = nullptr;    // CPML memory of set 0 (set 1 at + psi_set)
   float* psi_mid = nullptr;     // the sweep's memory after its first step (owned, same layout)
   long long psi_floats = 0;
@@ -4023,6 +4046,293 @@ int launch_tb(rfxh_plan* pl, hipStream_t s, hipEvent_t* ev, int from) {
   hipLaunchKernelGGL(k_advance2, dim3(1), dim3(64), 0, s, kp.step);
   HIPCHK(hipGetLastError());
   return 0;
+}
+
+// ---- resident step (host side) ----------------------------------------------
+
+constexpr int kResNX[] = {1, 2, 3, 4, 6, 8};
+
+const void* res_kernel(bool graded, int nx) {
+  switch (nx) {
+    case 1: return graded ? (const void*)k_resident<true, 1> : (const void*)k_resident<false, 1>;
+    case 2: return graded ? (const void*)k_resident<true, 2> : (const void*)k_resident<false, 2>;
+    case 3: return graded ? (const void*)k_resident<true, 3> : (const void*)k_resident<false, 3>;
+    case 4: return graded ? (const void*)k_resident<true, 4> : (const void*)k_resident<false, 4>;
+    case 6: return graded ? (const void*)k_resident<true, 6> : (const void*)k_resident<false, 6>;
+    default: return graded ? (const void*)k_resident<true, 8> : (const void*)k_resident<false, 8>;
+  }
+}
+
+// The workgroups of a resident launch wait for one another, so two such
+// launches must never share a device: each could hold half its compute units
+// for ever.  Within the process every launch waits for the device's previous
+// one (an event, whatever the streams); between processes the first one to
+// take the device's name (an abstract socket address, freed by the kernel
+// when its holder ends) keeps it while it has plans with a resident
+// workspace, and the plans of the others take the two-pass step.
+// hipLaunchCooperativeKernel would order them too, but streams created after
+// its first use ran 1.7 times slower (a 222 x 164 x 140 step 127 us instead of
+// 74), and each of its launches took 20 us instead of 4.
+struct ResDevice {
+  std::mutex mu;
+  hipEvent_t last = nullptr;   // the device's latest resident launch
+  int holders = 0;             // plans of this process with a workspace on it
+  int sock = -1;
+};
+constexpr int kResDevices = 64;
+ResDevice g_res_dev[kResDevices];
+
+bool res_hold(int dev) {
+  if (dev < 0 || dev >= kResDevices) return false;
+  ResDevice& d = g_res_dev[dev];
+  std::lock_guard<std::mutex> lock(d.mu);
+  if (d.holders == 0) {
+    char bus[64] = "";
+    if (hipDeviceGetPCIBusId(bus, sizeof(bus), dev) != hipSuccess) {
+      (void)hipGetLastError();
+      return false;
+    }
+    sockaddr_un a;
+    std::memset(&a, 0, sizeof(a));
+    a.sun_family = AF_UNIX;   // sun_path[0] = 0: an abstract name, no file
+    const int len = std::snprintf(a.sun_path + 1, sizeof(a.sun_path) - 1, "rfxhip-resident-%s", bus);
+    d.sock = socket(AF_UNIX, SOCK_DGRAM | SOCK_CLOEXEC, 0);
+    if (d.sock < 0) return false;
+    if (bind(d.sock, reinterpret_cast<sockaddr*>(&a),
+             (socklen_t)(offsetof(sockaddr_un, sun_path) + 1 + len)) != 0 ||
+        (!d.last && hipEventCreateWithFlags(&d.last, hipEventDisableTiming) != hipSuccess)) {
+      (void)hipGetLastError();
+      close(d.sock);
+      d.sock = -1;
+      return false;
+    }
+  }
+  ++d.holders;
+  return true;
+}
+
+void res_release(int dev) {
+  ResDevice& d = g_res_dev[dev];
+  std::lock_guard<std::mutex> lock(d.mu);
+  if (--d.holders > 0) return;
+  // its last launch has ended: the plan's memory is being freed
+  close(d.sock);
+  d.sock = -1;
+}
+
+// Cuts the grid into at most one block per compute unit, the cheapest cut by
+// a model of the step (microseconds): two exchanges, 0.55 + 0.65 per
+// thousand words of a workgroup, and 0.12 per plane and wavefront of a SIMD
+// (about 75 vector and LDS instructions a cell in each half).  Plans it does
+// not cover keep rp.ok false: dispersive poles and per-component eps, CPML
+// slabs that overlap, more snapshots or point operations in a block than it
+// stages, grids of more blocks than compute units.
+void res_choose(rfxh_plan* pl, const std::vector<rfxh_point_op>& ops) {
+  ResPlan& r = pl->rp;
+  const KParams& kp = pl->kp;
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    return;
+  const long long cells = (long long)kp.nx * kp.plane;
+  if (pl->n_pole > 0 || pl->aniso || cells > (long long)cus * 8 * kResThreads) return;
+  if (pl->planes.size() + pl->fluxes.size() > (size_t)kResSnaps) return;
+  const int N[3] = {kp.nx, kp.ny, kp.nz};
+  for (int a = 0; a < 3; ++a)
+    if (kp.cn[2 * a] + kp.cn[2 * a + 1] > N[a]) return;
+  if ((long long)pl->psi_foff[5] + 4LL * pl->psi_fs[5] >= (1LL << 30)) return;
+  double best = 1e30;
+  for (int nx : kResNX) {
+    const int ntx = (kp.nx + nx - 1) / nx;
+    if (ntx > cus) continue;
+    for (int ntz = 1; ntz <= cus / ntx; ++ntz) {
+      const int tz = (kp.nz + ntz - 1) / ntz;
+      if (tz > kResThreads || (ntz > 1 && (kp.nz + tz - 1) / tz != ntz)) continue;
+      for (int nty = 1; nty <= cus / (ntx * ntz); ++nty) {
+        const int ty = (kp.ny + nty - 1) / nty;
+        if (nty > 1 && (kp.ny + ty - 1) / ty != nty) continue;
+        if (ty * tz > kResThreads || (ty + 1) * (tz + 1) > kResPS || ty + tz > kResEdge) continue;
+        const int threads = std::max(kResOps, (ty * tz + 63) / 64 * 64);
+        const int words = 2 * ty * tz + 2 * nx * (ty + tz);
+        if (2 * nx * (ty + tz) > kResWords * threads) continue;
+        const double t = 2 * (0.55 + 0.65e-3 * words) + nx * std::max(0.1, 0.12 * threads / 256);
+        if (t >= best) continue;
+        best = t;
+        r.nx = nx;
+        r.ty = ty;
+        r.tz = tz;
+        r.ntx = ntx;
+        r.nty = nty;
+        r.ntz = ntz;
+        r.threads = threads;
+      }
+    }
+  }
+  if (best > 1e29) return;
+  if ((int)ops.size() > kResOps) {
+    std::map<long long, int> cnt;
+    for (const rfxh_point_op& op : ops) {
+      const int i = (int)(op.cell / kp.plane), f = (int)(op.cell % kp.plane);
+      const long long t = ((long long)(i / r.nx) * r.nty + f / kp.nz / r.ty) * r.ntz +
+                          f % kp.nz / r.tz;
+      if (++cnt[t] > kResOps) return;
+    }
+  }
+  r.ok = true;
+}
+
+// Allocates the mailboxes and staging rings; 1: the device has no room or
+// another process holds it (the caller takes the other step kernels).
+int res_setup(rfxh_plan* pl, hipStream_t s) {
+  ResPlan& r = pl->rp;
+  const long long n_box = 4LL * r.ntx * r.nty * r.ntz * res_words(r.nx);
+  long long per_step = 0;
+  for (const PlaneParams& q : pl->planes) per_step += 4LL * q.n1 * q.n2;
+  for (const FluxParams& q : pl->fluxes) per_step += 16LL * q.n1 * q.n2;
+  // rings of about 64 MiB in all: a launch's fixed cost (about 10 us) is
+  // then a few percent of its steps
+  r.chunk = per_step ? std::min<long long>(4096, std::max<long long>(16, (64LL << 20) / per_step))
+                     : (1LL << 20);
+  const long long rows = std::min<long long>(r.chunk, std::max<long long>(1, pl->max_steps));
+  const long long ring = per_step / 4 * rows;
+  const size_t n_snap = pl->planes.size() + pl->fluxes.size();
+  int dev = 0;
+  HIPCHK(hipGetDevice(&dev));
+  if (!res_hold(dev)) return 1;
+  r.dev = dev;
+  char* base = nullptr;
+  const size_t bytes = n_box * sizeof(u64) + 256 + ring * sizeof(float);
+  if (hipMalloc(&base, bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    return 1;
+  }
+  pl->owned.push_back(base);
+  HIPCHK(hipMemsetAsync(base, 0, n_box * sizeof(u64) + 256, s));
+  r.box = reinterpret_cast<u64*>(base);
+  r.stop = reinterpret_cast<unsigned*>(base + n_box * sizeof(u64));
+  float* at = reinterpret_cast<float*>(base + n_box * sizeof(u64) + 256);
+  std::vector<ResSnap> snaps;
+  for (size_t q = 0; q < n_snap; ++q) {
+    ResSnap sn;
+    std::memset(&sn, 0, sizeof(sn));
+    if (q < pl->planes.size()) {
+      const PlaneParams& pp = pl->planes[q];
+      sn.axis = pp.axis;
+      sn.index = pp.index;
+      sn.hi1 = pp.n1;
+      sn.hi2 = pp.n2;
+      sn.ncomp = 1;
+      sn.comp[0] = pl->plane_comp[q];
+      sn.n2 = pp.n2;
+      sn.npts = (long long)pp.n1 * pp.n2;
+    } else {
+      const size_t u = q - pl->planes.size();
+      const FluxParams& fp = pl->fluxes[u];
+      sn.axis = fp.axis;
+      sn.index = fp.index;
+      sn.lo1 = fp.lo1;
+      sn.hi1 = fp.lo1 + fp.n1;
+      sn.lo2 = fp.lo2;
+      sn.hi2 = fp.lo2 + fp.n2;
+      sn.ncomp = 4;
+      for (int t = 0; t < 4; ++t) sn.comp[t] = pl->flux_comp[4 * u + t];
+      sn.avg = fp.index_m1 != fp.index;
+      sn.n2 = fp.n2;
+      sn.npts = (long long)fp.n1 * fp.n2;
+    }
+    sn.out = at;
+    r.rings.push_back(at);
+    at += sn.npts * sn.ncomp * rows;
+    snaps.push_back(sn);
+  }
+  r.chunk = rows;
+  if (int rc = dev_copy(pl, &pl->kp, 1, &r.kp)) return rc;
+  if (n_snap) {
+    const int rc = dev_copy(pl, snaps.data(), snaps.size(), &r.snaps);
+    if (rc) return rc;
+  }
+  return 0;
+}
+
+// n_steps steps from step0 in place on the current set: launches of at most
+// rp.chunk steps, each followed by the folds of what it staged.
+int run_resident(rfxh_plan* pl, hipStream_t s, int64_t step0, int64_t n_steps) {
+  ResPlan& r = pl->rp;
+  const KParams& kp = pl->kp;
+  ResIO io;
+  std::memset(&io, 0, sizeof(io));
+  for (int c = 0; c < 6; ++c) io.f[c] = pl->set[pl->cur][c];
+  io.psi = pl->psi_base ? pl->psi_base + pl->cur * pl->psi_set : nullptr;
+  for (int f = 0; f < 6; ++f) {
+    io.foff[f] = pl->psi_foff[f];
+    io.fs[f] = pl->psi_fs[f];
+  }
+  io.box = r.box;
+  io.stop = r.stop;
+  io.snaps = r.snaps;
+  io.n_snap = (int)r.rings.size();
+  io.ty = r.ty;
+  io.tz = r.tz;
+  io.ntx = r.ntx;
+  io.nty = r.nty;
+  io.ntz = r.ntz;
+  const dim3 grid((unsigned)(r.ntx * r.nty * r.ntz)), blk((unsigned)r.threads);
+  for (int64_t done = 0; done < n_steps;) {
+    const int cnt = (int)std::min<int64_t>(r.chunk, n_steps - done);
+    io.n_steps = cnt;
+    io.step0 = step0 + done;
+    if (r.tag > 0xffffffffu - 2u * (unsigned)cnt - 2u) {
+      // the tags are used up: start them again over cleared mailboxes
+      HIPCHK(hipMemsetAsync(r.box, 0, 4LL * grid.x * res_words(r.nx) * sizeof(u64), s));
+      r.tag = 0;
+    }
+    io.tag0 = r.tag;
+    r.tag += 2u * (unsigned)cnt;
+    void* args[] = {&r.kp, &io};
+    {
+      ResDevice& d = g_res_dev[r.dev];
+      std::lock_guard<std::mutex> lock(d.mu);
+      HIPCHK(hipStreamWaitEvent(s, d.last, 0));
+      HIPCHK(hipLaunchKernel(res_kernel(kp.graded != 0, r.nx), grid, blk, args, 0, s));
+      HIPCHK(hipEventRecord(d.last, s));
+    }
+    for (size_t q = 0; q < r.rings.size(); ++q) {
+      const bool plane = q < pl->planes.size();
+      const size_t u = q - (plane ? 0 : pl->planes.size());
+      const long long npts = plane ? (long long)pl->planes[u].n1 * pl->planes[u].n2
+                                   : (long long)pl->fluxes[u].n1 * pl->fluxes[u].n2;
+      const int nf = plane ? pl->planes[u].nf : pl->fluxes[u].nf, ncomp = plane ? 1 : 4;
+      const dim3 g((unsigned)((npts + 255) / 256), (unsigned)ncomp,
+                   (unsigned)((nf + kFoldF - 1) / kFoldF));
+      if (plane) {
+        const PlaneParams& pp = pl->planes[u];
+        hipLaunchKernelGGL(k_res_fold, g, dim3(256), 0, s, r.rings[q], ncomp, npts, pp.tw, pp.tw,
+                           pp.acc, nf, (long long)(step0 + done), cnt);
+      } else {
+        const FluxParams& fp = pl->fluxes[u];
+        hipLaunchKernelGGL(k_res_fold, g, dim3(256), 0, s, r.rings[q], ncomp, npts, fp.twe, fp.twh,
+                           fp.acc, nf, (long long)(step0 + done), cnt);
+      }
+    }
+    done += cnt;
+  }
+  HIPCHK(hipGetLastError());
+  return 0;
+}
+
+// Whether a run of n_steps takes the resident step: not while its stream is
+// being captured (the launch's order with other streams and a first
+// run's allocation do not belong in a graph) or single steps are being timed, and not for a handful
+// of steps, which the launch's fixed cost (the state's way in and out)
+// outweighs.
+bool res_takes(rfxh_plan* pl, hipStream_t s, int64_t n_steps) {
+  if (!pl->res || !pl->rp.ok || pl->timing || n_steps < 4) return false;
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return st == hipStreamCaptureStatusNone;
 }
 
 // Launch grid of the plan's workgroup order.
@@ -4489,6 +4799,9 @@ int rfxh_plan_create(const rfxh_desc* d, rfxh_plan** out) {
   const char* ord = std::getenv("RFXH_ORDER");
   kp.order = (ord && std::string(ord) == "bands") ? 0 : 1;
   if ((rc = plan_grid(pl))) return bail(rc);
+  res_choose(pl, ops);
+  // the default of every grid that fits: 3-6 times the two-pass step's speed
+  pl->res = pl->rp.ok && kname.empty();
   pl->tev.resize(4 * kTimingSamples);
   for (auto& e : pl->tev) {
     if (hipEventCreate(&e) != hipSuccess) return bail(fail(RFXH_EHIP, "hipEventCreate"));
@@ -4507,6 +4820,7 @@ int rfxh_plan_destroy(rfxh_plan* pl) {
   for (auto e : pl->tev)
     if (e) (void)hipEventDestroy(e);
   for (void* p : pl->owned) (void)hipFree(p);
+  if (pl->rp.dev >= 0) res_release(pl->rp.dev);
   delete pl;
   return RFXH_OK;
 }
@@ -4619,6 +4933,12 @@ int rfxh_run(rfxh_plan* pl, int64_t step0, int64_t n_steps, void* stream, int us
   dft_begin(pl, s, step0);
   HIPCHK(hipGetLastError());
   if (n_steps == 0) return RFXH_OK;
+  if (res_takes(pl, s, n_steps)) {
+    const int rc = pl->rp.box ? 0 : res_setup(pl, s);
+    if (rc < 0) return rc;
+    if (rc == 0) return run_resident(pl, s, step0, n_steps);
+    pl->rp.ok = pl->res = false;
+  }
   if (pl->tb) return run_tb(pl, s, n_steps, use_graph);
   const int flip = pl->fused ? 1 : 0;
   if (!use_graph || pl->timing || n_steps < pl->graph_chunk) {
@@ -4724,7 +5044,15 @@ static PsiIO psi_io(const rfxh_plan* pl, int set) {
 }
 
 int rfxh_set_variant(rfxh_plan* pl, int kernel, int param) {
-  if (!pl || kernel < 0 || kernel > 8) return fail(RFXH_EINVAL, "bad variant");
+  if (!pl || kernel < 0 || kernel > 9) return fail(RFXH_EINVAL, "bad variant");
+  if (kernel == 9) {
+    if (param != 0) return fail(RFXH_EINVAL, "the resident step takes no parameter");
+    if (!pl->rp.ok)
+      return fail(RFXH_EINVAL, "the resident step covers grids of one block per compute unit, "
+                               "without poles or per-component eps");
+    pl->res = true;
+    return RFXH_OK;
+  }
   if (kernel == 8) {
     if (param < 0) return fail(RFXH_EINVAL, "bad segment count");
     if (!pl->set[1][0]) return fail(RFXH_EINVAL, "the temporal-blocked march needs a second field set");
@@ -4756,6 +5084,7 @@ int rfxh_set_variant(rfxh_plan* pl, int kernel, int param) {
       pl->psi_mid = static_cast<float*>(m);
     }
     pl->tb = true;
+    pl->res = false;
     pl->tb_seg = param;
     pl->fused = pl->march = pl->wmarch = false;
     for (int g = 0; g < 2; ++g)
@@ -4797,7 +5126,7 @@ int rfxh_set_variant(rfxh_plan* pl, int kernel, int param) {
   pl->fused = pingpong;
   pl->march = kernel == 2 || kernel == 3;
   pl->wmarch = kernel == 7;
-  pl->tb = false;
+  pl->tb = pl->res = false;
   for (int g = 0; g < 2; ++g)
     if (pl->graph_exec[g]) {
       (void)hipGraphExecDestroy(pl->graph_exec[g]);
@@ -4808,12 +5137,14 @@ int rfxh_set_variant(rfxh_plan* pl, int kernel, int param) {
 
 int rfxh_get_variant(rfxh_plan* pl, int* kernel, int* param) {
   if (!pl || !kernel || !param) return fail(RFXH_EINVAL, "bad arguments");
-  *kernel = pl->tb ? 8
+  *kernel = pl->res ? 9
+          : pl->tb ? 8
           : pl->wmarch ? 7
           : pl->march ? 2 + pl->march_tile
           : pl->fused ? 1
           : pl->ncol == 2 ? 4 : pl->ncol == 4 ? 5 : pl->ncol == 3 ? 6 : 0;
-  *param = pl->tb ? pl->tb_seg
+  *param = pl->res ? 0
+         : pl->tb ? pl->tb_seg
          : pl->wmarch ? pl->wmarch_seg : pl->march ? pl->march_seg : pl->kp.order;
   return RFXH_OK;
 }
