@@ -220,7 +220,8 @@ int rfxh_kernel_time_ms(rfxh_plan* plan, int which, double* avg_ms, int64_t* cou
  * the two-step sweep); 9: the resident step, a whole run in one
  * launch with the state in registers (param = 0; in place, either field
  * set; grids cut into at most one block per compute unit, about a million
- * cells, no dispersion or per-component eps, at most 32 planes, monitors
+ * cells, one mu_r, kappa = 1 in the CPML, no dispersion or per-component
+ * eps, at most 32 planes, monitors
  * and NTFF faces in all and 256 point operations a block).  It is the
  * default of every plan that fits; runs of fewer than 4 steps, timed runs
  * and runs on a stream under capture take the two-pass step instead.  Its

@@ -48,13 +48,15 @@ def variants(dr):
     (same orders) and the marching steps 2 / 3 (6- / 14-row tiles) and the
     wave-march 7 with their number of x segments (0 = automatic), and the
     temporal-blocked march 8 (two time steps per sweep: temporal-block depth
-    2 against depth 1 for every other variant) with its x segments."""
+    2 against depth 1 for every other variant) with its x segments.  The
+    resident step 9 (small grids, a whole run in one launch), which many
+    plans refuse, is not in the list; ``autotune`` tries it first."""
     out = [(0, 1), (0, 0)]
     for kern in (4, 6, 5):                  # columns of 2, 3, 4 cells
         out += [(kern, order) for order in (1, 0)]
     nx = dr.prob.shape[0]
     if len(dr.sets) == 2:
-        out += [(9, 0), (1, 1), (1, 0)]
+        out += [(1, 1), (1, 0)]
         # the wave-march and temporal-blocked steps stage the material table
         # in LDS (at most 1024 ids)
         small = len(dr.flags) <= 1024

@@ -26,18 +26,24 @@
 // NaN.
 //
 // Measured (one step, two-pass column step -> resident): 87 x 47 x 42 cells
-// 15.5 -> 4.9 us, 41^3 without CPML 14 -> 3.6, 114 x 97 x 80 with a DFT plane
-// 30.5 -> 14; what is left is the two exchanges (1.5 us each here) and, from
-// 3000 cells a workgroup up, its arithmetic.
+// 15.5 -> 4.65 us, 41^3 without CPML 14 -> 3.05, 114 x 97 x 80 with a DFT plane
+// 30.5 -> 12.2.  What is left is the two exchanges (0.9-1.5 us each) and, from
+// 3000 cells a workgroup up, the arithmetic of the blocks in a corner of the
+// CPML, which the others wait for.  What mattered in the loop: no global
+// load outside the exchange (vector memory returns in order, so any other
+// load waits for the mailbox stores before it: 0.4 us a step for a per-cell
+// ch), source values staged for many steps, a barrier for LDS alone, lane
+// conditions as bits of one register, and the z slabs' columns gathered in
+// the last wavefronts (12.6 -> 10.7 us at 114 x 97 x 80).
 //
-// The arithmetic is that of h_core and e_core_co, product for product: the
+// The arithmetic is that of h_core and e_core_co for kappa = 1, product for product: the
 // fused multiply-adds are written out as the compiler forms them there, so
 // the fields are the two-pass step's bit for bit.
 
 constexpr int kResThreads = 512;    // most threads of a workgroup
 constexpr int kResPS = 640;         // LDS floats of one plane of a block (with its halo)
 constexpr int kResOps = 256;        // point operations a block may hold
-constexpr int kResStage = 16;       // steps of source values staged at once
+constexpr int kResWave = 4096;      // source values staged at once (steps x operations)
 constexpr int kResWords = 3;        // y/z halo words a thread fetches per exchange
 constexpr int kResEdge = 192;       // most rows plus columns of a block
 constexpr int kResSnaps = 32;       // DFT planes, flux monitors and NTFF faces
@@ -59,6 +65,10 @@ struct ResIO {
   float* f[6];                      // state, updated in place
   float* psi;                       // CPML memory of the current set (null: none)
   unsigned foff[6], fs[6];          // each face's terms in it (as TBCpml)
+  const float* src_wave;            // the plan's point-operation tables
+  float* probe_out;
+  float* port_out;
+  int n_src, n_probe, n_port;
   u64* box;                         // mailboxes [phase][parity][workgroup][words]
   unsigned* stop;                   // set by a workgroup that gave up
   const ResSnap* snaps;
@@ -69,8 +79,10 @@ struct ResIO {
   unsigned tag0;                    // this launch's tags are tag0 + 1 .. tag0 + 2 n_steps
 };
 
+// A point operation of the block, staged in LDS in the order of its cell's
+// thread and then of the plan, so that a thread's operations lie together.
 struct ResOp {
-  unsigned cell;
+  int own;          // thread * NX + plane of the cell
   int kind, comp, slot;
   float d_par;
   float loop[3];
@@ -80,9 +92,9 @@ template <int NX>
 struct ResShared {
   float e[3][NX][kResPS];           // row r, column c at r * (tz + 1) + c; halo row ty, column tz
   float h[3][NX][kResPS];           // at (r + 1) * (tz + 1) + c + 1; halo row and column 0
-  float4 xprof[NX];                 // (b, c, 1/kappa - 1, 1/size) of an x slab's planes
-  ResOp ops[kResOps];               // the block's point operations, sorted by (cell, order)
-  float w[kResStage][kResOps];      // their source values of the next steps
+  float4 xprof[NX];                 // (b, c, 1/size, 0) of an x slab's planes
+  ResOp ops[kResOps];               // the block's point operations
+  float w[kResWave];                // their source values of the next steps [step][operation]
   float gx[2][NX];                  // graded: the planes' inverse spacings (H, E)
   ResSnap snap[kResSnaps];
   int n_ops, bad;
@@ -106,7 +118,7 @@ __device__ __forceinline__ void res_st2(u64* base, unsigned off, float a, float 
 // plane the y face's pairs (by column) and the z face's (by row).
 constexpr unsigned res_words(int nx) { return 2u * (kResThreads + (unsigned)nx * kResEdge); }
 
-// iy * a - iz * b and the two memory-term products, as the two-pass kernels round them.
+// iy * a - iz * b and the memory's recursion, as the two-pass kernels round them.
 __device__ __forceinline__ float res_curl(float i1, float a, float i2, float b) {
 #pragma clang fp contract(off)
   const float t = i2 * b;
@@ -117,76 +129,49 @@ __device__ __forceinline__ float res_psi(float b, float psi, float c, float g) {
   const float t = b * psi;
   return __builtin_fmaf(c, g, t);
 }
-__device__ __forceinline__ float res_corr(float co, float s, float km1, float g) {
-#pragma clang fp contract(off)
-  const float t = co * s, u = co * km1;
-  return __builtin_fmaf(g, u, t);
-}
-
-// Point operations of a cell (point_ops from the staged list).
-template <int NX>
-__device__ __forceinline__ void res_point_ops(const KParams& p, const ResShared<NX>& sh,
-                                              unsigned cell, float& e0, float& e1, float& e2,
-                                              float hx, float hy, float hz, float hx_j, float hx_k,
-                                              float hy_i, float hy_k, float hz_i, float hz_j,
-                                              long long n, int par) {
-  int lo = 0, hi = sh.n_ops;
-  while (lo < hi) {
-    const int mid = (lo + hi) >> 1;
-    if (sh.ops[mid].cell < cell) lo = mid + 1;
-    else hi = mid;
-  }
-  for (int q = lo; q < sh.n_ops && sh.ops[q].cell == cell; ++q) {
-    const ResOp& op = sh.ops[q];
-    if (op.kind == RFXH_OP_PORT) {
-      const float v = -pick3(op.comp, e0, e1, e2) * op.d_par;
-      float cur;
-      if (op.comp == 2)
-        cur = (hy - hy_i) * op.loop[1] - (hx - hx_j) * op.loop[0];
-      else if (op.comp == 0)
-        cur = (hz - hz_j) * op.loop[2] - (hy - hy_k) * op.loop[1];
-      else
-        cur = (hx - hx_k) * op.loop[0] - (hz - hz_i) * op.loop[2];
-      float* o = p.port_out + (n * p.n_port + op.slot) * 2;
-      o[0] = v;
-      o[1] = cur;
-    } else if (op.kind == RFXH_OP_INJECT) {
-      const float w = sh.w[par][q];
-      if (op.comp == 0) e0 += w;
-      else if (op.comp == 1) e1 += w;
-      else e2 += w;
-    } else {
-      p.probe_out[n * p.n_probe + op.slot] =
-          op.comp < 3 ? pick3(op.comp, e0, e1, e2) : pick3(op.comp - 3, hx, hy, hz);
-    }
-  }
-}
-
-// One slab term pair of an axis: memory s0, s1 advanced, corrections added
-// to a (+) and b (-) -- the signs of h_core; e_core_co's are the opposite.
+// One slab term pair of an axis: the memory m0, m1 advanced, the corrections
+// in d0, d1 (kappa is 1 in every slab: the plan checks that 1/kappa - 1 = 0,
+// so the correction is the memory's product alone).
 struct ResSlab {
-  float b, c, km1, inv;
+  float b, c, inv;
 };
 __device__ __forceinline__ void res_slab(const ResSlab& s, float co, float g0, float g1, float& m0,
                                          float& m1, float& d0, float& d1) {
-  g0 *= s.inv;
-  g1 *= s.inv;
-  m0 = res_psi(s.b, m0, s.c, g0);
-  m1 = res_psi(s.b, m1, s.c, g1);
-  d0 = res_corr(co, m0, s.km1, g0);
-  d1 = res_corr(co, m1, s.km1, g1);
+#pragma clang fp contract(off)
+  m0 = res_psi(s.b, m0, s.c, g0 * s.inv);
+  m1 = res_psi(s.b, m1, s.c, g1 * s.inv);
+  d0 = co * m0;
+  d1 = co * m1;
 }
 
 template <bool GRADED, int NX>
 __global__ __launch_bounds__(kResThreads) void k_resident(const KParams* __restrict__ pp,
                                                           ResIO io) {
   __shared__ ResShared<NX> sh;
-  constexpr int G = NX < 4 ? NX : NX % 4 ? 3 : 4;   // cells whose neighbours are in flight together
+  constexpr int G = NX < 4 ? NX : NX == 4 ? 4 : 2;  // cells whose neighbours are in flight together
   const int tid = (int)threadIdx.x, T = (int)blockDim.x;
   const int ty = io.ty, tz = io.tz, tyz = ty * tz, rs = tz + 1;
   const int wg = (int)blockIdx.x, n_wg = (int)gridDim.x;
   const int bz = wg % io.ntz, by = (wg / io.ntz) % io.nty, bx = wg / (io.ntz * io.nty);
-  const int row = tid / tz, col = tid - row * tz;
+  // Thread to (row, column): the columns outside the z slabs first, row by
+  // row, then those inside, so that only the last wavefronts run the z slabs'
+  // code (with the columns in order every wavefront has some of them).
+  const int sz_lo = min(max(pp->cn[4] - bz * tz, 0), tz);
+  const int sz_hi = min(max(bz * tz + tz - (pp->nz - pp->cn[5]), 0), tz - sz_lo);
+  const int n_in = tz - sz_lo - sz_hi, n_sl = sz_lo + sz_hi;
+  int row, col;
+  if (tid < ty * n_in) {
+    row = tid / n_in;
+    col = sz_lo + tid - row * n_in;
+  } else if (n_sl > 0) {
+    const int u = tid - ty * n_in;
+    row = u / n_sl;
+    col = u - row * n_sl;
+    if (col >= sz_lo) col += n_in;
+  } else {
+    row = ty;                       // past the block
+    col = 0;
+  }
   const int i0 = bx * NX, j = by * ty + row, k = bz * tz + col;
   const bool in_tile = tid < tyz;
 
@@ -197,10 +182,10 @@ __global__ __launch_bounds__(kResThreads) void k_resident(const KParams* __restr
   float ex[NX], ey[NX], ez[NX], hx[NX], hy[NX], hz[NX];
   float ca[NX], cb[NX], ce[NX];
   // 4 bits per cell: E components held at zero (outer PEC faces, PEC mask,
-  // cells outside the grid), point operations
+  // cells outside the grid)
   unsigned fl = 0u;
   float px[4][NX], py[4][NX], pz[4][NX];
-  ResSlab sy = {0.f, 0.f, 0.f, 0.f}, sz = sy;
+  ResSlab sy = {0.f, 0.f, 0.f}, sz = sy;
   bool in_y = false, in_z = false;
   unsigned in_x = 0u;               // bit q: plane i0 + q lies in an x slab
   float ghy = 0.f, ghz = 0.f, gey = 0.f, gez = 0.f;
@@ -208,6 +193,140 @@ __global__ __launch_bounds__(kResThreads) void k_resident(const KParams* __restr
   unsigned snap_bits = 0u;
   const int m0 = in_tile ? row * rs + col : 0;   // this thread's cell in sh.e; + rs + 1 in sh.h
 
+  // ---- LDS: fields, profiles, point operations, snapshots --------------------
+  for (int t = tid; t < 3 * NX * kResPS; t += T) {
+    (&sh.e[0][0][0])[t] = 0.f;
+    (&sh.h[0][0][0])[t] = 0.f;
+  }
+  {
+    const KParams& p = *pp;
+#pragma unroll
+    for (int q = 0; q < NX; ++q) {
+      const int i = i0 + q, lx = i < p.cn[0] ? i : i - (p.nx - p.cn[1]);
+      const bool xlo = i < p.cn[0], slab = i < p.nx && (xlo || lx >= 0);
+      if (slab) in_x |= 1u << q;
+      if (tid == q && i < p.nx) {
+        sh.xprof[q] = slab ? make_float4(gld(xlo ? p.pb[0] : p.pb[1], lx),
+                                         gld(xlo ? p.pc[0] : p.pc[1], lx),
+                                         xlo ? p.cinv[0] : p.cinv[1], 0.f)
+                           : make_float4(0.f, 0.f, 0.f, 0.f);
+        sh.gx[0][q] = GRADED ? gld(p.inv_h[0], i) : 0.f;
+        sh.gx[1][q] = GRADED ? gld(p.inv_e[0], i) : 0.f;
+      }
+    }
+  }
+  if (tid < io.n_snap) sh.snap[tid] = io.snaps[tid];
+  if (tid == 0) {
+    sh.n_ops = 0;
+    sh.bad = 0;
+  }
+  __syncthreads();
+  int op_lo = 0, op_n = 0;          // this thread's operations
+  {
+    // stable compaction of the block's operations (the plan checks the count)
+    const KParams& p = *pp;
+    for (int base = 0; base < p.n_ops; base += T) {
+      const int t = base + tid;
+      bool in = false;
+      rfxh_point_op op;
+      int own = 0;
+      if (t < p.n_ops) {
+        op = p.ops[t];
+        const int i = (int)(op.cell / p.plane);
+        const int r = (int)(op.cell - (long long)i * p.plane);
+        const int oj = r / p.nz - by * ty, ok = r % p.nz - bz * tz;
+        in = i >= i0 && i < i0 + NX && oj >= 0 && oj < ty && ok >= 0 && ok < tz;
+        own = ok < sz_lo ? ty * n_in + oj * n_sl + ok
+              : ok < sz_lo + n_in ? oj * n_in + ok - sz_lo
+                                  : ty * n_in + oj * n_sl + ok - n_in;
+        own = own * NX + i - i0;
+      }
+      const u64 bal = __ballot(in);
+      const int w = tid >> 6, l = tid & 63;
+      if (l == 0) sh.wcnt[w] = __popcll(bal);
+      __syncthreads();
+      int off = sh.n_ops + __popcll(bal & ((1ull << l) - 1ull));
+      for (int u = 0; u < w; ++u) off += sh.wcnt[u];
+      if (in && off < kResOps) {
+        ResOp& d = sh.ops[off];
+        d.own = own;
+        d.kind = op.kind;
+        d.comp = op.comp;
+        d.slot = op.slot;
+        d.d_par = op.d_par;
+        d.loop[0] = op.loop[0];
+        d.loop[1] = op.loop[1];
+        d.loop[2] = op.loop[2];
+      }
+      __syncthreads();
+      if (tid == 0) {
+        int tot = sh.n_ops;
+        for (int u = 0; u < (T + 63) / 64; ++u) tot += sh.wcnt[u];
+        sh.n_ops = min(tot, kResOps);
+      }
+      __syncthreads();
+    }
+    // into the order of their threads (rank by counting: few, and once)
+    const int n = sh.n_ops;
+    ResOp mine;
+    int rank = 0;
+    if (tid < n) {
+      mine = sh.ops[tid];
+      for (int t = 0; t < n; ++t)
+        rank += sh.ops[t].own < mine.own || (sh.ops[t].own == mine.own && t < tid);
+    }
+    __syncthreads();
+    if (tid < n) sh.ops[rank] = mine;
+    __syncthreads();
+    for (int t = 0; t < n; ++t) {
+      const int th = sh.ops[t].own / NX;
+      op_lo += th < tid;
+      op_n += th == tid;
+    }
+  }
+  const int n_ops = __builtin_amdgcn_readfirstlane(sh.n_ops);
+  const int stage = n_ops > 0 ? min(kResWave / n_ops, 64) : 64;
+
+  // ---- halo words ------------------------------------------------------------
+  const int per_q = ty + tz, n_yz = 2 * NX * per_q;
+  constexpr unsigned kW = 8u * res_words(NX), kQ = 16u * kResEdge, kYZ = 16u * kResThreads;
+  const unsigned half = (unsigned)n_wg * res_words(NX);     // one phase and parity
+  const bool x_next = bx + 1 < io.ntx, y_next = by + 1 < io.nty, z_next = bz + 1 < io.ntz;
+  const bool x_prev = bx > 0, y_prev = by > 0, z_prev = bz > 0;
+  const int wx = io.ntz * io.nty, wy = io.ntz;          // workgroup strides along x, y
+  // where a word goes in LDS (-1: this thread has no such word) and comes from
+  // in a mailbox half (a thread without one reads its own mailbox, unused)
+  int lds_e[kResWords], lds_h[kResWords];
+  unsigned src_e[kResWords], src_h[kResWords];
+#pragma unroll
+  for (int m = 0; m < kResWords; ++m) {
+    const KParams& p = *pp;
+    const int w = tid + m * T;
+    lds_e[m] = lds_h[m] = -1;
+    src_e[m] = src_h[m] = (unsigned)wg * kW;
+    if (w >= n_yz) continue;
+    const int c = w & 1, r = w >> 1, q = r / per_q, pos = r - q * per_q;
+    const unsigned at = kYZ + (unsigned)q * kQ + 16u * (unsigned)pos + 8u * (unsigned)c;
+    const bool yw = pos < tz;
+    const int comp = c == 0 ? 0 : yw ? 2 : 1;
+    const int base = (comp * NX + q) * kResPS;
+    if (yw ? y_next : z_next) {
+      lds_e[m] = base + (yw ? ty * rs + pos : (pos - tz) * rs + tz);
+      src_e[m] = (unsigned)(wg + (yw ? wy : 1)) * kW + at;
+      // the first H update takes the neighbour's E from memory
+      const int hi = i0 + q, hj = yw ? by * ty + ty : by * ty + pos - tz;
+      const int hk = yw ? bz * tz + pos : bz * tz + tz;
+      if (hi < p.nx && hj < p.ny && hk < p.nz) {
+        const float* fp = comp == 0 ? io.f[0] : comp == 1 ? io.f[1] : io.f[2];
+        (&sh.e[0][0][0])[lds_e[m]] =
+            ldf(fp, ((unsigned)hi * (unsigned)p.ny + (unsigned)hj) * (unsigned)p.nz + (unsigned)hk);
+      }
+    }
+    if (yw ? y_prev : z_prev) {
+      lds_h[m] = base + (yw ? pos + 1 : (pos - tz + 1) * rs);
+      src_h[m] = (unsigned)(wg - (yw ? wy : 1)) * kW + at;
+    }
+  }
   // The state and the memory to or from registers (out = false, true).
   auto state = [&](bool out, bool bad, const int i0, const int j, const int k) {
     const KParams& p = *pp;
@@ -233,13 +352,11 @@ __global__ __launch_bounds__(kResThreads) void k_resident(const KParams* __restr
       if (iy) {
         sy.b = gld(ylo ? p.pb[2] : p.pb[3], ly);
         sy.c = gld(ylo ? p.pc[2] : p.pc[3], ly);
-        sy.km1 = gld(ylo ? p.pk[2] : p.pk[3], ly);
         sy.inv = ylo ? p.cinv[2] : p.cinv[3];
       }
       if (iz) {
         sz.b = gld(zlo ? p.pb[4] : p.pb[5], lz);
         sz.c = gld(zlo ? p.pc[4] : p.pc[5], lz);
-        sz.km1 = gld(zlo ? p.pk[4] : p.pk[5], lz);
         sz.inv = zlo ? p.cinv[4] : p.cinv[5];
       }
       if (GRADED && live) {
@@ -296,7 +413,7 @@ __global__ __launch_bounds__(kResThreads) void k_resident(const KParams* __restr
       ca[q] = co.x;
       cb[q] = co.y;
       ce[q] = co.z;
-      unsigned f = __float_as_uint(co.w) & 15u;
+      unsigned f = __float_as_uint(co.w) & 7u;
       if ((p.pec_axes & 1) && (i == 0 || i == p.nx - 1)) f |= RFXH_ZERO_EY | RFXH_ZERO_EZ;
       if ((p.pec_axes & 2) && (j == 0 || j == p.ny - 1)) f |= RFXH_ZERO_EX | RFXH_ZERO_EZ;
       if (p.pec_axes & 4) {
@@ -316,118 +433,8 @@ __global__ __launch_bounds__(kResThreads) void k_resident(const KParams* __restr
       xez = ldf(io.f[2], c0 + (unsigned)NX * P);
     }
   };
+  // (after the set-up above, whose temporaries would not fit beside it)
   state(false, false, i0, j, k);
-
-  // ---- LDS: fields, profiles, point operations, snapshots --------------------
-  for (int t = tid; t < 3 * NX * kResPS; t += T) {
-    (&sh.e[0][0][0])[t] = 0.f;
-    (&sh.h[0][0][0])[t] = 0.f;
-  }
-  {
-    const KParams& p = *pp;
-#pragma unroll
-    for (int q = 0; q < NX; ++q) {
-      const int i = i0 + q, lx = i < p.cn[0] ? i : i - (p.nx - p.cn[1]);
-      const bool xlo = i < p.cn[0], slab = i < p.nx && (xlo || lx >= 0);
-      if (slab) in_x |= 1u << q;
-      if (tid == q && i < p.nx) {
-        sh.xprof[q] = slab ? make_float4(gld(xlo ? p.pb[0] : p.pb[1], lx),
-                                         gld(xlo ? p.pc[0] : p.pc[1], lx),
-                                         gld(xlo ? p.pk[0] : p.pk[1], lx),
-                                         xlo ? p.cinv[0] : p.cinv[1])
-                           : make_float4(0.f, 0.f, 0.f, 0.f);
-        sh.gx[0][q] = GRADED ? gld(p.inv_h[0], i) : 0.f;
-        sh.gx[1][q] = GRADED ? gld(p.inv_e[0], i) : 0.f;
-      }
-    }
-  }
-  if (tid < io.n_snap) sh.snap[tid] = io.snaps[tid];
-  if (tid == 0) {
-    sh.n_ops = 0;
-    sh.bad = 0;
-  }
-  __syncthreads();
-  {
-    // stable compaction of the block's operations (the plan checks the count)
-    const KParams& p = *pp;
-    for (int base = 0; base < p.n_ops; base += T) {
-      const int t = base + tid;
-      bool in = false;
-      rfxh_point_op op;
-      if (t < p.n_ops) {
-        op = p.ops[t];
-        const int i = (int)(op.cell / p.plane);
-        const int r = (int)(op.cell - (long long)i * p.plane);
-        const int oj = r / p.nz, ok = r - oj * p.nz;
-        in = i >= i0 && i < i0 + NX && oj >= by * ty && oj < by * ty + ty && ok >= bz * tz &&
-             ok < bz * tz + tz;
-      }
-      const u64 bal = __ballot(in);
-      const int w = tid >> 6, l = tid & 63;
-      if (l == 0) sh.wcnt[w] = __popcll(bal);
-      __syncthreads();
-      int off = sh.n_ops + __popcll(bal & ((1ull << l) - 1ull));
-      for (int u = 0; u < w; ++u) off += sh.wcnt[u];
-      if (in && off < kResOps) {
-        ResOp& d = sh.ops[off];
-        d.cell = (unsigned)op.cell;
-        d.kind = op.kind;
-        d.comp = op.comp;
-        d.slot = op.slot;
-        d.d_par = op.d_par;
-        d.loop[0] = op.loop[0];
-        d.loop[1] = op.loop[1];
-        d.loop[2] = op.loop[2];
-      }
-      __syncthreads();
-      if (tid == 0) {
-        int tot = sh.n_ops;
-        for (int u = 0; u < (T + 63) / 64; ++u) tot += sh.wcnt[u];
-        sh.n_ops = min(tot, kResOps);
-      }
-      __syncthreads();
-    }
-  }
-  const int n_ops = __builtin_amdgcn_readfirstlane(sh.n_ops);
-
-  // ---- halo words ------------------------------------------------------------
-  const int per_q = ty + tz, n_yz = 2 * NX * per_q;
-  constexpr unsigned kW = 8u * res_words(NX), kQ = 16u * kResEdge, kYZ = 16u * kResThreads;
-  const unsigned half = (unsigned)n_wg * res_words(NX);     // one phase and parity
-  const bool x_next = bx + 1 < io.ntx, y_next = by + 1 < io.nty, z_next = bz + 1 < io.ntz;
-  const bool x_prev = bx > 0, y_prev = by > 0, z_prev = bz > 0;
-  const int wx = io.ntz * io.nty, wy = io.ntz;          // workgroup strides along x, y
-  int lds_e[kResWords], lds_h[kResWords];               // -1: no such word
-  unsigned src_e[kResWords], src_h[kResWords];          // where it comes from in a mailbox half
-#pragma unroll
-  for (int m = 0; m < kResWords; ++m) {
-    const KParams& p = *pp;
-    const int w = tid + m * T;
-    lds_e[m] = lds_h[m] = -1;
-    src_e[m] = src_h[m] = 0u;
-    if (w >= n_yz) continue;
-    const int c = w & 1, r = w >> 1, q = r / per_q, pos = r - q * per_q;
-    const unsigned at = kYZ + (unsigned)q * kQ + 16u * (unsigned)pos + 8u * (unsigned)c;
-    const bool yw = pos < tz;
-    const int comp = c == 0 ? 0 : yw ? 2 : 1;
-    const int base = (comp * NX + q) * kResPS;
-    if (yw ? y_next : z_next) {
-      lds_e[m] = base + (yw ? ty * rs + pos : (pos - tz) * rs + tz);
-      src_e[m] = (unsigned)(wg + (yw ? wy : 1)) * kW + at;
-      // the first H update takes the neighbour's E from memory
-      const int hi = i0 + q, hj = yw ? by * ty + ty : by * ty + pos - tz;
-      const int hk = yw ? bz * tz + pos : bz * tz + tz;
-      if (hi < p.nx && hj < p.ny && hk < p.nz) {
-        const float* fp = comp == 0 ? io.f[0] : comp == 1 ? io.f[1] : io.f[2];
-        (&sh.e[0][0][0])[lds_e[m]] =
-            ldf(fp, ((unsigned)hi * (unsigned)p.ny + (unsigned)hj) * (unsigned)p.nz + (unsigned)hk);
-      }
-    }
-    if (yw ? y_prev : z_prev) {
-      lds_h[m] = base + (yw ? pos + 1 : (pos - tz + 1) * rs);
-      src_h[m] = (unsigned)(wg - (yw ? wy : 1)) * kW + at;
-    }
-  }
 #pragma unroll
   for (int q = 0; q < NX; ++q)
     if (in_tile) {
@@ -444,34 +451,38 @@ __global__ __launch_bounds__(kResThreads) void k_resident(const KParams* __restr
     else hit = hit && a + NX > s.lo1 && a < s.hi1 && (s.axis == 1 ? j : k) == s.index;
     if (hit) snap_bits |= 1u << t;
   }
-  // fetch the halo of one phase: the tagged words of `src` into LDS and the
-  // two x words of workgroup x_wg into a, b
+  // Fetch the halo of one phase: the tagged words of `src` into LDS and the
+  // two x words at xsrc into a, b.  Every lane loads every word, so that the
+  // loads are in flight together with no branch between them.
   auto fetch = [&](const u64* from, unsigned tag, const int (&dst)[kResWords],
-                   const unsigned (&src)[kResWords], float* lds, bool has_x, unsigned xsrc,
+                   const unsigned (&src)[kResWords], float* lds, unsigned need_x, unsigned xsrc,
                    float& a, float& b) {
-    u64 v[kResWords], va = 0, vb = 0;
+    u64 v[kResWords], va, vb;
     for (int n = 0;;) {
-      bool ok = true;
-      if (has_x) {
-        va = res_ld(from, xsrc);
-        vb = res_ld(from, xsrc + 8u);
+      // (opaque: 32-bit offsets from the scalar base, not 64-bit addresses)
+      unsigned ox = xsrc;
+      __asm__ volatile("" : "+v"(ox));
+      va = res_ld(from, ox);
+      vb = res_ld(from, ox + 8u);
+#pragma unroll
+      for (int m = 0; m < kResWords; ++m) {
+        unsigned o = src[m];
+        __asm__ volatile("" : "+v"(o));
+        v[m] = res_ld(from, o);
       }
+      unsigned off = (((unsigned)(va >> 32) ^ tag) | ((unsigned)(vb >> 32) ^ tag)) & need_x;
 #pragma unroll
-      for (int m = 0; m < kResWords; ++m) v[m] = dst[m] >= 0 ? res_ld(from, src[m]) : 0;
-      if (has_x) ok = (unsigned)(va >> 32) == tag && (unsigned)(vb >> 32) == tag;
-#pragma unroll
-      for (int m = 0; m < kResWords; ++m) ok = ok && (dst[m] < 0 || (unsigned)(v[m] >> 32) == tag);
-      if (ok) break;
+      for (int m = 0; m < kResWords; ++m)
+        off |= ((unsigned)(v[m] >> 32) ^ tag) & (unsigned)~(dst[m] >> 31);
+      if (off == 0u) break;
       if (++n >= kResSpin || ((n & 4095) == 0 &&
                               __hip_atomic_load(io.stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
         sh.bad = 1;
         break;
       }
     }
-    if (has_x) {
-      a = __uint_as_float((unsigned)va);
-      b = __uint_as_float((unsigned)vb);
-    }
+    a = need_x ? __uint_as_float((unsigned)va) : 0.f;
+    b = need_x ? __uint_as_float((unsigned)vb) : 0.f;
 #pragma unroll
     for (int m = 0; m < kResWords; ++m)
       if (dst[m] >= 0) lds[dst[m]] = __uint_as_float((unsigned)v[m]);
@@ -483,17 +494,26 @@ __global__ __launch_bounds__(kResThreads) void k_resident(const KParams* __restr
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
   };
-  // loop-invariant scalars
-  const float ch_all = pp->ch_all, inv_h0 = pp->inv_h0, inv_e0 = pp->inv_e0;
-  const bool any_x = in_x != 0u;
-  const bool edge_y = in_tile && row == ty - 1 && y_next, edge_z = in_tile && col == tz - 1 && z_next;
-  const bool low_y = in_tile && row == 0 && y_prev, low_z = in_tile && col == 0 && z_prev;
-  const unsigned xs_h = (unsigned)(wg - wx) * kW + 16u * (unsigned)tid;
-  const unsigned xs_e = (unsigned)(wg + wx) * kW + 16u * (unsigned)tid;
+  // Loop-invariant scalars.  What differs between lanes is kept as bits of one
+  // register and tested where it is used: as lane masks in scalar registers
+  // these conditions spilled, with the parameters they pushed out.
+  const float ch = pp->ch_all, inv_h0 = pp->inv_h0, inv_e0 = pp->inv_e0;
+  const unsigned roles = (in_tile ? 1u : 0u) | (in_tile && x_next ? 2u : 0u) |
+                         (in_tile && x_prev ? 4u : 0u) |
+                         (in_tile && row == ty - 1 && y_next ? 8u : 0u) |
+                         (in_tile && col == tz - 1 && z_next ? 16u : 0u) |
+                         (in_tile && row == 0 && y_prev ? 32u : 0u) |
+                         (in_tile && col == 0 && z_prev ? 64u : 0u) | (in_y ? 128u : 0u) |
+                         (in_z ? 256u : 0u);
+  const unsigned need_h = (roles & 4u) ? ~0u : 0u, need_e = (roles & 2u) ? ~0u : 0u;
+  const unsigned xs_h = (unsigned)(need_h ? wg - wx : wg) * kW + 16u * (unsigned)tid;
+  const unsigned xs_e = (unsigned)(need_e ? wg + wx : wg) * kW + 16u * (unsigned)tid;
   const int n_steps = io.n_steps;
   __syncthreads();
 
   bool bad = false;
+  unsigned tag = io.tag0;
+  int w_base = 0, w_next = 0;           // first step of the staged source values, of the next ones
   for (int n = 0; n < n_steps; ++n) {
     const int par = n & 1;
     u64* const box_h = io.box + (unsigned)par * half;
@@ -503,21 +523,23 @@ __global__ __launch_bounds__(kResThreads) void k_resident(const KParams* __restr
     unsigned out_x = (unsigned)wg * kW + 16u * (unsigned)tid;
     unsigned out_y = (unsigned)wg * kW + kYZ + 16u * (unsigned)col;
     unsigned out_z = (unsigned)wg * kW + kYZ + 16u * (unsigned)(tz + row);
-    __asm__ volatile("" : "+v"(out_x), "+v"(out_y), "+v"(out_z));
-    const unsigned tag_h = io.tag0 + 2u * (unsigned)n + 1u, tag_e = tag_h + 1u;
-    if (n_ops > 0 && n % kResStage == 0) {
-      // the source values of the next kResStage steps
-      const KParams& p = *pp;
-      for (int t = tid; t < n_ops * kResStage; t += T) {
+    unsigned role = roles;
+    __asm__ volatile("" : "+v"(out_x), "+v"(out_y), "+v"(out_z), "+v"(role));
+    const unsigned tag_h = ++tag, tag_e = ++tag;
+    if (n_ops > 0 && n == w_next) {
+      // the source values of the next `stage` steps
+      w_base = n;
+      w_next = n + stage;
+      for (int t = tid; t < n_ops * stage; t += T) {
         const int s = t / n_ops, o = t - s * n_ops;
         if (sh.ops[o].kind == RFXH_OP_INJECT && n + s < n_steps)
-          sh.w[s][o] = p.src_wave[(io.step0 + n + s) * p.n_src + sh.ops[o].slot];
+          sh.w[t] = io.src_wave[(io.step0 + n + s) * io.n_src + sh.ops[o].slot];
       }
     }
     // ---- H (cells outside the grid stay zero: so do their forward neighbours)
 #pragma unroll
     for (int q0 = 0; q0 < NX; q0 += G) {
-      float dzy[G], dyz[G], dxz[G], dzx[G], dyx[G], dxy[G], ch[G];
+      float dzy[G], dyz[G], dxz[G], dzx[G], dyx[G], dxy[G];
 #pragma unroll
       for (int u = 0; u < G; ++u) {
         const int q = q0 + u;
@@ -525,15 +547,6 @@ __global__ __launch_bounds__(kResThreads) void k_resident(const KParams* __restr
         dzy[u] = sh.e[2][q][m0 + rs];
         dxz[u] = sh.e[0][q][m0 + 1];
         dyz[u] = sh.e[1][q][m0 + 1];
-        ch[u] = ch_all;
-      }
-      if (ch_all <= 0.f) {
-        const KParams& p = *pp;
-#pragma unroll
-        for (int u = 0; u < G; ++u)
-          if (j < p.ny && k < p.nz && in_tile && i0 + q0 + u < p.nx)
-            ch[u] = ld_ch(p.coef, ldu16(p.mat, ((unsigned)(i0 + q0 + u) * (unsigned)p.ny +
-                                                (unsigned)j) * (unsigned)p.nz + (unsigned)k));
       }
 #pragma unroll
       for (int u = 0; u < G; ++u) {
@@ -546,59 +559,59 @@ __global__ __launch_bounds__(kResThreads) void k_resident(const KParams* __restr
         dyx[u] = (q + 1 < NX ? ey[q + 1 < NX ? q + 1 : q] : xey) - ey[q];
         const float ix = GRADED ? sh.gx[0][q] : inv_h0;
         const float iy = GRADED ? ghy : inv_h0, iz = GRADED ? ghz : inv_h0;
-        hx[q] = __builtin_fmaf(-ch[u], res_curl(iy, dzy[u], iz, dyz[u]), hx[q]);
-        hy[q] = __builtin_fmaf(-ch[u], res_curl(iz, dxz[u], ix, dzx[u]), hy[q]);
-        hz[q] = __builtin_fmaf(-ch[u], res_curl(ix, dyx[u], iy, dxy[u]), hz[q]);
+        hx[q] = __builtin_fmaf(-ch, res_curl(iy, dzy[u], iz, dyz[u]), hx[q]);
+        hy[q] = __builtin_fmaf(-ch, res_curl(iz, dxz[u], ix, dzx[u]), hy[q]);
+        hz[q] = __builtin_fmaf(-ch, res_curl(ix, dyx[u], iy, dxy[u]), hz[q]);
       }
-      if (any_x) {
+      if (in_x) {
 #pragma unroll
         for (int u = 0; u < G; ++u) {
           const int q = q0 + u;
           if (!((in_x >> q) & 1u)) continue;
           const float4 pr = sh.xprof[q];
-          const ResSlab s = {pr.x, pr.y, pr.z, pr.w};
+          const ResSlab s = {pr.x, pr.y, pr.z};
           float d0, d1;
-          res_slab(s, ch[u], dzx[u], dyx[u], px[0][q], px[1][q], d0, d1);
+          res_slab(s, ch, dzx[u], dyx[u], px[0][q], px[1][q], d0, d1);
           hy[q] += d0;
           hz[q] -= d1;
         }
       }
-      if (in_y) {
+      if (role & 128u) {
 #pragma unroll
         for (int u = 0; u < G; ++u) {
           const int q = q0 + u;
           float d0, d1;
-          res_slab(sy, ch[u], dzy[u], dxy[u], py[0][q], py[1][q], d0, d1);
+          res_slab(sy, ch, dzy[u], dxy[u], py[0][q], py[1][q], d0, d1);
           hx[q] -= d0;
           hz[q] += d1;
         }
       }
-      if (in_z) {
+      if (role & 256u) {
 #pragma unroll
         for (int u = 0; u < G; ++u) {
           const int q = q0 + u;
           float d0, d1;
-          res_slab(sz, ch[u], dyz[u], dxz[u], pz[0][q], pz[1][q], d0, d1);
+          res_slab(sz, ch, dyz[u], dxz[u], pz[0][q], pz[1][q], d0, d1);
           hx[q] += d0;
           hy[q] -= d1;
         }
       }
     }
     // ---- H of the high faces to the workgroups ahead, own H to LDS
-    if (in_tile && x_next) res_st2(box_h, out_x, hy[NX - 1], hz[NX - 1], tag_h);
-    if (edge_y) {
+    if (role & 2u) res_st2(box_h, out_x, hy[NX - 1], hz[NX - 1], tag_h);
+    if (role & 8u) {
 #pragma unroll
       for (int q = 0; q < NX; ++q) {
         res_st2(box_h, out_y + (unsigned)q * kQ, hx[q], hz[q], tag_h);
       }
     }
-    if (edge_z) {
+    if (role & 16u) {
 #pragma unroll
       for (int q = 0; q < NX; ++q) {
         res_st2(box_h, out_z + (unsigned)q * kQ, hx[q], hy[q], tag_h);
       }
     }
-    if (in_tile) {
+    if (role & 1u) {
 #pragma unroll
       for (int q = 0; q < NX; ++q) {
         sh.h[0][q][m0 + rs + 1] = hx[q];
@@ -606,7 +619,7 @@ __global__ __launch_bounds__(kResThreads) void k_resident(const KParams* __restr
         sh.h[2][q][m0 + rs + 1] = hz[q];
       }
     }
-    fetch(box_h, tag_h, lds_h, src_h, &sh.h[0][0][0], x_prev && in_tile, xs_h, xhy, xhz);
+    fetch(box_h, tag_h, lds_h, src_h, &sh.h[0][0][0], need_h, xs_h, xhy, xhz);
     lds_barrier();
     // ---- E
 #pragma unroll
@@ -638,20 +651,20 @@ __global__ __launch_bounds__(kResThreads) void k_resident(const KParams* __restr
           ez[q] = __builtin_fmaf(ez[q], ca[q], res_curl(ix, dyx[u], iy, dxy[u]) * cb[q]);
         }
       }
-      if (any_x) {
+      if (in_x) {
 #pragma unroll
         for (int u = 0; u < G; ++u) {
           const int q = q0 + u;
           if (!((in_x >> q) & 1u)) continue;
           const float4 pr = sh.xprof[q];
-          const ResSlab s = {pr.x, pr.y, pr.z, pr.w};
+          const ResSlab s = {pr.x, pr.y, pr.z};
           float d0, d1;
           res_slab(s, ce[q], dzx[u], dyx[u], px[2][q], px[3][q], d0, d1);
           ey[q] -= d0;
           ez[q] += d1;
         }
       }
-      if (in_y) {
+      if (role & 128u) {
 #pragma unroll
         for (int u = 0; u < G; ++u) {
           const int q = q0 + u;
@@ -661,7 +674,7 @@ __global__ __launch_bounds__(kResThreads) void k_resident(const KParams* __restr
           ez[q] -= d1;
         }
       }
-      if (in_z) {
+      if (role & 256u) {
 #pragma unroll
         for (int u = 0; u < G; ++u) {
           const int q = q0 + u;
@@ -675,39 +688,74 @@ __global__ __launch_bounds__(kResThreads) void k_resident(const KParams* __restr
     if (fl) {
 #pragma unroll
       for (int q = 0; q < NX; ++q) {
-        const unsigned f = (fl >> (4 * q)) & 15u;
-        if (f & RFXH_ZERO_EX) ex[q] = 0.f;
-        if (f & RFXH_ZERO_EY) ey[q] = 0.f;
-        if (f & RFXH_ZERO_EZ) ez[q] = 0.f;
-        if (f & RFXH_POINT) {
-          const KParams& p = *pp;
-          const int at = m0 + rs + 1;
-          res_point_ops<NX>(p, sh, ((unsigned)(i0 + q) * (unsigned)p.ny + (unsigned)j) *
-                                           (unsigned)p.nz + (unsigned)k,
-                            ex[q], ey[q], ez[q], hx[q], hy[q], hz[q], sh.h[0][q][at - rs],
-                            sh.h[0][q][at - 1], q > 0 ? hy[q > 0 ? q - 1 : 0] : xhy,
-                            sh.h[1][q][at - 1], q > 0 ? hz[q > 0 ? q - 1 : 0] : xhz,
-                            sh.h[2][q][at - rs], io.step0 + n, n % kResStage);
+        const unsigned f = fl >> (4 * q);
+        ex[q] = (f & RFXH_ZERO_EX) ? 0.f : ex[q];
+        ey[q] = (f & RFXH_ZERO_EY) ? 0.f : ey[q];
+        ez[q] = (f & RFXH_ZERO_EZ) ? 0.f : ez[q];
+      }
+    }
+    for (int o = op_lo; o < op_lo + op_n; ++o) {
+      // (point_ops; H of the cell and behind it from LDS, E from registers)
+      const ResOp op = sh.ops[o];
+      const int c = op.comp, oq = op.own - tid * NX, at = m0 + rs + 1;
+      if (op.kind == RFXH_OP_INJECT) {
+        const float w = sh.w[(n - w_base) * n_ops + o];
+#pragma unroll
+        for (int q = 0; q < NX; ++q) {
+          if (q != oq) continue;
+          if (c == 0) ex[q] += w;
+          else if (c == 1) ey[q] += w;
+          else ez[q] += w;
         }
+        continue;
+      }
+      float e0 = ex[0], e1 = ey[0], e2 = ez[0];
+#pragma unroll
+      for (int q = 1; q < NX; ++q)
+        if (q == oq) {
+          e0 = ex[q];
+          e1 = ey[q];
+          e2 = ez[q];
+        }
+      const float h0 = sh.h[0][oq][at], h1 = sh.h[1][oq][at], h2 = sh.h[2][oq][at];
+      if (op.kind == RFXH_OP_PORT) {
+        const float v = -pick3(c, e0, e1, e2) * op.d_par;
+        const float hx_j = sh.h[0][oq][at - rs], hz_j = sh.h[2][oq][at - rs];
+        const float hx_k = sh.h[0][oq][at - 1], hy_k = sh.h[1][oq][at - 1];
+        const float hy_i = oq > 0 ? sh.h[1][max(oq - 1, 0)][at] : xhy;
+        const float hz_i = oq > 0 ? sh.h[2][max(oq - 1, 0)][at] : xhz;
+        float cur;
+        if (c == 2)
+          cur = (h1 - hy_i) * op.loop[1] - (h0 - hx_j) * op.loop[0];
+        else if (c == 0)
+          cur = (h2 - hz_j) * op.loop[2] - (h1 - hy_k) * op.loop[1];
+        else
+          cur = (h0 - hx_k) * op.loop[0] - (h2 - hz_i) * op.loop[2];
+        float* const out = io.port_out + ((io.step0 + n) * io.n_port + op.slot) * 2;
+        out[0] = v;
+        out[1] = cur;
+      } else {
+        io.probe_out[(io.step0 + n) * io.n_probe + op.slot] =
+            c < 3 ? pick3(c, e0, e1, e2) : pick3(c - 3, h0, h1, h2);
       }
     }
     const bool last = n + 1 == n_steps;
     if (!last) {
       // ---- E of the low faces to the workgroups behind, own E to LDS
-      if (in_tile && x_prev) res_st2(box_e, out_x, ey[0], ez[0], tag_e);
-      if (low_y) {
+      if (role & 4u) res_st2(box_e, out_x, ey[0], ez[0], tag_e);
+      if (role & 32u) {
 #pragma unroll
         for (int q = 0; q < NX; ++q) {
           res_st2(box_e, out_y + (unsigned)q * kQ, ex[q], ez[q], tag_e);
         }
       }
-      if (low_z) {
+      if (role & 64u) {
 #pragma unroll
         for (int q = 0; q < NX; ++q) {
           res_st2(box_e, out_z + (unsigned)q * kQ, ex[q], ey[q], tag_e);
         }
       }
-      if (in_tile) {
+      if (role & 1u) {
 #pragma unroll
         for (int q = 0; q < NX; ++q) {
           sh.e[0][q][m0] = ex[q];
@@ -747,10 +795,12 @@ __global__ __launch_bounds__(kResThreads) void k_resident(const KParams* __restr
       }
     }
     if (last) break;
-    fetch(box_e, tag_e, lds_e, src_e, &sh.e[0][0][0], x_next && in_tile, xs_e, xey, xez);
+    fetch(box_e, tag_e, lds_e, src_e, &sh.e[0][0][0], need_e, xs_e, xey, xez);
     lds_barrier();
-    bad = sh.bad;
-    if (bad) break;
+    if ((n & 31) == 31) {
+      bad = sh.bad;
+      if (bad) break;
+    }
   }
   bad = bad || sh.bad;
   if (bad && tid == 0)

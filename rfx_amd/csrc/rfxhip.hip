@@ -4300,10 +4300,12 @@ void res_release(int dev) {
 // a model of the step (microseconds): two exchanges, 0.55 + 0.65 per
 // thousand words of a workgroup, and 0.12 per plane and wavefront of a SIMD
 // (about 75 vector and LDS instructions a cell in each half).  Plans it does
-// not cover keep rp.ok false: dispersive poles and per-component eps, CPML
-// slabs that overlap, more snapshots or point operations in a block than it
+// not cover keep rp.ok false: dispersive poles, per-component eps, several
+// mu_r (a load of ch in the loop would wait for the mailbox stores), CPML
+// slabs that overlap or whose kappa is not 1, more snapshots or point operations in a block than it
 // stages, grids of more blocks than compute units.
-void res_choose(rfxh_plan* pl, const std::vector<rfxh_point_op>& ops) {
+void res_choose(rfxh_plan* pl, const std::vector<rfxh_point_op>& ops,
+                const std::vector<float>& km1) {
   ResPlan& r = pl->rp;
   const KParams& kp = pl->kp;
   int dev = 0, cus = 0;
@@ -4311,11 +4313,13 @@ void res_choose(rfxh_plan* pl, const std::vector<rfxh_point_op>& ops) {
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
     return;
   const long long cells = (long long)kp.nx * kp.plane;
-  if (pl->n_pole > 0 || pl->aniso || cells > (long long)cus * 8 * kResThreads) return;
+  if (pl->n_pole > 0 || pl->aniso || kp.ch_all <= 0.f || cells > (long long)cus * 8 * kResThreads) return;
   if (pl->planes.size() + pl->fluxes.size() > (size_t)kResSnaps) return;
   const int N[3] = {kp.nx, kp.ny, kp.nz};
   for (int a = 0; a < 3; ++a)
     if (kp.cn[2 * a] + kp.cn[2 * a + 1] > N[a]) return;
+  for (float k : km1)
+    if (k != 0.f) return;
   if ((long long)pl->psi_foff[5] + 4LL * pl->psi_fs[5] >= (1LL << 30)) return;
   double best = 1e30;
   for (int nx : kResNX) {
@@ -4443,6 +4447,12 @@ int run_resident(rfxh_plan* pl, hipStream_t s, int64_t step0, int64_t n_steps) {
     io.foff[f] = pl->psi_foff[f];
     io.fs[f] = pl->psi_fs[f];
   }
+  io.src_wave = kp.src_wave;
+  io.probe_out = kp.probe_out;
+  io.port_out = kp.port_out;
+  io.n_src = kp.n_src;
+  io.n_probe = kp.n_probe;
+  io.n_port = kp.n_port;
   io.box = r.box;
   io.stop = r.stop;
   io.snaps = r.snaps;
@@ -4975,7 +4985,9 @@ int rfxh_plan_create(const rfxh_desc* d, rfxh_plan** out) {
   const char* ord = std::getenv("RFXH_ORDER");
   kp.order = (ord && std::string(ord) == "bands") ? 0 : 1;
   if ((rc = plan_grid(pl))) return bail(rc);
-  res_choose(pl, ops);
+  std::vector<float> km1;
+  for (int f = 0; f < 6; ++f) km1.insert(km1.end(), d->cpml_km1[f], d->cpml_km1[f] + d->cpml_n[f]);
+  res_choose(pl, ops, km1);
   // the default of every grid that fits: 3-6 times the two-pass step's speed
   pl->res = pl->rp.ok && kname.empty();
   pl->tev.resize(4 * kTimingSamples);
@@ -5225,7 +5237,7 @@ int rfxh_set_variant(rfxh_plan* pl, int kernel, int param) {
     if (param != 0) return fail(RFXH_EINVAL, "the resident step takes no parameter");
     if (!pl->rp.ok)
       return fail(RFXH_EINVAL, "the resident step covers grids of one block per compute unit, "
-                               "without poles or per-component eps");
+                               "without poles, per-component eps or several mu_r");
     pl->res = true;
     return RFXH_OK;
   }

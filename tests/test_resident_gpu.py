@@ -23,7 +23,7 @@ def R():
     return rfx_amd
 
 
-def _spec(n, cpml, mag=False, probes=True):
+def _spec(n, cpml, mag=False):
     dx = 1e-3
     dom = tuple((v - 0.5) * dx for v in n)
     c = [v * dx for v in (n[0] // 2, n[1] // 2, n[2] // 2)]
@@ -38,7 +38,7 @@ def _spec(n, cpml, mag=False, probes=True):
                 cpml_layers=cpml, materials=mats, geometry=geom,
                 ports=[(tuple(c), "ez", 0.0, o.Pulse(12e9, 0.9), True),
                        (src, "ex", 0.0, o.Pulse(9e9, 0.8), True)],
-                probes=[(tuple(c), "ez"), (src, "hx"), ((0.0, 0.0, 0.0), "ey")] if probes else [],
+                probes=[(tuple(c), "ez"), (src, "hx"), ((0.0, 0.0, 0.0), "ey")],
                 dft_planes=[("z", c[2], "ez", np.array([5e9, 9e9, 12e9, 14e9, 20e9]), 5),
                             ("x", c[0], "hy", np.array([8e9]), 1)],
                 flux_monitors=[("x", c[0], np.array([8e9, 9e9]), 2, None, None, "rect", 0.25),
@@ -73,20 +73,20 @@ def _same(dr, n, pieces=None):
     assert float(res[(9, 0)][0].abs().max()) > 0
 
 
-@pytest.mark.parametrize("n, cpml, mag, steps", [
-    ((3, 3, 3), 0, False, 9),            # one block, smaller than a wavefront
-    ((6, 5, 40), 0, False, 33),
-    ((11, 12, 13), 6, True, 41),         # per-cell ch; slabs on most cells
-    ((40, 30, 9), 8, False, 60),
-    ((70, 30, 25), 8, False, 37),        # the README quick start's grid
-    ((5, 150, 17), 6, False, 30),        # flat, many rows
-    ((96, 80, 63), 8, False, 24),        # near the most cells
-    ((200, 21, 37), 6, False, 24),
+@pytest.mark.parametrize("n, cpml, steps", [
+    ((3, 3, 3), 0, 9),                   # one block, smaller than a wavefront
+    ((6, 5, 40), 0, 33),
+    ((11, 12, 13), 6, 41),               # slabs on most cells
+    ((40, 30, 9), 8, 60),
+    ((70, 30, 25), 8, 37),               # the README quick start's grid
+    ((5, 150, 17), 6, 30),               # flat, many rows
+    ((96, 80, 63), 8, 24),               # near the most cells
+    ((200, 21, 37), 6, 24),
 ])
-def test_equals_the_two_pass_step(R, n, cpml, mag, steps):
+def test_equals_the_two_pass_step(R, n, cpml, steps):
     from rfx_amd.engine import DeviceRun
     print("[gpu-case] resident", n, cpml, flush=True)
-    sim = cases.to_sim(_spec(n, cpml, mag))
+    sim = cases.to_sim(_spec(n, cpml))
     _, prob, _ = sim._build_problem(steps, "run")
     for two in (True, False):
         dr = DeviceRun(prob, steps, "cuda", two_sets=two)
@@ -97,7 +97,8 @@ def test_equals_the_two_pass_step(R, n, cpml, mag, steps):
 def test_pieces_ports_and_graded(R):
     from rfx_amd.engine import DeviceRun
     print("[gpu-case] resident, graded mixed case in pieces", flush=True)
-    spec = cases.mixed_graded_case()
+    spec = dict(cases.mixed_graded_case())
+    spec["materials"] = {k: (e, s, 1.0) for k, (e, s, _) in spec["materials"].items()}
     sim = cases.to_sim(spec)
     _, prob, _ = sim._build_problem(71, "run", s11_freqs=np.asarray(spec["s11_freqs"], np.float32))
     dr = DeviceRun(prob, 71, "cuda")
@@ -142,6 +143,9 @@ def test_refused_and_default(R):
     with pytest.raises(_lib.RfxHipError):
         at.set_variant(small, 9, 1)
     small.close()
+    mag = DeviceRun(cases.to_sim(_spec((12, 12, 12), 6, True))._build_problem(8, "run")[1], 8, "cuda")
+    assert at.get_variant(mag) != (9, 0)          # several mu_r
+    mag.close()
     big = DeviceRun(cases.to_sim(_spec((150, 150, 80), 0))._build_problem(8, "run")[1], 8, "cuda")
     with pytest.raises(_lib.RfxHipError):
         at.set_variant(big, 9, 0)
