@@ -1831,8 +1831,16 @@ __device__ __forceinline__ void two_pass_e(const KParams& p, const PsiIO& ps, in
   e_cell<GRADED, DISP>(p, Eo, En, ps, i, j, k, hx, hy, hz, hy_i, hz_i, hx_j, hz_j, hx_k, hy_k);
 }
 
+// The H pass of a step counts it (nothing in the pass reads the step): a
+// counter kernel of its own after every step cost 3-5 us, on every grid too
+// large for the resident step (222x164x140: 73.5 -> 71.1 us a step).
+__device__ __forceinline__ void count_step(const KParams& p) {
+  if (blockIdx.x == 0 && threadIdx.x == 0 && threadIdx.y == 0) *p.step += 1;
+}
+
 template <bool GRADED, bool ONE_MU>
 __global__ __launch_bounds__(kWG) void k_update_h(KParams p, PsiIO ps) {
+  count_step(p);
   int i, j, k;
   if (!cell_of(p, i, j, k)) return;
   two_pass_h<GRADED, ONE_MU>(p, ps, i, j, k);
@@ -1968,6 +1976,7 @@ __device__ __forceinline__ void col_e(const KParams& p, const PsiIO& ps, int i0,
 template <bool GRADED, int NP, bool ONE_MU>
 __global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(NP == 2 ? 8 : 1)))
 void k_update_h_col(KParams p, const PsiIO* __restrict__ psp) {
+  count_step(p);
   const PsiIO& ps = *psp;
   int ib, j, k;
   if (!cell_at(p, xcd_remap((int)blockIdx.x, (int)gridDim.x), ib, j, k, (p.nx + NP - 1) / NP))
@@ -2027,6 +2036,8 @@ __global__ __launch_bounds__(kWG) void k_batch_pass(const BatchEntry* __restrict
   const int q = batch_instance(start, n_act, L);
   const KParams& p = ents[q].p;
   int i, j, k;
+  // (as count_step: the instance's first workgroup counts its step)
+  if (PASS == 0 && L == gld(start, q) && threadIdx.x == 0 && threadIdx.y == 0) *p.step += 1;
   if (!cell_at(p, L - gld(start, q), i, j, k)) return;
   if (PASS == 0) {
     if (p.graded) two_pass_h<true, ONE_MU>(p, ents[q].ps, i, j, k);
@@ -2037,6 +2048,7 @@ __global__ __launch_bounds__(kWG) void k_batch_pass(const BatchEntry* __restrict
   }
 }
 
+// (after a run's last steps: every counter one past its instance's last step)
 __global__ void k_batch_advance(const BatchEntry* __restrict__ ents, int n_act) {
   const int q = (int)(blockIdx.x * blockDim.x + threadIdx.x);
   if (q < n_act) {
@@ -2048,7 +2060,7 @@ __global__ void k_batch_advance(const BatchEntry* __restrict__ ents, int n_act) 
 __global__ void k_batch_set_steps(const BatchEntry* __restrict__ ents, const long long* __restrict__ v,
                                   int n) {
   const int q = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-  if (q < n) *ents[q].p.step = v[q];
+  if (q < n) *ents[q].p.step = v[q] - 1;   // the first H pass counts up to it
 }
 
 // ---------------------------------------------------------------------------
@@ -2059,6 +2071,19 @@ __global__ void k_batch_set_steps(const BatchEntry* __restrict__ ents, const lon
 // per frequency and plane cell) are read and written once per kDftK steps
 // instead of every step.  The additions happen in the same order as one
 // step at a time (acc, then step lo, lo+1, ...), so the sums are unchanged.
+// (Pointers as RFX_G: the parameters may come from device memory.)
+__device__ __forceinline__ double2 ld2(const double2* base, long long idx) {
+  typedef double v2 __attribute__((ext_vector_type(2)));
+  const v2 v = ((const RFX_G v2*)base)[idx];
+  return make_double2(v.x, v.y);
+}
+__device__ __forceinline__ void st2(double2* base, long long idx, double2 d) {
+  typedef double v2 __attribute__((ext_vector_type(2)));
+  v2 v;
+  v.x = d.x;
+  v.y = d.y;
+  ((RFX_G v2*)base)[idx] = v;
+}
 __device__ __forceinline__ void dft_fold(const PlaneParams& q, long long pidx, long long npts,
                                          long long lo, long long hi, bool hi_in_reg, float xhi) {
   float xs[kDftK];
@@ -2067,21 +2092,22 @@ __device__ __forceinline__ void dft_fold(const PlaneParams& q, long long pidx, l
   for (int m = 0; m < kDftK; ++m) {
     if (m < cnt) {
       const long long st = lo + m;
-      xs[m] = (hi_in_reg && st == hi) ? xhi : q.snap[(st % kDftRing) * npts + pidx];
+      xs[m] = (hi_in_reg && st == hi) ? xhi
+                                      : ((const RFX_G float*)q.snap)[(st % kDftRing) * npts + pidx];
     }
   }
   for (int f0 = 0; f0 < q.nf; f0 += kFoldF) {
     double2 cur[kFoldF];
 #pragma unroll
     for (int u = 0; u < kFoldF; ++u)
-      if (f0 + u < q.nf) cur[u] = q.acc[(long long)(f0 + u) * npts + pidx];
+      if (f0 + u < q.nf) cur[u] = ld2(q.acc, (long long)(f0 + u) * npts + pidx);
 #pragma unroll
     for (int u = 0; u < kFoldF; ++u) {
       if (f0 + u >= q.nf) break;
 #pragma unroll
       for (int m = 0; m < kDftK; ++m) {
         if (m < cnt) {
-          const double2 w = q.tw[(lo + m) * q.nf + f0 + u];
+          const double2 w = ld2(q.tw, (lo + m) * q.nf + f0 + u);
           const double x = (double)xs[m];
           cur[u].x += w.x * x;
           cur[u].y += w.y * x;
@@ -2090,28 +2116,26 @@ __device__ __forceinline__ void dft_fold(const PlaneParams& q, long long pidx, l
     }
 #pragma unroll
     for (int u = 0; u < kFoldF; ++u)
-      if (f0 + u < q.nf) q.acc[(long long)(f0 + u) * npts + pidx] = cur[u];
+      if (f0 + u < q.nf) st2(q.acc, (long long)(f0 + u) * npts + pidx, cur[u]);
   }
 }
 
-__global__ __launch_bounds__(256) void k_dft_plane(PlaneParams q) {
+__device__ __forceinline__ void dft_plane_block(const PlaneParams& q, int block) {
   const long long npts = (long long)q.n1 * q.n2;
-  const long long pidx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  const long long pidx = (long long)block * 256 + threadIdx.x;
   if (pidx >= npts) return;
   const long long n = *q.step;
   if (n < 0 || n >= q.max_steps) return;
   const int u = (int)(pidx / q.n2), v = (int)(pidx % q.n2);
-  int ii[3];
-  const int a1 = q.axis == 0 ? 1 : 0, a2 = q.axis == 2 ? 1 : 2;
-  ii[q.axis] = q.index;
-  ii[a1] = u;
-  ii[a2] = v;
-  const float x = q.fld[((long long)ii[0] * q.ny + ii[1]) * q.nz + ii[2]];
+  const int i = q.axis == 0 ? q.index : u;
+  const int j = q.axis == 0 ? u : q.axis == 1 ? q.index : v;
+  const int k = q.axis == 2 ? q.index : v;
+  const float x = ((const RFX_G float*)q.fld)[((long long)i * q.ny + j) * q.nz + k];
   if (n % kDftK == kDftK - 1) {
     const long long lo = max(*q.acc_from, n - (kDftK - 1));
     dft_fold(q, pidx, npts, lo, n, true, x);
   } else {
-    q.snap[(n % kDftRing) * npts + pidx] = x;
+    ((RFX_G float*)q.snap)[(n % kDftRing) * npts + pidx] = x;
   }
 }
 
@@ -2138,7 +2162,7 @@ __global__ __launch_bounds__(256) void k_dft_flush(PlaneParams q) {
   const long long last = *q.step - 1;
   if (last < 0) return;
   const int slot = (int)(last % kDftK);
-  if (slot == kDftK - 1) return;   // folded by k_dft_plane / k_dft_fold2
+  if (slot == kDftK - 1) return;   // folded by k_monitors / k_dft_fold2
   const long long lo = max(*q.acc_from, last - slot);
   if (lo > last) return;
   dft_fold(q, pidx, npts, lo, last, false, 0.f);
@@ -2166,7 +2190,9 @@ __device__ __forceinline__ void flux_fold(const FluxParams& q, int t, long long 
   for (int m = 0; m < kDftK; ++m) {
     if (m < cnt) {
       const long long st = lo + m;
-      xs[m] = (hi_in_reg && st == hi) ? xhi : q.snap[((st % kDftK) * 4 + t) * npts + pidx];
+      xs[m] = (hi_in_reg && st == hi)
+                  ? xhi
+                  : ((const RFX_G float*)q.snap)[((st % kDftK) * 4 + t) * npts + pidx];
     }
   }
   const double2* tw = t < 2 ? q.twe : q.twh;
@@ -2176,14 +2202,14 @@ __device__ __forceinline__ void flux_fold(const FluxParams& q, int t, long long 
     double2 cur[kFoldF];
 #pragma unroll
     for (int u = 0; u < kFoldF; ++u)
-      if (f0 + u < q.nf) cur[u] = q.acc[((long long)t * q.nf + f0 + u) * npts + pidx];
+      if (f0 + u < q.nf) cur[u] = ld2(q.acc, ((long long)t * q.nf + f0 + u) * npts + pidx);
 #pragma unroll
     for (int u = 0; u < kFoldF; ++u) {
       if (f0 + u >= q.nf) break;
 #pragma unroll
       for (int m = 0; m < kDftK; ++m) {
         if (m < cnt) {
-          const double2 w = tw[(lo + m) * q.nf + f0 + u];
+          const double2 w = ld2(tw, (lo + m) * q.nf + f0 + u);
           const double x = (double)xs[m];
           cur[u].x += w.x * x;
           cur[u].y += w.y * x;
@@ -2192,34 +2218,57 @@ __device__ __forceinline__ void flux_fold(const FluxParams& q, int t, long long 
     }
 #pragma unroll
     for (int u = 0; u < kFoldF; ++u)
-      if (f0 + u < q.nf) q.acc[((long long)t * q.nf + f0 + u) * npts + pidx] = cur[u];
+      if (f0 + u < q.nf) st2(q.acc, ((long long)t * q.nf + f0 + u) * npts + pidx, cur[u]);
   }
 }
 
-__global__ __launch_bounds__(256) void k_flux(FluxParams q) {
+// t: component E1, E2, H1, H2
+__device__ __forceinline__ void flux_block(const FluxParams& q, int block, int t) {
   const long long npts = (long long)q.n1 * q.n2;
-  const long long pidx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  const int t = (int)blockIdx.y;   // component: E1, E2, H1, H2
+  const long long pidx = (long long)block * 256 + threadIdx.x;
   if (pidx >= npts) return;
   const long long n = *q.step;
   if (n < 0 || n >= q.max_steps) return;
   const int u = (int)(pidx / q.n2) + q.lo1, v = (int)(pidx % q.n2) + q.lo2;
-  int ii[3], im[3];
-  const int a1 = q.axis == 0 ? 1 : 0, a2 = q.axis == 2 ? 1 : 2;
-  ii[q.axis] = q.index;
-  im[q.axis] = q.index_m1;
-  ii[a1] = im[a1] = u;
-  ii[a2] = im[a2] = v;
-  const long long c = ((long long)ii[0] * q.ny + ii[1]) * q.nz + ii[2];
-  const long long cm = ((long long)im[0] * q.ny + im[1]) * q.nz + im[2];
-  const float* f = q.f[t];
-  const float x = t < 2 ? f[c] : (f[cm] + f[c]) * 0.5f;
+  const long long step = q.axis == 0 ? (long long)q.ny * q.nz : q.axis == 1 ? q.nz : 1;
+  const int i = q.axis == 0 ? 0 : u, j = q.axis == 0 ? u : q.axis == 1 ? 0 : v;
+  const long long c = ((long long)i * q.ny + j) * q.nz + (q.axis == 2 ? 0 : v);
+  const RFX_G float* const f = (const RFX_G float*)(t == 0   ? q.f[0]
+                                                    : t == 1 ? q.f[1]
+                                                    : t == 2 ? q.f[2]
+                                                             : q.f[3]);
+  const float a = f[c + q.index * step];
+  const float x = t < 2 ? a : (f[c + q.index_m1 * step] + a) * 0.5f;
   const int slot = (int)(n % kDftK);
   if (slot == kDftK - 1) {
     const long long lo = max(*q.acc_from, n - (kDftK - 1));
     flux_fold(q, t, pidx, npts, lo, n, true, x);
   } else {
-    q.snap[((long long)slot * 4 + t) * npts + pidx] = x;
+    ((RFX_G float*)q.snap)[((long long)slot * 4 + t) * npts + pidx] = x;
+  }
+}
+
+// Every DFT plane, flux monitor and NTFF face of a plan in one launch: entry
+// e takes the blocks from start[e] on (a plane's points, or a face's points
+// once per component).  The faces are small against the chip (209^2 points
+// are 171 workgroups), so a launch each was bound by its own start: 7 of them
+// cost 43 us of a 206 us step at 209^3, all in one 17 us.
+struct MonEntry {
+  int flux;          // f, else p
+  PlaneParams p;
+  FluxParams f;
+};
+
+__global__ __launch_bounds__(256) void k_monitors(const MonEntry* __restrict__ ents,
+                                                  const int* __restrict__ start, int n) {
+  const int b = (int)blockIdx.x, e = batch_instance(start, n, b);
+  const MonEntry& m = ents[e];
+  const int lb = b - gld(start, e);
+  if (m.flux) {
+    const int nb = (int)(((long long)m.f.n1 * m.f.n2 + 255) / 256);
+    flux_block(m.f, lb % nb, lb / nb);
+  } else {
+    dft_plane_block(m.p, lb);
   }
 }
 
@@ -2231,7 +2280,7 @@ __global__ __launch_bounds__(256) void k_flux_flush(FluxParams q) {
   const long long last = *q.step - 1;
   if (last < 0) return;
   const int slot = (int)(last % kDftK);
-  if (slot == kDftK - 1) return;   // folded by k_flux
+  if (slot == kDftK - 1) return;   // folded by k_monitors
   const long long lo = max(*q.acc_from, last - slot);
   if (lo > last) return;
   flux_fold(q, (int)blockIdx.y, pidx, npts, lo, last, false, 0.f);
@@ -3778,12 +3827,8 @@ __global__ void k_set_step(long long* step, long long value) {
   if (blockIdx.x == 0 && threadIdx.x == 0) *step = value;
 }
 
-__global__ void k_advance(long long* step) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) *step = *step + 1;
-}
-
-__global__ void k_advance2(long long* step) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) *step = *step + 2;
+__global__ void k_advance(long long* step, int by) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *step = *step + by;
 }
 
 }  // namespace
@@ -3842,6 +3887,9 @@ struct rfxh_plan {
   std::vector<int> plane_comp;
   std::vector<FluxParams> fluxes;
   std::vector<int> flux_comp;     // 4 field components per monitor
+  MonEntry* mon = nullptr;        // k_monitors' entries on set 0, then on set 1 (device)
+  int* mon_start = nullptr;       // their first blocks
+  int mon_blocks = 0;
   std::vector<void*> owned;     // device allocations owned by the plan
   long long max_steps = 0;
   hipStream_t cap_stream = nullptr;
@@ -3935,20 +3983,48 @@ long long march_blocks(const KParams& kp, int rows, int want_seg, MarchIO* io, i
   return tiles * nseg;
 }
 
-// DFT-plane and flux-monitor kernels on field set `set` (after the step).
+// DFT planes, flux monitors and NTFF faces on field set `set` (after the step).
 void launch_accumulators(rfxh_plan* pl, hipStream_t s, int set) {
-  for (size_t q = 0; q < pl->planes.size(); ++q) {
-    PlaneParams pp = pl->planes[q];
-    pp.fld = pl->set[set][pl->plane_comp[q]];
-    const long long npts = (long long)pp.n1 * pp.n2;
-    hipLaunchKernelGGL(k_dft_plane, dim3((unsigned)((npts + 255) / 256)), dim3(256), 0, s, pp);
+  const int n = (int)(pl->planes.size() + pl->fluxes.size());
+  if (n > 0)
+    hipLaunchKernelGGL(k_monitors, dim3((unsigned)pl->mon_blocks), dim3(256), 0, s,
+                       pl->mon + set * n, pl->mon_start, n);
+}
+
+// The monitors' table for k_monitors: the entries on field set 0, then on set 1.
+int monitor_table(rfxh_plan* pl) {
+  const size_t np = pl->planes.size(), n = np + pl->fluxes.size();
+  if (n == 0) return 0;
+  std::vector<MonEntry> ents(2 * n);
+  std::vector<int> start(n + 1, 0);
+  for (size_t e = 0; e < n; ++e) {
+    long long nb;
+    if (e < np) {
+      nb = ((long long)pl->planes[e].n1 * pl->planes[e].n2 + 255) / 256;
+    } else {
+      const FluxParams& f = pl->fluxes[e - np];
+      nb = 4 * (((long long)f.n1 * f.n2 + 255) / 256);
+    }
+    if (start[e] + nb > 0x7fffffffLL) return fail(RFXH_EINVAL, "monitors too large");
+    start[e + 1] = start[e] + (int)nb;
+    for (int set = 0; set < 2; ++set) {
+      MonEntry& m = ents[set * n + e];
+      std::memset(&m, 0, sizeof(m));
+      if (!pl->set[set][0]) continue;
+      if (e < np) {
+        m.p = pl->planes[e];
+        m.p.fld = pl->set[set][pl->plane_comp[e]];
+      } else {
+        m.flux = 1;
+        m.f = pl->fluxes[e - np];
+        for (int t = 0; t < 4; ++t) m.f.f[t] = pl->set[set][pl->flux_comp[4 * (e - np) + t]];
+      }
+    }
   }
-  for (size_t q = 0; q < pl->fluxes.size(); ++q) {
-    FluxParams fp = pl->fluxes[q];
-    for (int t = 0; t < 4; ++t) fp.f[t] = pl->set[set][pl->flux_comp[4 * q + t]];
-    const long long npts = (long long)fp.n1 * fp.n2;
-    hipLaunchKernelGGL(k_flux, dim3((unsigned)((npts + 255) / 256), 4), dim3(256), 0, s, fp);
-  }
+  pl->mon_blocks = start[n];
+  int rc = dev_copy(pl, ents.data(), ents.size(), &pl->mon);
+  if (rc == 0) rc = dev_copy(pl, start.data(), start.size(), &pl->mon_start);
+  return rc;
 }
 
 // Start of a run at step0: steps before it are already folded into the
@@ -4121,9 +4197,16 @@ int launch_step(rfxh_plan* pl, hipStream_t s, hipEvent_t* ev, int from) {
   if (ev) HIPCHK(hipEventRecord(ev[2], s));
   launch_accumulators(pl, s, to);
   if (ev) HIPCHK(hipEventRecord(ev[3], s));
-  hipLaunchKernelGGL(k_advance, dim3(1), dim3(64), 0, s, pl->kp.step);
+  if (pl->fused) hipLaunchKernelGGL(k_advance, dim3(1), dim3(64), 0, s, pl->kp.step, 1);
   HIPCHK(hipGetLastError());
   return 0;
+}
+
+// The step counter names the current step while its kernels run.  The H pass
+// of a two-pass step counts up to it, so such steps start from one less and a
+// run of them ends on its last step; the single-launch steps count after.
+void advance(rfxh_plan* pl, hipStream_t s, int by) {
+  hipLaunchKernelGGL(k_advance, dim3(1), dim3(64), 0, s, pl->kp.step, by);
 }
 
 // Tiles and x segments of the temporal-blocked march.  Automatic segments:
@@ -4219,7 +4302,7 @@ int launch_tb(rfxh_plan* pl, hipStream_t s, hipEvent_t* ev, int from) {
     hipLaunchKernelGGL(k_dft_fold2, dim3((unsigned)((npts + 255) / 256)), dim3(256), 0, s, pp);
   }
   if (ev) HIPCHK(hipEventRecord(ev[3], s));
-  hipLaunchKernelGGL(k_advance2, dim3(1), dim3(64), 0, s, kp.step);
+  advance(pl, s, 2);
   HIPCHK(hipGetLastError());
   return 0;
 }
@@ -4980,6 +5063,7 @@ int rfxh_plan_create(const rfxh_desc* d, rfxh_plan** out) {
       for (int t = 0; t < 4; ++t) pl->flux_comp.push_back(kNtffComp[ax][t]);
     }
   }
+  if ((rc = monitor_table(pl))) return bail(rc);
   // workgroup order (RFXH_ORDER = flat (default) | bands, for comparisons;
   // rfxh_set_variant changes it later)
   const char* ord = std::getenv("RFXH_ORDER");
@@ -5058,8 +5142,10 @@ static int run_tb(rfxh_plan* pl, hipStream_t s, int64_t n_steps, int use_graph) 
       pl->cur ^= 1;
     }
     if (n_steps & 1) {
+      advance(pl, s, -1);
       const int rc = launch_step(pl, s, nullptr, pl->cur);
       if (rc) return rc;
+      advance(pl, s, 1);
     }
     dft_flush(pl, s);
     HIPCHK(hipGetLastError());
@@ -5102,8 +5188,10 @@ static int run_tb(rfxh_plan* pl, hipStream_t s, int64_t n_steps, int use_graph) 
     pl->cur ^= 1;
   }
   if (done < n_steps) {
+    advance(pl, pl->cap_stream, -1);
     const int rc = launch_step(pl, pl->cap_stream, nullptr, pl->cur);
     if (rc) return rc;
+    advance(pl, pl->cap_stream, 1);
   }
   dft_flush(pl, pl->cap_stream);
   HIPCHK(hipGetLastError());
@@ -5129,6 +5217,7 @@ int rfxh_run(rfxh_plan* pl, int64_t step0, int64_t n_steps, void* stream, int us
   }
   if (pl->tb) return run_tb(pl, s, n_steps, use_graph);
   const int flip = pl->fused ? 1 : 0;
+  if (!pl->fused) advance(pl, s, -1);
   if (!use_graph || pl->timing || n_steps < pl->graph_chunk) {
     // timing: sample up to kTimingSamples evenly spaced steps; the host does
     // not wait inside the loop, so the queue stays full and each event pair
@@ -5143,6 +5232,7 @@ int rfxh_run(rfxh_plan* pl, int64_t step0, int64_t n_steps, void* stream, int us
       if (rc) return rc;
       pl->cur ^= flip;
     }
+    if (!pl->fused) advance(pl, s, 1);
     dft_flush(pl, s);
     HIPCHK(hipGetLastError());
     if (n_samples) return collect_timing(pl, n_samples);
@@ -5182,6 +5272,7 @@ int rfxh_run(rfxh_plan* pl, int64_t step0, int64_t n_steps, void* stream, int us
     if (rc) return rc;
     pl->cur ^= flip;
   }
+  if (!pl->fused) advance(pl, pl->cap_stream, 1);
   dft_flush(pl, pl->cap_stream);
   HIPCHK(hipGetLastError());
   HIPCHK(hipEventRecord(pl->ev_out, pl->cap_stream));
@@ -5362,7 +5453,7 @@ int rfxh_run_record_ex(rfxh_plan* pl, int64_t step0, int64_t n_steps, const rfxh
   if (!d_rec) return fail(RFXH_EINVAL, "record buffer missing");
   hipStream_t s = static_cast<hipStream_t>(stream);
   const RegionParams rp = region_params(region);
-  hipLaunchKernelGGL(k_set_step, dim3(1), dim3(64), 0, s, pl->kp.step, (long long)step0);
+  hipLaunchKernelGGL(k_set_step, dim3(1), dim3(64), 0, s, pl->kp.step, (long long)step0 - 1);
   dft_begin(pl, s, step0);
   // two-pass sub-steps in place on the current set, with the record taken
   // between the H and the E update (E^n and H^{n+1/2} both in memory)
@@ -5382,8 +5473,8 @@ int rfxh_run_record_ex(rfxh_plan* pl, int64_t step0, int64_t n_steps, const rfxh
                          rh, rk);
     launch_pass(pl, s, kp, ps, 1, pl->cur);
     launch_accumulators(pl, s, pl->cur);
-    hipLaunchKernelGGL(k_advance, dim3(1), dim3(64), 0, s, pl->kp.step);
   }
+  advance(pl, s, 1);
   dft_flush(pl, s);
   HIPCHK(hipGetLastError());
   return RFXH_OK;
@@ -5695,8 +5786,6 @@ int batch_step(rfxh_batch* b, hipStream_t s, int n_act) {
     rfxh_plan* pl = b->plans[b->order[q]];
     launch_accumulators(pl, s, pl->cur);
   }
-  hipLaunchKernelGGL(k_batch_advance, dim3((unsigned)((n_act + 63) / 64)), dim3(64), 0, s, b->d_ents,
-                     n_act);
   HIPCHK(hipGetLastError());
   return 0;
 }
@@ -5831,6 +5920,7 @@ int rfxh_batch_run(rfxh_batch* b, const int64_t* step0, const int64_t* n_steps, 
       if (rc) return rc;
     }
   }
+  hipLaunchKernelGGL(k_batch_advance, dim3((unsigned)((n + 63) / 64)), dim3(64), 0, w, b->d_ents, n);
   for (int q = 0; q < n; ++q) dft_flush(b->plans[q], w);
   HIPCHK(hipGetLastError());
   if (use_graph) {
@@ -5895,9 +5985,8 @@ int rfxh_batch_run_record(rfxh_batch* b, const int64_t* step0, const int64_t* n_
                        b->d_xstart, act);
     if (accumulate)
       for (int r = 0; r < act; ++r) launch_accumulators(b->plans[order[r]], s, b->plans[order[r]]->cur);
-    hipLaunchKernelGGL(k_batch_advance, dim3((unsigned)((act + 63) / 64)), dim3(64), 0, s,
-                       b->d_xents, act);
   }
+  hipLaunchKernelGGL(k_batch_advance, dim3((unsigned)((na + 63) / 64)), dim3(64), 0, s, b->d_xents, na);
   if (accumulate)
     for (int q : order) dft_flush(b->plans[q], s);
   HIPCHK(hipGetLastError());
