@@ -131,6 +131,17 @@ struct PsiIO {
   int pol_lo[3], pol_n[3];
 };
 
+// CPML memory of one field set and the profiles, from one base each: face f's
+// four terms (H0, H1, E0, E1) lie at psi + foff[f] + t * fs[f] in the slab
+// order of psi_idx, its profile row l is prof[poff[f] + l] = (b, c,
+// 1/kappa - 1, 0).
+struct SlabIO {
+  float* psi;
+  const float4* prof;
+  unsigned foff[6], fs[6];
+  int poff[6];
+};
+
 constexpr int kDftK = 16;   // steps staged per fold of the DFT-plane accumulators
 // ring slots of a DFT plane: two groups of kDftK, so a two-step sweep can
 // stage the first step of the next group before the fold of the current one
@@ -356,6 +367,76 @@ __device__ __forceinline__ void point_ops(const KParams& p, unsigned cell, float
   }
 }
 
+// One axis of a cell's CPML correction where the slabs of an axis do not
+// meet (a cell is in at most one per axis): its memory, profile and place,
+// loaded by slab_load before the cell's fields are waited for.
+// The passes spend their time waiting for loads, and with rows of a few
+// hundred cells a third of the wavefronts hold cells of a z slab: loading the
+// memory only after the curl gave those a second and third wait each, per
+// cell of a column (223x165x141 with 8 layers: 68 -> 61 us a step, of which
+// 52 without CPML; 326x326x146: 283 -> 268, one cell a thread).
+struct SlabAx {
+  bool in;
+  float s0, s1, inv;
+  float4 pr;
+  unsigned q, fs;   // element of the first term, distance to the second
+};
+
+template <bool E, int A>
+__device__ __forceinline__ void slab_load(const KParams& p, const SlabIO& cm, int i, int j, int k,
+                                          SlabAx& s) {
+  const int pos = A == 0 ? i : A == 1 ? j : k;
+  const bool lo = pos < p.slo[A];
+  s.in = lo | (pos >= p.shi[A]);
+  s.s0 = s.s1 = s.inv = 0.f;
+  s.pr = make_float4(0.f, 0.f, 0.f, 0.f);
+  s.q = s.fs = 0;
+  if (s.in) {
+    const int l = lo ? pos : pos - p.shi[A], n = lo ? p.cn[2 * A] : p.cn[2 * A + 1];
+    const unsigned fs = lo ? cm.fs[2 * A] : cm.fs[2 * A + 1];
+    s.fs = fs;
+    s.q = (lo ? cm.foff[2 * A] : cm.foff[2 * A + 1]) + (E ? 2u * fs : 0u) +
+          (unsigned)psi_idx(2 * A, l, i, j, k, n, p.ny, p.nz);
+    s.pr = gld(cm.prof, (lo ? cm.poff[2 * A] : cm.poff[2 * A + 1]) + l);
+    s.inv = lo ? p.cinv[2 * A] : p.cinv[2 * A + 1];
+    s.s0 = ldf(cm.psi, s.q);
+    s.s1 = ldf(cm.psi, s.q + fs);
+  }
+}
+
+// The three axes of a cell (in.in all false outside the slabs).
+template <bool E>
+__device__ __forceinline__ void slabs_load(const KParams& p, const SlabIO& cm, int i, int j, int k,
+                                           SlabAx (&s)[3]) {
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    s[a].in = false;
+    s[a].s0 = s[a].s1 = s[a].inv = 0.f;
+    s[a].pr = make_float4(0.f, 0.f, 0.f, 0.f);
+    s[a].q = s[a].fs = 0;
+  }
+  // (a column's cells past the last plane are in no slab)
+  if (i < p.nx && in_slab(p, i, j, k)) {
+    slab_load<E, 0>(p, cm, i, j, k, s[0]);
+    slab_load<E, 1>(p, cm, i, j, k, s[1]);
+    slab_load<E, 2>(p, cm, i, j, k, s[2]);
+  }
+}
+
+// New memory of one axis from the two differences; d0, d1 the corrections
+// (the products and sums of the general path).
+__device__ __forceinline__ void slab_step(const SlabIO& cm, const SlabAx& s, float co, float g0,
+                                          float g1, float& d0, float& d1) {
+  g0 *= s.inv;
+  g1 *= s.inv;
+  const float s0 = fmaf(s.pr.y, g0, s.pr.x * s.s0), s1 = fmaf(s.pr.y, g1, s.pr.x * s.s1);
+  stf(cm.psi, s.q, s0);
+  stf(cm.psi, s.q + s.fs, s1);
+  const float ck = co * s.pr.z;
+  d0 = fmaf(ck, g0, co * s0);
+  d1 = fmaf(ck, g1, co * s1);
+}
+
 // ---------------------------------------------------------------------------
 // H at one cell from values: H^{n+1/2} = H^{n-1/2} - ch curl_fwd E^n
 // (yee.py:272-289, graded :429-451) plus the CPML-H correction
@@ -363,11 +444,12 @@ __device__ __forceinline__ void point_ops(const KParams& p, unsigned cell, float
 // past the last cell, yee.py:121-128) come in as values; CPML memory is
 // read from ps.hr and, when WRITE, the new memory is stored into ps.hw.
 // ---------------------------------------------------------------------------
-template <bool GRADED, bool WRITE>
+template <bool GRADED, bool WRITE, bool SLAB = false>
 __device__ __forceinline__ float3 h_core(const KParams& p, const PsiIO& ps, int i, int j, int k,
                                          float ch, float ex, float ey, float ez, float ex_j,
                                          float ez_j, float ex_k, float ey_k, float ey_i, float ez_i,
-                                         float hx, float hy, float hz, bool wr = true) {
+                                         float hx, float hy, float hz, bool wr = true,
+                                         const SlabIO* cm = nullptr, const SlabAx* sl = nullptr) {
   float ix, iy, iz;
   if (GRADED) {
     ix = gld(p.inv_h[0], i);
@@ -379,7 +461,26 @@ __device__ __forceinline__ float3 h_core(const KParams& p, const PsiIO& ps, int 
   hx = hx - ch * ((ez_j - ez) * iy - (ey_k - ey) * iz);
   hy = hy - ch * ((ex_k - ex) * iz - (ez_i - ez) * ix);
   hz = hz - ch * ((ey_i - ey) * ix - (ex_j - ex) * iy);
-  if (in_slab(p, i, j, k)) {
+  if (SLAB) {
+    if (sl[0].in | sl[1].in | sl[2].in) {
+      float d0, d1;
+      if (sl[0].in) {
+        slab_step(*cm, sl[0], ch, ez_i - ez, ey_i - ey, d0, d1);
+        hy += d0;
+        hz -= d1;
+      }
+      if (sl[1].in) {
+        slab_step(*cm, sl[1], ch, ez_j - ez, ex_j - ex, d0, d1);
+        hx -= d0;
+        hz += d1;
+      }
+      if (sl[2].in) {
+        slab_step(*cm, sl[2], ch, ey_k - ey, ex_k - ex, d0, d1);
+        hx += d0;
+        hy -= d1;
+      }
+    }
+  } else if (in_slab(p, i, j, k)) {
     // keep the CPML pointer and profile loads inside the slab branch: the
     // compiler would otherwise hoist them into every wavefront (and spill
     // them to VGPR lanes), slab cells or not
@@ -532,12 +633,13 @@ __device__ __noinline__ void dispersion_cell(const KParams& p, const PsiIO& ps, 
   }
 }
 
-template <bool GRADED, bool DISP = false>
+template <bool GRADED, bool DISP = false, bool SLAB = false>
 __device__ __forceinline__ float3 e_core_co(const KParams& p, const PsiIO& ps, int i, int j, int k,
                                             unsigned c, float4 co, uint32_t fl, float e0, float e1,
                                             float e2, float hx, float hy, float hz, float hy_i,
                                             float hz_i, float hx_j, float hz_j, float hx_k,
-                                            float hy_k) {
+                                            float hy_k, const SlabIO* cm = nullptr,
+                                            const SlabAx* sl = nullptr) {
   float ix, iy, iz;
   if (GRADED) {
     ix = gld(p.inv_e[0], i);
@@ -559,7 +661,26 @@ __device__ __forceinline__ float3 e_core_co(const KParams& p, const PsiIO& ps, i
     e2 = ca * e2 + cb * ((hy - hy_i) * ix - (hx - hx_j) * iy);
   }
   if (DISP && (fl & RFXH_POLES)) dispersion_cell(p, ps, i, j, k, c, o0, o1, o2, e0, e1, e2);
-  if (in_slab(p, i, j, k)) {
+  if (SLAB) {
+    if (sl[0].in | sl[1].in | sl[2].in) {
+      float d0, d1;
+      if (sl[0].in) {
+        slab_step(*cm, sl[0], ce, hz - hz_i, hy - hy_i, d0, d1);
+        e1 -= d0;
+        e2 += d1;
+      }
+      if (sl[1].in) {
+        slab_step(*cm, sl[1], ce, hz - hz_j, hx - hx_j, d0, d1);
+        e0 += d0;
+        e2 -= d1;
+      }
+      if (sl[2].in) {
+        slab_step(*cm, sl[2], ce, hy - hy_k, hx - hx_k, d0, d1);
+        e0 -= d0;
+        e1 += d1;
+      }
+    }
+  } else if (in_slab(p, i, j, k)) {
     // keep the CPML pointer and profile loads inside the slab branch: the
     // compiler would otherwise hoist them into every wavefront (and spill
     // them to VGPR lanes), slab cells or not
@@ -621,15 +742,16 @@ __device__ __forceinline__ float3 e_core_co(const KParams& p, const PsiIO& ps, i
   return make_float3(e0, e1, e2);
 }
 
-template <bool GRADED, bool DISP = false>
+template <bool GRADED, bool DISP = false, bool SLAB = false>
 __device__ __forceinline__ float3 e_core(const KParams& p, const PsiIO& ps, int i, int j, int k,
                                          unsigned c, unsigned m, float e0, float e1, float e2,
                                          float hx, float hy, float hz, float hy_i, float hz_i,
-                                         float hx_j, float hz_j, float hx_k, float hy_k) {
+                                         float hx_j, float hz_j, float hx_k, float hy_k,
+                                         const SlabIO* cm = nullptr, const SlabAx* sl = nullptr) {
   // one 16-byte row carries everything the E update needs
   const float4 ec = gld(p.ecoef, (int)m);
-  return e_core_co<GRADED, DISP>(p, ps, i, j, k, c, ec, __float_as_uint(ec.w), e0, e1, e2, hx, hy, hz,
-                           hy_i, hz_i, hx_j, hz_j, hx_k, hy_k);
+  return e_core_co<GRADED, DISP, SLAB>(p, ps, i, j, k, c, ec, __float_as_uint(ec.w), e0, e1, e2, hx,
+                                       hy, hz, hy_i, hz_i, hx_j, hz_j, hx_k, hy_k, cm, sl);
 }
 
 // E at one cell reading E^n from Eo, storing E^{n+1} into En.
@@ -1868,14 +1990,16 @@ __global__ __launch_bounds__(kWG) void k_update_e(KParams p, PsiIO ps) {
 // Column variants of the two passes: each thread updates NP consecutive
 // cells along x.  The x-neighbour one cell needs is the next (H pass) or
 // previous (E pass) cell's own value, already in registers, so x-neighbours
-// are re-read once per column instead of once per cell, and each thread
-// has NP cells' loads in flight at once.
+// are re-read once per column instead of once per cell.  NP = 1 is the
+// default: what bounds the passes is memory (36 bytes a cell in the H pass, 38
+// in the E pass; 7-8 TB/s where the state fits the 256 MB cache, 5-6 from
+// HBM), which many short wavefronts keep busier than few long ones.
 // ---------------------------------------------------------------------------
 // Cells i0 .. i0+NP-1 of the column, updating only those below iend
 // (iend <= nx; the others are read as neighbours only).
 template <bool GRADED, int NP, bool ONE_MU>
-__device__ __forceinline__ void col_h(const KParams& p, const PsiIO& ps, int i0, int j, int k,
-                                      int iend) {
+__device__ __forceinline__ void col_h(const KParams& p, const PsiIO& ps, const SlabIO& cm, int i0,
+                                      int j, int k) {
   const unsigned P = (unsigned)p.plane;
   const bool hj = j + 1 < p.ny, hk = k + 1 < p.nz;
   const unsigned c0 = ((unsigned)i0 * (unsigned)p.ny + (unsigned)j) * (unsigned)p.nz + (unsigned)k;
@@ -1883,6 +2007,9 @@ __device__ __forceinline__ void col_h(const KParams& p, const PsiIO& ps, int i0,
   float ex[NP + 1], ey[NP + 1], ez[NP + 1], exj[NP], ezj[NP], exk[NP], eyk[NP];
   float hx[NP], hy[NP], hz[NP];
   unsigned m[NP];
+  SlabAx sl[NP][3];
+#pragma unroll
+  for (int q = 0; q < NP; ++q) slabs_load<false>(p, cm, i0 + q, j, k, sl[q]);
 #pragma unroll
   for (int q = 0; q < NP; ++q) {
     const bool in = i0 + q < p.nx;
@@ -1910,14 +2037,14 @@ __device__ __forceinline__ void col_h(const KParams& p, const PsiIO& ps, int i0,
   }
 #pragma unroll
   for (int q = 0; q < NP; ++q) {
-    if (i0 + q >= iend) break;
+    if (i0 + q >= p.nx) break;
     const float exj_ = hj ? exj[q] : 0.f, ezj_ = hj ? ezj[q] : 0.f;
     const float exk_ = hk ? exk[q] : 0.f, eyk_ = hk ? eyk[q] : 0.f;
     const float eyi = (q + 1 < NP) ? ((i0 + q + 1 < p.nx) ? ey[q + 1] : 0.f) : ey[NP];
     const float ezi = (q + 1 < NP) ? ((i0 + q + 1 < p.nx) ? ez[q + 1] : 0.f) : ez[NP];
-    const float3 h = h_core<GRADED, true>(p, ps, i0 + q, j, k,
-                                          ONE_MU ? p.ch_all : ld_ch(p.coef, m[q]), ex[q], ey[q], ez[q],
-                                          exj_, ezj_, exk_, eyk_, eyi, ezi, hx[q], hy[q], hz[q]);
+    const float3 h = h_core<GRADED, true, true>(
+        p, ps, i0 + q, j, k, ONE_MU ? p.ch_all : ld_ch(p.coef, m[q]), ex[q], ey[q], ez[q], exj_,
+        ezj_, exk_, eyk_, eyi, ezi, hx[q], hy[q], hz[q], true, &cm, sl[q]);
     const unsigned c = c0 + (unsigned)q * P;
     stf(p.f[3], c, h.x);
     stf(p.f[4], c, h.y);
@@ -1926,8 +2053,8 @@ __device__ __forceinline__ void col_h(const KParams& p, const PsiIO& ps, int i0,
 }
 
 template <bool GRADED, int NP, bool DISP>
-__device__ __forceinline__ void col_e(const KParams& p, const PsiIO& ps, int i0, int j, int k,
-                                      int iend) {
+__device__ __forceinline__ void col_e(const KParams& p, const PsiIO& ps, const SlabIO& cm, int i0,
+                                      int j, int k) {
   const unsigned P = (unsigned)p.plane;
   const bool bj = j > 0, bk = k > 0;
   const unsigned c0 = ((unsigned)i0 * (unsigned)p.ny + (unsigned)j) * (unsigned)p.nz + (unsigned)k;
@@ -1936,6 +2063,9 @@ __device__ __forceinline__ void col_e(const KParams& p, const PsiIO& ps, int i0,
   float hx[NP + 1], hy[NP + 1], hz[NP + 1], hxj[NP], hzj[NP], hxk[NP], hyk[NP];
   float e0[NP], e1[NP], e2[NP];
   unsigned m[NP];
+  SlabAx sl[NP][3];
+#pragma unroll
+  for (int q = 0; q < NP; ++q) slabs_load<true>(p, cm, i0 + q, j, k, sl[q]);
   {
     const bool in = i0 > 0;
     const unsigned c = in ? c0 - P : c0;
@@ -1963,48 +2093,42 @@ __device__ __forceinline__ void col_e(const KParams& p, const PsiIO& ps, int i0,
   }
 #pragma unroll
   for (int q = 0; q < NP; ++q) {
-    if (i0 + q >= iend) break;
+    if (i0 + q >= p.nx) break;
     const unsigned c = c0 + (unsigned)q * P;
     const float hxj_ = bj ? hxj[q] : 0.f, hzj_ = bj ? hzj[q] : 0.f;
     const float hxk_ = bk ? hxk[q] : 0.f, hyk_ = bk ? hyk[q] : 0.f;
-    const float3 e = e_core<GRADED, DISP>(p, ps, i0 + q, j, k, c, m[q], e0[q], e1[q], e2[q],
-                                          hx[q + 1], hy[q + 1], hz[q + 1], hy[q], hz[q], hxj_, hzj_,
-                                          hxk_, hyk_);
+    const float3 e = e_core<GRADED, DISP, true>(p, ps, i0 + q, j, k, c, m[q], e0[q], e1[q], e2[q],
+                                                hx[q + 1], hy[q + 1], hz[q + 1], hy[q], hz[q], hxj_,
+                                                hzj_, hxk_, hyk_, &cm, sl[q]);
     stf(p.f[0], c, e.x);
     stf(p.f[1], c, e.y);
     stf(p.f[2], c, e.z);
   }
 }
 
-// The CPML pointers come through device memory (psp) rather than as
-// kernel arguments: as arguments the compiler loads all 48 of them up front
-// and spills them to VGPR lanes in every wavefront, although only the
-// wavefronts with slab cells use them.
 // ONE_MU: every material has the same ch (p.ch_all), so the H pass reads
 // no material id.
 template <bool GRADED, int NP, bool ONE_MU>
-__global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(NP == 2 ? 8 : 1)))
-void k_update_h_col(KParams p, const PsiIO* __restrict__ psp) {
+__global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(NP == 1 ? 8 : NP == 2 ? 5 : 1)))
+void k_update_h_col(KParams p, SlabIO cm, const PsiIO* __restrict__ psp) {
   count_step(p);
   const PsiIO& ps = *psp;
   int ib, j, k;
   if (!cell_at(p, xcd_remap((int)blockIdx.x, (int)gridDim.x), ib, j, k, (p.nx + NP - 1) / NP))
     return;
-  col_h<GRADED, NP, ONE_MU>(p, ps, ib * NP, j, k, p.nx);
+  col_h<GRADED, NP, ONE_MU>(p, ps, cm, ib * NP, j, k);
 }
 
-// 2-cell columns: an occupancy target of 7 wavefronts per SIMD.  With
-// 512-thread workgroups, holding the kernel to 64 VGPRs (8 wavefronts) was
-// 3.7 % faster than the compiler's own choice; with 256-thread workgroups
-// a target of 7 is 0.7-1 % faster than 8 and the unconstrained build.
+// Occupancy targets: one cell a thread fits 64 VGPRs (8 wavefronts per SIMD)
+// with its slab memory in flight, 2-cell columns 96 (5) without spilling.
 template <bool GRADED, int NP, bool DISP>
-__global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(NP == 2 ? 7 : 1)))
-void k_update_e_col(KParams p, const PsiIO* __restrict__ psp) {
+__global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(NP == 1 && !DISP ? 8 : NP == 2 ? 5 : 1)))
+void k_update_e_col(KParams p, SlabIO cm, const PsiIO* __restrict__ psp) {
   const PsiIO& ps = *psp;
   int ib, j, k;
   if (!cell_at(p, xcd_remap_rev((int)blockIdx.x, (int)gridDim.x), ib, j, k, (p.nx + NP - 1) / NP))
     return;
-  col_e<GRADED, NP, DISP>(p, ps, ib * NP, j, k, p.nx);
+  col_e<GRADED, NP, DISP>(p, ps, cm, ib * NP, j, k);
 }
 
 // ---------------------------------------------------------------------------
@@ -3873,6 +3997,7 @@ struct rfxh_plan {
   bool march = false;           // the ping-pong step uses the marching kernel
   int march_seg = 0;            // x segments of the marching kernel (0: automatic)
   int march_tile = 0;           // index into kMarchRows
+  bool slabs_meet = false;      // CPML slabs of one axis overlap (or their memory passes 4 GB)
   int ncol = 1;                 // two-pass step: cells per thread along x (1, 2, 3, 4)
   bool wmarch = false;          // the ping-pong step uses the wave-march kernel
   int wmarch_seg = 0;           // its x segments (0: automatic)
@@ -4061,30 +4186,43 @@ void dft_flush(rfxh_plan* pl, hipStream_t s) {
   hipLaunchKernelGGL(k_set_acc_from, dim3(1), dim3(64), 0, s, pl->acc_from, pl->kp.step);
 }
 
+SlabIO slab_io(const rfxh_plan* pl, int set) {
+  SlabIO c;
+  std::memset(&c, 0, sizeof(c));
+  c.psi = pl->psi_base ? pl->psi_base + set * pl->psi_set : nullptr;
+  c.prof = pl->cprof;
+  for (int f = 0; f < 6; ++f) {
+    c.foff[f] = pl->psi_foff[f];
+    c.fs[f] = pl->psi_fs[f];
+    c.poff[f] = pl->cprof_off[f];
+  }
+  return c;
+}
+
+// Columns of NP cells (NP = 0: plans whose CPML slabs of an axis meet; one
+// cell a thread, its memory loaded face by face).
 template <int PASS, bool GRADED, int NP>
 void launch_pass_n(const rfxh_plan* pl, hipStream_t s, const KParams& kp, const PsiIO& ps,
                    int set) {
-  const dim3 g = NP == 1 ? pl->grid : pl->grid_col, blk = pl->block;
-  if (NP == 1) {
+  const dim3 g = NP < 2 ? pl->grid : pl->grid_col, blk = pl->block;
+  const bool one_mu = kp.ch_all > 0.f, disp = pl->n_pole > 0 || pl->aniso;
+  if constexpr (NP == 0) {
     if (PASS == 0) {
-      if (kp.ch_all > 0.f) hipLaunchKernelGGL((k_update_h<GRADED, true>), g, blk, 0, s, kp, ps);
+      if (one_mu) hipLaunchKernelGGL((k_update_h<GRADED, true>), g, blk, 0, s, kp, ps);
       else hipLaunchKernelGGL((k_update_h<GRADED, false>), g, blk, 0, s, kp, ps);
+    } else {
+      if (disp) hipLaunchKernelGGL((k_update_e<GRADED, true>), g, blk, 0, s, kp, ps);
+      else hipLaunchKernelGGL((k_update_e<GRADED, false>), g, blk, 0, s, kp, ps);
     }
-    else if (pl->n_pole > 0 || pl->aniso)
-      hipLaunchKernelGGL((k_update_e<GRADED, true>), g, blk, 0, s, kp, ps);
-    else hipLaunchKernelGGL((k_update_e<GRADED, false>), g, blk, 0, s, kp, ps);
   } else {
     const PsiIO* psp = pl->d_psio + set;
+    const SlabIO cm = slab_io(pl, set);
     if (PASS == 0) {
-      if (kp.ch_all > 0.f)
-        hipLaunchKernelGGL((k_update_h_col<GRADED, NP, true>), g, blk, 0, s, kp, psp);
-      else
-        hipLaunchKernelGGL((k_update_h_col<GRADED, NP, false>), g, blk, 0, s, kp, psp);
+      if (one_mu) hipLaunchKernelGGL((k_update_h_col<GRADED, NP, true>), g, blk, 0, s, kp, cm, psp);
+      else hipLaunchKernelGGL((k_update_h_col<GRADED, NP, false>), g, blk, 0, s, kp, cm, psp);
     } else {
-      if (pl->n_pole > 0 || pl->aniso)
-        hipLaunchKernelGGL((k_update_e_col<GRADED, NP, true>), g, blk, 0, s, kp, psp);
-      else
-        hipLaunchKernelGGL((k_update_e_col<GRADED, NP, false>), g, blk, 0, s, kp, psp);
+      if (disp) hipLaunchKernelGGL((k_update_e_col<GRADED, NP, true>), g, blk, 0, s, kp, cm, psp);
+      else hipLaunchKernelGGL((k_update_e_col<GRADED, NP, false>), g, blk, 0, s, kp, cm, psp);
     }
   }
 }
@@ -4092,7 +4230,8 @@ void launch_pass_n(const rfxh_plan* pl, hipStream_t s, const KParams& kp, const 
 template <int PASS, bool GRADED>
 void launch_pass_g(const rfxh_plan* pl, hipStream_t s, const KParams& kp, const PsiIO& ps,
                    int set) {
-  switch (pl->ncol) {
+  switch (pl->slabs_meet ? 0 : pl->ncol) {
+    case 0: launch_pass_n<PASS, GRADED, 0>(pl, s, kp, ps, set); break;
     case 2: launch_pass_n<PASS, GRADED, 2>(pl, s, kp, ps, set); break;
     case 3: launch_pass_n<PASS, GRADED, 3>(pl, s, kp, ps, set); break;
     case 4: launch_pass_n<PASS, GRADED, 4>(pl, s, kp, ps, set); break;
@@ -4812,15 +4951,17 @@ int rfxh_plan_create(const rfxh_desc* d, rfxh_plan** out) {
     if ((rc = dev_copy(pl, tmp.data(), tmp.size(), &ec))) return bail(rc);
     kp.ecoef = ec;
   }
-  // default: the two-pass step with 2-cell columns along x, the fastest
-  // variant measured on MI355X at 533^3 and on the graded workloads;
+  // default: the two-pass step, one cell a thread: with the CPML memory
+  // loaded first its wavefronts are many and short (2-cell columns hold a
+  // third fewer: 65.7 against 62.5 us a step at 222x164x140, 303 against 290
+  // at 325x325x145 graded, 2534 against 2482 at 533^3);
   // RFXH_KERNEL = onecell | fused | march selects another (fused and march
   // need the second field set); rfxh_set_variant changes it later
   const char* kern = std::getenv("RFXH_KERNEL");
   const std::string kname = kern ? kern : "";
   pl->fused = has2 && d->n_pole == 0 && !d->aniso_coef && (kname == "fused" || kname == "march");
   pl->march = has2 && kname == "march";
-  pl->ncol = (pl->fused || kname == "onecell") ? 1 : 2;
+  pl->ncol = 1;
   for (int c = 0; c < 6; ++c) {
     pl->set[0][c] = d->d_f[c];
     pl->set[1][c] = has2 ? d->d_f2[c] : nullptr;
@@ -4856,6 +4997,11 @@ int rfxh_plan_create(const rfxh_desc* d, rfxh_plan** out) {
   if (!prof_rows.empty() && (rc = dev_copy(pl, prof_rows.data(), prof_rows.size(), &pl->cprof)))
     return bail(rc);
   pl->psi_floats = off;
+  // (k_update_*_col find a cell in at most one slab per axis, and index the
+  // memory with 32-bit byte offsets)
+  pl->slabs_meet = off >= (1LL << 30);
+  for (int a = 0; a < 3; ++a)
+    if (kp.cn[2 * a] + kp.cn[2 * a + 1] > N[a]) pl->slabs_meet = true;
   // Dispersive poles: cells whose material flags carry pole bits update their
   // polarisation in the box pol_lo + [0, pol_n)
   if (d->n_pole < 0 || d->n_pole > 16) return bail(fail(RFXH_EINVAL, "n_pole must be 0..16"));
