@@ -106,6 +106,7 @@ struct KParams {
   float ch_all;                  // > 0: every material has this ch (one mu_r), and the
                                  // column H pass reads no material id
   const float4* acoef;           // RFXH_ANISO ids: ca, cb of Ey and of Ez
+  unsigned long long pole_ids;   // material ids with poles (0: none, or an id past 63 has)
 };
 
 struct FusedIO {
@@ -574,63 +575,122 @@ __device__ __forceinline__ float3 h_cell(const KParams& p, const float* const Eo
 //     P_d^{n+1} = alpha P_d^n + beta (E^{n+1} + E^n)
 // before the CPML correction, PEC and point operations.  A cell outside the
 // state box is left alone (the host puts every cell with poles inside it).
-__device__ __noinline__ void dispersion_cell(const KParams& p, const PsiIO& ps, int i, int j,
-                                             int k, unsigned c, float o0, float o1, float o2,
-                                             float& e0, float& e1, float& e2) {
+//
+// poles_load takes the cell's first Lorentz and first Debye pole into
+// registers, so the one-cell E pass has them in flight with the fields; poles
+// past the first of a kind (rare) are read where they are used.  What bounds
+// a dispersive cell is that wait: with every pole read after the curl, in a
+// function call that held 99 registers, the E pass of 181x149x117 cells with
+// a Debye and a Lorentz pole took 57 us; now 29.
+struct Poles {
+  bool on;
+  unsigned r;          // cell of the state box
+  float l[6], d[3];    // first Lorentz pole: P^n, P^{n-1}; first Debye pole: P^n
+  float4 lc, dc;
+};
+
+__device__ __forceinline__ float4 ld4(const float* base, int row) {
+  return gld(reinterpret_cast<const float4*>(base), row);
+}
+
+__device__ __forceinline__ void poles_load(const PsiIO& ps, int i, int j, int k, unsigned m,
+                                           bool on, Poles& a) {
   const int li = i - ps.pol_lo[0], lj = j - ps.pol_lo[1], lk = k - ps.pol_lo[2];
-  if (!ps.pol || li < 0 || lj < 0 || lk < 0 || li >= ps.pol_n[0] || lj >= ps.pol_n[1] ||
-      lk >= ps.pol_n[2])
-    return;
+  a.on = on && ps.pol && li >= 0 && lj >= 0 && lk >= 0 && li < ps.pol_n[0] && lj < ps.pol_n[1] &&
+         lk < ps.pol_n[2];
+  a.r = 0;
+  a.lc = a.dc = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+  for (int t = 0; t < 6; ++t) a.l[t] = 0.f;
+#pragma unroll
+  for (int t = 0; t < 3; ++t) a.d[t] = 0.f;
+  if (!a.on) return;
   const unsigned R = (unsigned)ps.pol_n[0] * (unsigned)ps.pol_n[1] * (unsigned)ps.pol_n[2];
-  const unsigned r = ((unsigned)li * (unsigned)ps.pol_n[1] + (unsigned)lj) * (unsigned)ps.pol_n[2] +
-                     (unsigned)lk;
-  const unsigned m = ldu16(p.mat, c);
-  const float* pc = ps.pcoef + (size_t)m * ps.n_pole * 4;
-  const int nd = ps.n_debye;
-  float d0 = 0.f, d1 = 0.f, d2 = 0.f, ccl = 0.f;
-  for (int q = nd; q < ps.n_pole; ++q) {
-    const float a = pc[4 * q], b = pc[4 * q + 1], cl = pc[4 * q + 2];
-    ccl = pc[4 * q + 3];
-    float* P = ps.pol + (size_t)nd * 3 * R + (size_t)(q - nd) * 6 * R;
-    const float p0 = P[r], p1 = P[R + r], p2 = P[2 * R + r];
-    const float n0 = a * p0 + b * P[3 * R + r] + cl * o0;
-    const float n1 = a * p1 + b * P[4 * R + r] + cl * o1;
-    const float n2 = a * p2 + b * P[5 * R + r] + cl * o2;
-    d0 += n0 - p0;
-    d1 += n1 - p1;
-    d2 += n2 - p2;
-    P[3 * R + r] = p0;
-    P[4 * R + r] = p1;
-    P[5 * R + r] = p2;
-    P[r] = n0;
-    P[R + r] = n1;
-    P[2 * R + r] = n2;
+  a.r = ((unsigned)li * (unsigned)ps.pol_n[1] + (unsigned)lj) * (unsigned)ps.pol_n[2] + (unsigned)lk;
+  const int nd = ps.n_debye, row = (int)m * ps.n_pole;
+  if (nd < ps.n_pole) {
+    const RFX_G float* P = (const RFX_G float*)ps.pol + (size_t)nd * 3 * R;
+    a.lc = ld4(ps.pcoef, row + nd);
+#pragma unroll
+    for (int t = 0; t < 6; ++t) a.l[t] = P[(size_t)t * R + a.r];
   }
   if (nd > 0) {
-    float s0 = 0.f, s1 = 0.f, s2 = 0.f;
-    for (int q = 0; q < nd; ++q) {
-      const float cc = pc[4 * q + 2];
-      const float* P = ps.pol + (size_t)q * 3 * R;
-      s0 += cc * P[r];
-      s1 += cc * P[R + r];
-      s2 += cc * P[2 * R + r];
+    const RFX_G float* P = (const RFX_G float*)ps.pol;
+    a.dc = ld4(ps.pcoef, row);
+#pragma unroll
+    for (int t = 0; t < 3; ++t) a.d[t] = P[(size_t)t * R + a.r];
+  }
+}
+
+// One Lorentz pole: new P from P^n (p), P^{n-1} (b) and E^n; adds to dP.
+__device__ __forceinline__ void lorentz_step(RFX_G float* P, size_t R, unsigned r, const float4& c,
+                                             const float* p, const float* b, const float* o,
+                                             float* dp) {
+#pragma unroll
+  for (int t = 0; t < 3; ++t) {
+    const float n = fmaf(c.z, o[t], fmaf(c.x, p[t], c.y * b[t]));
+    dp[t] += n - p[t];
+    P[(3 + t) * R + r] = p[t];
+    P[t * R + r] = n;
+  }
+}
+
+__device__ __forceinline__ void poles_step(const PsiIO& ps, unsigned m, const Poles& a, float o0,
+                                           float o1, float o2, float& e0, float& e1, float& e2) {
+  const size_t R = (size_t)((unsigned)ps.pol_n[0] * (unsigned)ps.pol_n[1] * (unsigned)ps.pol_n[2]);
+  const unsigned r = a.r;
+  const int nd = ps.n_debye, row = (int)m * ps.n_pole;
+  const float o[3] = {o0, o1, o2};
+  float e[3] = {e0, e1, e2};
+  float dp[3] = {0.f, 0.f, 0.f}, ccl = 0.f;
+  if (nd < ps.n_pole) {
+    RFX_G float* P = (RFX_G float*)ps.pol + (size_t)nd * 3 * R;
+    lorentz_step(P, R, r, a.lc, a.l, a.l + 3, o, dp);
+    ccl = a.lc.w;
+#pragma unroll 1
+    for (int q = nd + 1; q < ps.n_pole; ++q) {
+      const float4 c = ld4(ps.pcoef, row + q);
+      P += 6 * R;
+      float v[6];
+#pragma unroll
+      for (int t = 0; t < 6; ++t) v[t] = P[t * R + r];
+      lorentz_step(P, R, r, c, v, v + 3, o, dp);
+      ccl = c.w;
     }
-    e0 += s0;
-    e1 += s1;
-    e2 += s2;
+  }
+  if (nd > 0) {
+    float s[3];
+#pragma unroll
+    for (int t = 0; t < 3; ++t) s[t] = fmaf(a.dc.z, a.d[t], 0.f);   // (rounded: not into e)
+#pragma unroll 1
+    for (int q = 1; q < nd; ++q) {
+      const float cc = ld4(ps.pcoef, row + q).z;
+      const RFX_G float* P = (const RFX_G float*)ps.pol + (size_t)q * 3 * R;
+#pragma unroll
+      for (int t = 0; t < 3; ++t) s[t] = fmaf(cc, P[t * R + r], s[t]);
+    }
+#pragma unroll
+    for (int t = 0; t < 3; ++t) e[t] += s[t];
   }
   if (nd < ps.n_pole) {
-    e0 -= ccl * d0;
-    e1 -= ccl * d1;
-    e2 -= ccl * d2;
+#pragma unroll
+    for (int t = 0; t < 3; ++t) e[t] = fmaf(-ccl, dp[t], e[t]);
   }
-  for (int q = 0; q < nd; ++q) {
-    const float a = pc[4 * q], b = pc[4 * q + 1];
-    float* P = ps.pol + (size_t)q * 3 * R;
-    P[r] = a * P[r] + b * (e0 + o0);
-    P[R + r] = a * P[R + r] + b * (e1 + o1);
-    P[2 * R + r] = a * P[2 * R + r] + b * (e2 + o2);
+  if (nd > 0) {
+    RFX_G float* P = (RFX_G float*)ps.pol;
+#pragma unroll
+    for (int t = 0; t < 3; ++t) P[t * R + r] = fmaf(a.dc.x, a.d[t], a.dc.y * (e[t] + o[t]));
+#pragma unroll 1
+    for (int q = 1; q < nd; ++q) {
+      const float4 c = ld4(ps.pcoef, row + q);
+      P += 3 * R;
+#pragma unroll
+      for (int t = 0; t < 3; ++t) P[t * R + r] = fmaf(c.x, P[t * R + r], c.y * (e[t] + o[t]));
+    }
   }
+  e0 = e[0];
+  e1 = e[1];
+  e2 = e[2];
 }
 
 template <bool GRADED, bool DISP = false, bool SLAB = false>
@@ -639,7 +699,8 @@ __device__ __forceinline__ float3 e_core_co(const KParams& p, const PsiIO& ps, i
                                             float e2, float hx, float hy, float hz, float hy_i,
                                             float hz_i, float hx_j, float hz_j, float hx_k,
                                             float hy_k, const SlabIO* cm = nullptr,
-                                            const SlabAx* sl = nullptr) {
+                                            const SlabAx* sl = nullptr, unsigned m = 0,
+                                            const Poles* pol = nullptr) {
   float ix, iy, iz;
   if (GRADED) {
     ix = gld(p.inv_e[0], i);
@@ -660,7 +721,12 @@ __device__ __forceinline__ float3 e_core_co(const KParams& p, const PsiIO& ps, i
     e1 = ca * e1 + cb * ((hx - hx_k) * iz - (hz - hz_i) * ix);
     e2 = ca * e2 + cb * ((hy - hy_i) * ix - (hx - hx_j) * iy);
   }
-  if (DISP && (fl & RFXH_POLES)) dispersion_cell(p, ps, i, j, k, c, o0, o1, o2, e0, e1, e2);
+  if (DISP && (fl & RFXH_POLES)) {
+    Poles own;
+    if (!pol) poles_load(ps, i, j, k, m, true, own);
+    const Poles& a = pol ? *pol : own;
+    if (a.on) poles_step(ps, m, a, o0, o1, o2, e0, e1, e2);
+  }
   if (SLAB) {
     if (sl[0].in | sl[1].in | sl[2].in) {
       float d0, d1;
@@ -747,11 +813,12 @@ __device__ __forceinline__ float3 e_core(const KParams& p, const PsiIO& ps, int 
                                          unsigned c, unsigned m, float e0, float e1, float e2,
                                          float hx, float hy, float hz, float hy_i, float hz_i,
                                          float hx_j, float hz_j, float hx_k, float hy_k,
-                                         const SlabIO* cm = nullptr, const SlabAx* sl = nullptr) {
+                                         const SlabIO* cm = nullptr, const SlabAx* sl = nullptr,
+                                         const Poles* pol = nullptr) {
   // one 16-byte row carries everything the E update needs
   const float4 ec = gld(p.ecoef, (int)m);
   return e_core_co<GRADED, DISP, SLAB>(p, ps, i, j, k, c, ec, __float_as_uint(ec.w), e0, e1, e2, hx,
-                                       hy, hz, hy_i, hz_i, hx_j, hz_j, hx_k, hy_k, cm, sl);
+                                       hy, hz, hy_i, hz_i, hx_j, hz_j, hx_k, hy_k, cm, sl, m, pol);
 }
 
 // E at one cell reading E^n from Eo, storing E^{n+1} into En.
@@ -2064,6 +2131,8 @@ __device__ __forceinline__ void col_e(const KParams& p, const PsiIO& ps, const S
   float e0[NP], e1[NP], e2[NP];
   unsigned m[NP];
   SlabAx sl[NP][3];
+  static_assert(!DISP || NP == 1, "dispersive plans: one cell a thread");
+  if (DISP) m[0] = ldu16(p.mat, c0);
 #pragma unroll
   for (int q = 0; q < NP; ++q) slabs_load<true>(p, cm, i0 + q, j, k, sl[q]);
   {
@@ -2079,7 +2148,7 @@ __device__ __forceinline__ void col_e(const KParams& p, const PsiIO& ps, const S
   for (int q = 0; q < NP; ++q) {
     const bool in = i0 + q < p.nx;
     const unsigned c = in ? c0 + (unsigned)q * P : c0;
-    m[q] = ldu16(p.mat, c);
+    if (!DISP) m[q] = ldu16(p.mat, c);
     hx[q + 1] = ldf(p.f[3], c);
     hy[q + 1] = ldf(p.f[4], c);
     hz[q + 1] = ldf(p.f[5], c);
@@ -2091,6 +2160,14 @@ __device__ __forceinline__ void col_e(const KParams& p, const PsiIO& ps, const S
     e1[q] = ldf(p.f[1], c);
     e2[q] = ldf(p.f[2], c);
   }
+  // (poles by the material's bit where the ids fit one word: their loads then
+  // wait for the id alone, not for its row)
+  Poles pol;
+  if (DISP)
+    poles_load(ps, i0, j, k, m[0],
+               p.pole_ids ? ((p.pole_ids >> m[0]) & 1u) != 0
+                          : (__float_as_uint(gld(p.ecoef, (int)m[0]).w) & RFXH_POLES) != 0,
+               pol);
 #pragma unroll
   for (int q = 0; q < NP; ++q) {
     if (i0 + q >= p.nx) break;
@@ -2099,7 +2176,7 @@ __device__ __forceinline__ void col_e(const KParams& p, const PsiIO& ps, const S
     const float hxk_ = bk ? hxk[q] : 0.f, hyk_ = bk ? hyk[q] : 0.f;
     const float3 e = e_core<GRADED, DISP, true>(p, ps, i0 + q, j, k, c, m[q], e0[q], e1[q], e2[q],
                                                 hx[q + 1], hy[q + 1], hz[q + 1], hy[q], hz[q], hxj_,
-                                                hzj_, hxk_, hyk_, &cm, sl[q]);
+                                                hzj_, hxk_, hyk_, &cm, sl[q], DISP ? &pol : nullptr);
     stf(p.f[0], c, e.x);
     stf(p.f[1], c, e.y);
     stf(p.f[2], c, e.z);
@@ -2122,7 +2199,7 @@ void k_update_h_col(KParams p, SlabIO cm, const PsiIO* __restrict__ psp) {
 // Occupancy targets: one cell a thread fits 64 VGPRs (8 wavefronts per SIMD)
 // with its slab memory in flight, 2-cell columns 96 (5) without spilling.
 template <bool GRADED, int NP, bool DISP>
-__global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(NP == 1 && !DISP ? 8 : NP == 2 ? 5 : 1)))
+__global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(NP == 1 ? (DISP ? 5 : 8) : NP == 2 ? 5 : 1)))
 void k_update_e_col(KParams p, SlabIO cm, const PsiIO* __restrict__ psp) {
   const PsiIO& ps = *psp;
   int ib, j, k;
@@ -4221,7 +4298,9 @@ void launch_pass_n(const rfxh_plan* pl, hipStream_t s, const KParams& kp, const 
       if (one_mu) hipLaunchKernelGGL((k_update_h_col<GRADED, NP, true>), g, blk, 0, s, kp, cm, psp);
       else hipLaunchKernelGGL((k_update_h_col<GRADED, NP, false>), g, blk, 0, s, kp, cm, psp);
     } else {
-      if (disp) hipLaunchKernelGGL((k_update_e_col<GRADED, NP, true>), g, blk, 0, s, kp, cm, psp);
+      // (dispersive cells are too wide for columns)
+      if (disp)
+        hipLaunchKernelGGL((k_update_e_col<GRADED, 1, true>), pl->grid, blk, 0, s, kp, cm, psp);
       else hipLaunchKernelGGL((k_update_e_col<GRADED, NP, false>), g, blk, 0, s, kp, cm, psp);
     }
   }
@@ -5021,6 +5100,14 @@ int rfxh_plan_create(const rfxh_desc* d, rfxh_plan** out) {
     float* pc;
     if ((rc = dev_copy(pl, d->pole_coef, (size_t)d->n_mat * d->n_pole * 4, &pc))) return bail(rc);
     pl->pcoef = pc;
+    for (int m = 0; m < d->n_mat; ++m) {
+      if (!(d->mat_flags[m] & RFXH_POLES)) continue;
+      if (m > 63) {
+        kp.pole_ids = 0;
+        break;
+      }
+      kp.pole_ids |= 1ull << m;
+    }
     pl->pol = d->d_pol;
     pl->n_pole = d->n_pole;
     pl->n_debye = d->n_debye;
