@@ -140,7 +140,8 @@ struct SlabIO {
   float* psi;
   const float4* prof;
   unsigned foff[6], fs[6];
-  int poff[6];
+  int poff[6], cn[6];
+  float inv[6];   // 1 / face cell size
 };
 
 constexpr int kDftK = 16;   // steps staged per fold of the DFT-plane accumulators
@@ -376,12 +377,23 @@ __device__ __forceinline__ void point_ops(const KParams& p, unsigned cell, float
 // memory only after the curl gave those a second and third wait each, per
 // cell of a column (223x165x141 with 8 layers: 68 -> 61 us a step, of which
 // 52 without CPML; 326x326x146: 283 -> 268, one cell a thread).
+// (Three floats of the profile row: the fourth of a 16-byte load is unused,
+// its register reused at once, and that reuse waited for the load: 290 -> 257
+// us a step at 325x325x145 graded, 166 -> 156 at 209^3 with 7 monitors.)
+struct Row3 {
+  float x, y, z;
+};
 struct SlabAx {
   bool in;
   float s0, s1, inv;
-  float4 pr;
+  Row3 pr;
   unsigned q, fs;   // element of the first term, distance to the second
 };
+
+__device__ __forceinline__ Row3 ld3(const float4* base, int row) {
+  const RFX_G float* q = (const RFX_G float*)base + 4 * row;
+  return Row3{q[0], q[1], q[2]};
+}
 
 template <bool E, int A>
 __device__ __forceinline__ void slab_load(const KParams& p, const SlabIO& cm, int i, int j, int k,
@@ -390,16 +402,16 @@ __device__ __forceinline__ void slab_load(const KParams& p, const SlabIO& cm, in
   const bool lo = pos < p.slo[A];
   s.in = lo | (pos >= p.shi[A]);
   s.s0 = s.s1 = s.inv = 0.f;
-  s.pr = make_float4(0.f, 0.f, 0.f, 0.f);
+  s.pr = Row3{0.f, 0.f, 0.f};
   s.q = s.fs = 0;
   if (s.in) {
-    const int l = lo ? pos : pos - p.shi[A], n = lo ? p.cn[2 * A] : p.cn[2 * A + 1];
+    const int l = lo ? pos : pos - p.shi[A], n = lo ? cm.cn[2 * A] : cm.cn[2 * A + 1];
     const unsigned fs = lo ? cm.fs[2 * A] : cm.fs[2 * A + 1];
     s.fs = fs;
     s.q = (lo ? cm.foff[2 * A] : cm.foff[2 * A + 1]) + (E ? 2u * fs : 0u) +
           (unsigned)psi_idx(2 * A, l, i, j, k, n, p.ny, p.nz);
-    s.pr = gld(cm.prof, (lo ? cm.poff[2 * A] : cm.poff[2 * A + 1]) + l);
-    s.inv = lo ? p.cinv[2 * A] : p.cinv[2 * A + 1];
+    s.pr = ld3(cm.prof, (lo ? cm.poff[2 * A] : cm.poff[2 * A + 1]) + l);
+    s.inv = lo ? cm.inv[2 * A] : cm.inv[2 * A + 1];
     s.s0 = ldf(cm.psi, s.q);
     s.s1 = ldf(cm.psi, s.q + fs);
   }
@@ -413,14 +425,17 @@ __device__ __forceinline__ void slabs_load(const KParams& p, const SlabIO& cm, i
   for (int a = 0; a < 3; ++a) {
     s[a].in = false;
     s[a].s0 = s[a].s1 = s[a].inv = 0.f;
-    s[a].pr = make_float4(0.f, 0.f, 0.f, 0.f);
+    s[a].pr = Row3{0.f, 0.f, 0.f};
     s[a].q = s[a].fs = 0;
   }
   // (a column's cells past the last plane are in no slab)
   if (i < p.nx && in_slab(p, i, j, k)) {
-    slab_load<E, 0>(p, cm, i, j, k, s[0]);
-    slab_load<E, 1>(p, cm, i, j, k, s[1]);
-    slab_load<E, 2>(p, cm, i, j, k, s[2]);
+    // (one copy: read through a table in memory, each choice of a face would
+    // otherwise become a load of its own with its own wait)
+    const SlabIO c = cm;
+    slab_load<E, 0>(p, c, i, j, k, s[0]);
+    slab_load<E, 1>(p, c, i, j, k, s[1]);
+    slab_load<E, 2>(p, c, i, j, k, s[2]);
   }
 }
 
@@ -2220,6 +2235,7 @@ void k_update_e_col(KParams p, SlabIO cm, const PsiIO* __restrict__ psp) {
 struct BatchEntry {
   KParams p;   // p.f = the instance's current field set
   PsiIO ps;
+  SlabIO cm;
 };
 
 __device__ __forceinline__ int batch_instance(const int* __restrict__ start, int n, int L) {
@@ -2232,15 +2248,17 @@ __device__ __forceinline__ int batch_instance(const int* __restrict__ start, int
   return lo;
 }
 
-// One cell per thread (the two-pass kernels' bodies).  Measured on a
-// 48-instance sweep: 46 Gcell-steps/s, against 40 with the 2-cell column
-// bodies and 35 with the column bodies at one cell; the instance
+// One cell per thread (the two-pass kernels' bodies); the instance
 // parameters stay behind a reference into the table (a by-value copy
-// measured as slow as the column bodies).
+// measured slower).
 // ONE_MU: every instance has one mu_r (its ch_all), so the H pass reads no
-// material id.
-template <int PASS, bool ONE_MU, bool DISP>
-__global__ __launch_bounds__(kWG) void k_batch_pass(const BatchEntry* __restrict__ ents,
+// material id.  KIND: 0 any instances (CPML memory loaded face by face), 1
+// all uniform and 2 all graded, with no instance's slabs meeting (the memory
+// loaded first; one body, as two need 20 registers more and spill).  8 instances of
+// 64 to 128 cells a side, 600k cells each: H 40 -> 36 us, E 43 -> 39.
+template <int PASS, bool ONE_MU, bool DISP, int KIND>
+__global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(KIND && !DISP ? 8 : 1)))
+void k_batch_pass(const BatchEntry* __restrict__ ents,
                                                    const int* __restrict__ start, int n_act) {
   const int L = PASS == 0 ? xcd_remap((int)blockIdx.x, (int)gridDim.x)
                           : xcd_remap_rev((int)blockIdx.x, (int)gridDim.x);
@@ -2251,8 +2269,14 @@ __global__ __launch_bounds__(kWG) void k_batch_pass(const BatchEntry* __restrict
   if (PASS == 0 && L == gld(start, q) && threadIdx.x == 0 && threadIdx.y == 0) *p.step += 1;
   if (!cell_at(p, L - gld(start, q), i, j, k)) return;
   if (PASS == 0) {
-    if (p.graded) two_pass_h<true, ONE_MU>(p, ents[q].ps, i, j, k);
-    else two_pass_h<false, ONE_MU>(p, ents[q].ps, i, j, k);
+    if (KIND) {
+      col_h<KIND == 2, 1, ONE_MU>(p, ents[q].ps, ents[q].cm, i, j, k);
+    } else {
+      if (p.graded) two_pass_h<true, ONE_MU>(p, ents[q].ps, i, j, k);
+      else two_pass_h<false, ONE_MU>(p, ents[q].ps, i, j, k);
+    }
+  } else if (KIND) {
+    col_e<KIND == 2, 1, DISP>(p, ents[q].ps, ents[q].cm, i, j, k);
   } else {
     if (p.graded) two_pass_e<true, DISP>(p, ents[q].ps, i, j, k);
     else two_pass_e<false, DISP>(p, ents[q].ps, i, j, k);
@@ -3986,6 +4010,7 @@ struct BatchRecEntry {
 // recording its E^n, curl H^{n+1/2} and CPML-E term at the instance's
 // current step (the update then finds the same inputs in cache).  Plain
 // isotropic plans only (the record path refuses the others).
+template <int KIND>
 __global__ __launch_bounds__(kWG) void k_batch_e_rec(const BatchEntry* __restrict__ ents,
                                                      const BatchRecEntry* __restrict__ recs,
                                                      const int* __restrict__ start, int n_act) {
@@ -3998,11 +4023,15 @@ __global__ __launch_bounds__(kWG) void k_batch_e_rec(const BatchEntry* __restric
   const long long t = region_index(e.r, i, j, k);
   if (t >= 0) {
     float* rec = e.rec + (*p.step - e.rec_step0) * 9 * e.r.n;
-    if (p.graded) record_cell<true>(p, ents[q].ps, e.r, t, rec);
+    if (KIND ? KIND == 2 : p.graded) record_cell<true>(p, ents[q].ps, e.r, t, rec);
     else record_cell<false>(p, ents[q].ps, e.r, t, rec);
   }
-  if (p.graded) two_pass_e<true, false>(p, ents[q].ps, i, j, k);
-  else two_pass_e<false, false>(p, ents[q].ps, i, j, k);
+  if (KIND) {
+    col_e<KIND == 2, 1, false>(p, ents[q].ps, ents[q].cm, i, j, k);
+  } else {
+    if (p.graded) two_pass_e<true, false>(p, ents[q].ps, i, j, k);
+    else two_pass_e<false, false>(p, ents[q].ps, i, j, k);
+  }
 }
 
 // Reverse step r (counted from each instance's hi) of the active instances:
@@ -4272,6 +4301,8 @@ SlabIO slab_io(const rfxh_plan* pl, int set) {
     c.foff[f] = pl->psi_foff[f];
     c.fs[f] = pl->psi_fs[f];
     c.poff[f] = pl->cprof_off[f];
+    c.cn[f] = pl->kp.cn[f];
+    c.inv[f] = pl->kp.cinv[f];
   }
   return c;
 }
@@ -5988,6 +6019,7 @@ int batch_table(const rfxh_batch* b, const std::vector<int>& order, std::vector<
     ents[r].p = pl->kp;
     for (int c = 0; c < 6; ++c) ents[r].p.f[c] = pl->set[pl->cur][c];
     ents[r].ps = psi_io(pl, pl->cur);
+    ents[r].cm = slab_io(pl, pl->cur);
     const long long nb = (long long)start[r] + batch_blocks(pl);
     if (nb > 0x7fffffffLL) return fail(RFXH_EINVAL, "batch too large for one launch");
     start[r + 1] = (int)nb;
@@ -5995,29 +6027,45 @@ int batch_table(const rfxh_batch* b, const std::vector<int>& order, std::vector<
   return RFXH_OK;
 }
 
+// The batched kernels' KIND for these instances.
+int batch_kind(const rfxh_batch* b, const std::vector<int>& order, int n_act) {
+  bool graded = false, uniform = false;
+  for (int q = 0; q < n_act; ++q) {
+    const rfxh_plan* pl = b->plans[order[q]];
+    if (pl->slabs_meet) return 0;
+    (pl->kp.graded ? graded : uniform) = true;
+  }
+  return graded && uniform ? 0 : graded ? 2 : 1;
+}
+
+template <int KIND>
+void batch_pass_k(const rfxh_batch* b, hipStream_t s, const BatchEntry* d_ents, const int* d_start,
+                  const std::vector<int>& order, unsigned nb, int n_act, int pass) {
+  const dim3 g(nb), blk(kBX, kTY);
+  bool one_mu = true, disp = false;
+  for (int q = 0; q < n_act; ++q) {
+    const rfxh_plan* pl = b->plans[order[q]];
+    one_mu = one_mu && pl->kp.ch_all > 0.f;
+    disp = disp || pl->n_pole > 0 || pl->aniso;
+  }
+  if (pass == 0 && one_mu)
+    hipLaunchKernelGGL((k_batch_pass<0, true, false, KIND>), g, blk, 0, s, d_ents, d_start, n_act);
+  else if (pass == 0)
+    hipLaunchKernelGGL((k_batch_pass<0, false, false, KIND>), g, blk, 0, s, d_ents, d_start, n_act);
+  else if (disp)
+    hipLaunchKernelGGL((k_batch_pass<1, false, true, KIND>), g, blk, 0, s, d_ents, d_start, n_act);
+  else
+    hipLaunchKernelGGL((k_batch_pass<1, false, false, KIND>), g, blk, 0, s, d_ents, d_start, n_act);
+}
+
 // One pass (0: H, 1: E) of the first n_act instances of a table whose rows
 // are the plans in `order`; nb = their logical workgroups.
 void batch_pass(const rfxh_batch* b, hipStream_t s, const BatchEntry* d_ents, const int* d_start,
                 const std::vector<int>& order, unsigned nb, int n_act, int pass) {
-  if (pass == 0) {
-    bool one_mu = true;
-    for (int q = 0; q < n_act; ++q) one_mu = one_mu && b->plans[order[q]]->kp.ch_all > 0.f;
-    if (one_mu)
-      hipLaunchKernelGGL((k_batch_pass<0, true, false>), dim3(nb), dim3(kBX, kTY), 0, s, d_ents,
-                         d_start, n_act);
-    else
-      hipLaunchKernelGGL((k_batch_pass<0, false, false>), dim3(nb), dim3(kBX, kTY), 0, s, d_ents,
-                         d_start, n_act);
-  } else {
-    bool disp = false;
-    for (int q = 0; q < n_act; ++q)
-      disp = disp || b->plans[order[q]]->n_pole > 0 || b->plans[order[q]]->aniso;
-    if (disp)
-      hipLaunchKernelGGL((k_batch_pass<1, false, true>), dim3(nb), dim3(kBX, kTY), 0, s, d_ents,
-                         d_start, n_act);
-    else
-      hipLaunchKernelGGL((k_batch_pass<1, false, false>), dim3(nb), dim3(kBX, kTY), 0, s, d_ents,
-                         d_start, n_act);
+  switch (batch_kind(b, order, n_act)) {
+    case 1: batch_pass_k<1>(b, s, d_ents, d_start, order, nb, n_act, pass); break;
+    case 2: batch_pass_k<2>(b, s, d_ents, d_start, order, nb, n_act, pass); break;
+    default: batch_pass_k<0>(b, s, d_ents, d_start, order, nb, n_act, pass); break;
   }
 }
 
@@ -6225,8 +6273,18 @@ int rfxh_batch_run_record(rfxh_batch* b, const int64_t* step0, const int64_t* n_
     while (act > 0 && n_steps[order[act - 1]] <= t) --act;
     const unsigned nb = (unsigned)start[act];
     batch_pass(b, s, b->d_xents, b->d_xstart, order, nb, act, 0);
-    hipLaunchKernelGGL(k_batch_e_rec, dim3(nb), dim3(kBX, kTY), 0, s, b->d_xents, b->d_rents,
-                       b->d_xstart, act);
+    const dim3 g(nb), blk(kBX, kTY);
+    switch (batch_kind(b, order, act)) {
+      case 1:
+        hipLaunchKernelGGL(k_batch_e_rec<1>, g, blk, 0, s, b->d_xents, b->d_rents, b->d_xstart, act);
+        break;
+      case 2:
+        hipLaunchKernelGGL(k_batch_e_rec<2>, g, blk, 0, s, b->d_xents, b->d_rents, b->d_xstart, act);
+        break;
+      default:
+        hipLaunchKernelGGL(k_batch_e_rec<0>, g, blk, 0, s, b->d_xents, b->d_rents, b->d_xstart, act);
+        break;
+    }
     if (accumulate)
       for (int r = 0; r < act; ++r) launch_accumulators(b->plans[order[r]], s, b->plans[order[r]]->cur);
   }

@@ -48,7 +48,8 @@ def test_equals_the_batched_pass(nd, nl, extra):
     torch.cuda.synchronize()
     alone = _outputs(dr)
     dr.close()
-    b = Batch([sim], steps)
+    # (the second instance's slabs meet, so the batch takes the general pass)
+    b = Batch([sim, cases.to_sim(_spec((3, 17, 40), 6))], steps)
     b.run()
     both = _outputs(b.runs[0])
     b.close()
