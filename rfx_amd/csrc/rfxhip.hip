@@ -3595,16 +3595,137 @@ __global__ __launch_bounds__(256) void k_flux_adj(FluxParams q, const double2* G
   }
 }
 
+// One axis of a cell in a reverse pass, where the slabs of an axis do not
+// meet: the other pass's g-bar at the cell (own) and at the neighbour the
+// forward difference took (nb: +1 in the H-bar pass, -1 in the E-bar pass), and
+// this pass's own memory and profile, all loaded before the adjoint fields are
+// waited for (as SlabAx in the forward passes).
+struct AdjAx {
+  bool own, nb, same;     // same: both in one face's slab
+  float g0, g1, n0, n1;   // g-bar at the cell, at the neighbour
+  float s0, s1, inv, ninv;
+  Row3 pr;
+  unsigned q, fs;
+};
+
+template <bool E, int A>
+__device__ __forceinline__ void adj_slab_load(const KParams& p, const SlabIO& cm,
+                                              const float* gbar, int i, int j, int k, AdjAx& s) {
+  const int pos = A == 0 ? i : A == 1 ? j : k, d = E ? -1 : 1;
+  const int N = A == 0 ? p.nx : A == 1 ? p.ny : p.nz;
+  const int np = pos + d;
+  const bool lo = pos < p.slo[A], nlo = np < p.slo[A];
+  s.own = lo | (pos >= p.shi[A]);
+  s.nb = (np >= 0) & (np < N) & (nlo | (np >= p.shi[A]));
+  s.same = s.own & s.nb & (lo == nlo);
+  s.g0 = s.g1 = s.n0 = s.n1 = s.s0 = s.s1 = s.inv = s.ninv = 0.f;
+  s.pr = Row3{0.f, 0.f, 0.f};
+  s.q = s.fs = 0;
+  if (s.own) {
+    const int l = lo ? pos : pos - p.shi[A], n = lo ? cm.cn[2 * A] : cm.cn[2 * A + 1];
+    const unsigned fs = lo ? cm.fs[2 * A] : cm.fs[2 * A + 1];
+    const unsigned q = (lo ? cm.foff[2 * A] : cm.foff[2 * A + 1]) +
+                       (unsigned)psi_idx(2 * A, l, i, j, k, n, p.ny, p.nz);
+    s.fs = fs;
+    s.q = q + (E ? 2u * fs : 0u);
+    s.pr = ld3(cm.prof, (lo ? cm.poff[2 * A] : cm.poff[2 * A + 1]) + l);
+    s.inv = lo ? cm.inv[2 * A] : cm.inv[2 * A + 1];
+    s.s0 = ldf(cm.psi, s.q);
+    s.s1 = ldf(cm.psi, s.q + fs);
+    const unsigned g = q + (E ? 0u : 2u * fs);
+    s.g0 = ldf(gbar, g);
+    s.g1 = ldf(gbar, g + fs);
+  }
+  if (s.nb) {
+    const int l = nlo ? np : np - p.shi[A], n = nlo ? cm.cn[2 * A] : cm.cn[2 * A + 1];
+    const unsigned fs = nlo ? cm.fs[2 * A] : cm.fs[2 * A + 1];
+    const unsigned g = (nlo ? cm.foff[2 * A] : cm.foff[2 * A + 1]) + (E ? 0u : 2u * fs) +
+                       (unsigned)psi_idx(2 * A, l, A == 0 ? np : i, A == 1 ? np : j,
+                                         A == 2 ? np : k, n, p.ny, p.nz);
+    s.ninv = nlo ? cm.inv[2 * A] : cm.inv[2 * A + 1];
+    s.n0 = ldf(gbar, g);
+    s.n1 = ldf(gbar, g + fs);
+  }
+}
+
+template <bool E>
+__device__ __forceinline__ void adj_slabs_load(const KParams& p, const SlabIO& cm,
+                                               const float* gbar, int i, int j, int k,
+                                               AdjAx (&s)[3]) {
+  const SlabIO c = cm;
+  adj_slab_load<E, 0>(p, c, gbar, i, j, k, s[0]);
+  adj_slab_load<E, 1>(p, c, gbar, i, j, k, s[1]);
+  adj_slab_load<E, 2>(p, c, gbar, i, j, k, s[2]);
+}
+
+// Adds one axis's transposed CPML differences to the two components it
+// corrects (u of term 0, v of term 1): the general path's sums, face by face
+// from the low one.
+template <bool E>
+__device__ __forceinline__ void adj_diff(const AdjAx& s, float& u, float& v) {
+  if (s.same) {
+    float d0 = E ? s.n0 - s.g0 : s.g0 - s.n0, d1 = E ? s.n1 - s.g1 : s.g1 - s.n1;
+    d0 *= s.inv;
+    d1 *= s.inv;
+    u += d0;
+    v += d1;
+    return;
+  }
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    const bool own = E ? r == 1 : r == 0;   // the lower of the two comes first
+    if (own ? !s.own : !s.nb) continue;
+    float d0 = own ? s.g0 : s.n0, d1 = own ? s.g1 : s.n1;
+    if (own == E) {
+      d0 = -d0;
+      d1 = -d1;
+    }
+    d0 *= own ? s.inv : s.ninv;
+    d1 *= own ? s.inv : s.ninv;
+    u += d0;
+    v += d1;
+  }
+}
+
+// Memory adjoint of one axis: co the cell's coefficient, h0 and h1 the two
+// components' adjoints, with term 1's sign opposite to sg, term 0's.
+template <bool E>
+__device__ __forceinline__ void adj_mem(const SlabIO& cm, float* gbar, const AdjAx& s, float sg,
+                                        float co, float h0, float h1) {
+  const float bb = s.pr.x, cc = s.pr.y, km1 = s.pr.z;
+  const float t0 = s.s0 + sg * co * h0;
+  const float t1 = s.s1 + -sg * co * h1;
+  stf(gbar, s.q, cc * t0 + sg * co * km1 * h0);
+  stf(gbar, s.q + s.fs, cc * t1 + -sg * co * km1 * h1);
+  stf(cm.psi, s.q, bb * t0);
+  stf(cm.psi, s.q + s.fs, bb * t1);
+}
+
 // The single-instance reverse kernels: the bodies of adj_h_cell and
 // adj_e_cell written out in the kernels (the same arithmetic; through a
 // device function taking the by-value kernel arguments by reference the
 // compiler copies them into registers whole and spills, 4 % slower on a
 // 277 x 277 x 149 grid).  The batched kernels below call the functions.
-template <bool GRADED>
-__global__ __launch_bounds__(kWG) void k_adj_h(KParams p, AdjParams a, long long n) {
+//
+// KIND 0: any plan.  1: no axis's CPML slabs meet, so every CPML operand is
+// loaded first.  2: and every material has one ch, which is then not read.
+// What bounds these passes is memory, as in the forward passes (40 bytes a
+// cell and 38): at 277x277x149 172 -> 138 us (H-bar) and 188 -> 128 (E-bar), the
+// latter also by having the adjoint fields in flight before the coefficient row
+// is waited for.
+template <bool GRADED, int KIND>
+__global__ __launch_bounds__(kWG) void k_adj_h(KParams p, AdjParams a, SlabIO cm, float* gbar,
+                                               long long n) {
   int i, j, k;
   if (!cell_of(p, i, j, k)) return;
   const unsigned c = ((unsigned)i * (unsigned)p.ny + (unsigned)j) * (unsigned)p.nz + (unsigned)k;
+  constexpr bool SLAB = KIND > 0;
+  AdjAx ax[3];
+  float ch_own = p.ch_all;
+  if (SLAB) {
+    adj_slabs_load<false>(p, cm, gbar, i, j, k, ax);
+    if (KIND == 1 && (ax[0].own | ax[1].own | ax[2].own)) ch_own = ldf(a.chv, c);
+  }
   const unsigned P = (unsigned)p.plane;
   const bool hj = j + 1 < p.ny, hk = k + 1 < p.nz, hi = i + 1 < p.nx;
   float ix, iy, iz, ixn, iyn, izn;  // E-update spacings at the cell and at its forward neighbour
@@ -3635,7 +3756,11 @@ __global__ __launch_bounds__(kWG) void k_adj_h(KParams p, AdjParams a, long long
   hy += -vx * iz + vx_k * izn + vz * ix - vz_i * ixn;
   hx += vy * iz - vy_k * izn - vz * iy + vz_j * iyn;
   // transpose of the CPML-E differences g = (H(x) - H(x - e)) / d
-  if (in_slab(p, i, j, k) || in_slab(p, hi ? i + 1 : i, hj ? j + 1 : j, hk ? k + 1 : k)) {
+  if (SLAB) {
+    adj_diff<false>(ax[0], hz, hy);
+    adj_diff<false>(ax[1], hz, hx);
+    adj_diff<false>(ax[2], hy, hx);
+  } else if (in_slab(p, i, j, k) || in_slab(p, hi ? i + 1 : i, hj ? j + 1 : j, hk ? k + 1 : k)) {
 #pragma unroll
     for (int face = 0; face < 6; ++face) {
       if (p.cn[face] == 0) continue;
@@ -3689,7 +3814,11 @@ __global__ __launch_bounds__(kWG) void k_adj_h(KParams p, AdjParams a, long long
     }
   }
   // CPML-H memory adjoint (cpml.py:875-1043 transposed)
-  if (in_slab(p, i, j, k)) {
+  if (SLAB) {
+    if (ax[0].own) adj_mem<false>(cm, gbar, ax[0], 1.f, ch_own, hy, hz);
+    if (ax[1].own) adj_mem<false>(cm, gbar, ax[1], -1.f, ch_own, hx, hz);
+    if (ax[2].own) adj_mem<false>(cm, gbar, ax[2], 1.f, ch_own, hx, hy);
+  } else if (in_slab(p, i, j, k)) {
     const float ch = ldf(a.chv, c);
 #pragma unroll
     for (int face = 0; face < 6; ++face) {
@@ -3750,18 +3879,31 @@ __device__ __forceinline__ long long adj_pol_row(const AdjParams& a, int i, int 
   return ((long long)li * a.pol_n[1] + lj) * a.pol_n[2] + lk;
 }
 
-template <bool GRADED, bool DISP = false>
-__global__ __launch_bounds__(kWG) void k_adj_e(KParams p, AdjParams a, int gather, long long m) {
+template <bool GRADED, bool DISP, int KIND>
+__global__ __launch_bounds__(kWG) void k_adj_e(KParams p, AdjParams a, SlabIO cm, float* gbar,
+                                               int gather, long long m) {
   int i, j, k;
   if (!cell_at(p, xcd_remap_rev((int)blockIdx.x, (int)gridDim.x), i, j, k)) return;
   const unsigned c = ((unsigned)i * (unsigned)p.ny + (unsigned)j) * (unsigned)p.nz + (unsigned)k;
   const unsigned P = (unsigned)p.plane;
   const unsigned mid0 = ldu16(p.mat, c);
-  const float4 co = p.coef[mid0];
+  constexpr bool SLAB = KIND > 0;
+  AdjAx ax[3];
+  if (SLAB) adj_slabs_load<true>(p, cm, gbar, i, j, k, ax);
   float ex = ldf(a.a[0], c), ey = ldf(a.a[1], c), ez = ldf(a.a[2], c);
+  // (the adjoint fields before the coefficient row, whose load waits for the id)
+  const bool hj = j > 0, hk = k > 0, hi = i > 0;
+  const unsigned cj = hj ? c - p.nz : c, ck = hk ? c - 1 : c, ci = hi ? c - P : c;
+  float hb[9] = {};
+  if (gather) {
+    hb[0] = ldf(a.a[3], c), hb[1] = ldf(a.a[4], c), hb[2] = ldf(a.a[5], c);
+    hb[3] = ldf(a.a[3], cj), hb[4] = ldf(a.a[5], cj);
+    hb[5] = ldf(a.a[3], ck), hb[6] = ldf(a.a[4], ck);
+    hb[7] = ldf(a.a[4], ci), hb[8] = ldf(a.a[5], ci);
+  }
+  const float4 co = p.coef[mid0];
   const float bx = ex, by = ey, bz = ez;   // adjoint of E^{m+2} before the E update's transpose
   if (gather) {
-    const bool hj = j > 0, hk = k > 0, hi = i > 0;
     float ix, iy, iz, ixp, iyp, izp;  // H-update spacings at the cell and its backward neighbour
     if (GRADED) {
       ix = p.inv_h[0][i];
@@ -3777,18 +3919,24 @@ __global__ __launch_bounds__(kWG) void k_adj_e(KParams p, AdjParams a, int gathe
       izp = hk ? p.inv_h0 : 0.f;
     }
     const float ch0 = co.w;
-    const float ux = ch0 * ldf(a.a[3], c), uy = ch0 * ldf(a.a[4], c), uz = ch0 * ldf(a.a[5], c);
-    const unsigned cj = hj ? c - p.nz : c, ck = hk ? c - 1 : c, ci = hi ? c - P : c;
-    const float chj = ldf(a.chv, cj), chk = ldf(a.chv, ck), chi = ldf(a.chv, ci);
-    const float ux_j = chj * ldf(a.a[3], cj), uz_j = chj * ldf(a.a[5], cj);
-    const float ux_k = chk * ldf(a.a[3], ck), uy_k = chk * ldf(a.a[4], ck);
-    const float uy_i = chi * ldf(a.a[4], ci), uz_i = chi * ldf(a.a[5], ci);
+    const float ux = ch0 * hb[0], uy = ch0 * hb[1], uz = ch0 * hb[2];
+    const float chj = KIND == 2 ? p.ch_all : ldf(a.chv, cj);
+    const float chk = KIND == 2 ? p.ch_all : ldf(a.chv, ck);
+    const float chi = KIND == 2 ? p.ch_all : ldf(a.chv, ci);
+    const float ux_j = chj * hb[3], uz_j = chj * hb[4];
+    const float ux_k = chk * hb[5], uy_k = chk * hb[6];
+    const float uy_i = chi * hb[7], uz_i = chi * hb[8];
     // transpose of H -= ch curl_fwd E (yee.py:272-289), plus ca E-bar
     ex = co.x * ex + uy * iz - uy_k * izp - uz * iy + uz_j * iyp;
     ey = co.x * ey - ux * iz + ux_k * izp + uz * ix - uz_i * ixp;
     ez = co.x * ez + ux * iy - ux_j * iyp - uy * ix + uy_i * ixp;
     // transpose of the CPML-H differences g = (E(x + e) - E(x)) / d
-    if (in_slab(p, i, j, k) || in_slab(p, hi ? i - 1 : i, hj ? j - 1 : j, hk ? k - 1 : k)) {
+    if (SLAB) {
+      adj_diff<true>(ax[0], ez, ey);
+      adj_diff<true>(ax[1], ez, ex);
+      adj_diff<true>(ax[2], ey, ex);
+    } else if (in_slab(p, i, j, k) ||
+               in_slab(p, hi ? i - 1 : i, hj ? j - 1 : j, hk ? k - 1 : k)) {
 #pragma unroll
       for (int face = 0; face < 6; ++face) {
         if (p.cn[face] == 0) continue;
@@ -3916,7 +4064,11 @@ __global__ __launch_bounds__(kWG) void k_adj_e(KParams p, AdjParams a, int gathe
     if (fl & RFXH_ZERO_EY) ey = 0.f;
     if (fl & RFXH_ZERO_EZ) ez = 0.f;
     // CPML-E memory adjoint (cpml.py:608-777 transposed)
-    if (in_slab(p, i, j, k)) {
+    if (SLAB) {
+      if (ax[0].own) adj_mem<true>(cm, gbar, ax[0], -1.f, co.z, ey, ez);
+      if (ax[1].own) adj_mem<true>(cm, gbar, ax[1], 1.f, co.z, ex, ez);
+      if (ax[2].own) adj_mem<true>(cm, gbar, ax[2], -1.f, co.z, ex, ey);
+    } else if (in_slab(p, i, j, k)) {
       const float ce = co.z;
 #pragma unroll
       for (int face = 0; face < 6; ++face) {
@@ -5937,18 +6089,29 @@ int rfxh_adjoint(rfxh_plan* pl, const rfxh_adjoint_desc* ad, int64_t lo, int64_t
       }
   };
   const bool disp = pl->n_pole > 0;
+  const int kind = pl->slabs_meet ? 0 : pl->kp.ch_all > 0.f ? 2 : 1;
+  SlabIO cm = slab_io(pl, pl->cur);   // (the adjoint memory has the forward one's layout)
+  cm.psi = ad->d_adj_psi;
   auto adj_e = [&](int gather, long long m) {
+    auto go = [&](auto kern) {
+      hipLaunchKernelGGL(kern, pl->grid, pl->block, 0, s, pl->kp, a, cm, ad->d_gbar, gather, m);
+    };
+    auto pick = [&](auto k0, auto k1, auto k2) { go(kind == 0 ? k0 : kind == 1 ? k1 : k2); };
     if (pl->kp.graded) {
-      if (disp)
-        hipLaunchKernelGGL((k_adj_e<true, true>), pl->grid, pl->block, 0, s, pl->kp, a, gather, m);
-      else
-        hipLaunchKernelGGL(k_adj_e<true>, pl->grid, pl->block, 0, s, pl->kp, a, gather, m);
+      if (disp) pick(k_adj_e<true, true, 0>, k_adj_e<true, true, 1>, k_adj_e<true, true, 2>);
+      else pick(k_adj_e<true, false, 0>, k_adj_e<true, false, 1>, k_adj_e<true, false, 2>);
     } else {
-      if (disp)
-        hipLaunchKernelGGL((k_adj_e<false, true>), pl->grid, pl->block, 0, s, pl->kp, a, gather, m);
-      else
-        hipLaunchKernelGGL(k_adj_e<false>, pl->grid, pl->block, 0, s, pl->kp, a, gather, m);
+      if (disp) pick(k_adj_e<false, true, 0>, k_adj_e<false, true, 1>, k_adj_e<false, true, 2>);
+      else pick(k_adj_e<false, false, 0>, k_adj_e<false, false, 1>, k_adj_e<false, false, 2>);
     }
+  };
+  auto adj_h = [&](long long n) {
+    auto go = [&](auto kern) {
+      hipLaunchKernelGGL(kern, pl->grid, pl->block, 0, s, pl->kp, a, cm, ad->d_gbar, n);
+    };
+    auto pick = [&](auto k0, auto k1, auto k2) { go(kind == 0 ? k0 : kind == 1 ? k1 : k2); };
+    if (pl->kp.graded) pick(k_adj_h<true, 0>, k_adj_h<true, 1>, k_adj_h<true, 2>);
+    else pick(k_adj_h<false, 0>, k_adj_h<false, 1>, k_adj_h<false, 2>);
   };
   // prologue of step hi-1 (E-bar holds the adjoint of E^{hi})
   if (e_planes) plane_adj(true, (long long)(hi - 1));
@@ -5960,10 +6123,7 @@ int rfxh_adjoint(rfxh_plan* pl, const rfxh_adjoint_desc* ad, int64_t lo, int64_t
       hipLaunchKernelGGL(k_port_adj_h, dim3((unsigned)((pl->kp.n_ops + 63) / 64)), dim3(64), 0, s,
                          pl->kp, a, (long long)n);
     if (h_planes) plane_adj(false, (long long)n);
-    if (pl->kp.graded)
-      hipLaunchKernelGGL(k_adj_h<true>, pl->grid, pl->block, 0, s, pl->kp, a, (long long)n);
-    else
-      hipLaunchKernelGGL(k_adj_h<false>, pl->grid, pl->block, 0, s, pl->kp, a, (long long)n);
+    adj_h((long long)n);
     if (e_planes && m >= 0) {
       // the gather, then the E-plane adjoints of step m, then its prologue
       adj_e(1, -1);
