@@ -4261,6 +4261,7 @@ struct rfxh_plan {
   int wmarch_seg = 0;           // its x segments (0: automatic)
   bool aniso = false;           // ids with per-component eps (subpixel smoothing)
   bool tb = false;              // two steps per sweep (temporal-blocked march), ping-pong
+  bool tb_auto = false;         // chosen by default: runs keep the field set they began in
   int tb_seg = 0;               // its x segments (0: automatic)
   int tb_ops_max = 0;           // most point operations in one of its tile columns
   ResPlan rp;                   // the resident step's blocks (rp.ok: the plan can take it)
@@ -5073,6 +5074,7 @@ int64_t rfxh_psi_floats(const rfxh_desc* d) {
 }
 
 static PsiIO psi_io(const rfxh_plan* pl, int set);
+static void tb_choose(rfxh_plan* pl, bool free_choice);
 
 int rfxh_plan_create(const rfxh_desc* d, rfxh_plan** out) {
   if (!d || !out) return fail(RFXH_EINVAL, "null descriptor or output");
@@ -5505,6 +5507,7 @@ int rfxh_plan_create(const rfxh_desc* d, rfxh_plan** out) {
   for (auto& e : pl->tev) {
     if (hipEventCreate(&e) != hipSuccess) return bail(fail(RFXH_EHIP, "hipEventCreate"));
   }
+  tb_choose(pl, kname.empty() && !ord);
   *out = pl;
   return RFXH_OK;
 }
@@ -5555,8 +5558,20 @@ int rfxh_kernel_time_ms(rfxh_plan* pl, int which, double* avg_ms, int64_t* count
 
 // rfxh_run with the temporal-blocked march: pairs of steps per sweep (each
 // flips the field set), an odd last step on the two-pass kernels in place.
+// Where the sweep is only the default, an even number of sweeps, so that the
+// state stays in the set it was in, as with the two-pass step.
 static int run_tb(rfxh_plan* pl, hipStream_t s, int64_t n_steps, int use_graph) {
-  const int64_t pairs = n_steps / 2;
+  const int64_t pairs = pl->tb_auto ? n_steps / 4 * 2 : n_steps / 2;
+  auto rest = [&](hipStream_t st, int64_t n) {
+    if (n == 0) return 0;
+    advance(pl, st, -1);
+    for (; n > 0; --n) {
+      const int rc = launch_step(pl, st, nullptr, pl->cur);
+      if (rc) return rc;
+    }
+    advance(pl, st, 1);
+    return 0;
+  };
   if (!use_graph || pl->timing || n_steps < pl->graph_chunk) {
     const int64_t every = std::max<int64_t>(1, pairs / kTimingSamples);
     int n_samples = 0;
@@ -5568,12 +5583,8 @@ static int run_tb(rfxh_plan* pl, hipStream_t s, int64_t n_steps, int use_graph) 
       if (rc) return rc;
       pl->cur ^= 1;
     }
-    if (n_steps & 1) {
-      advance(pl, s, -1);
-      const int rc = launch_step(pl, s, nullptr, pl->cur);
-      if (rc) return rc;
-      advance(pl, s, 1);
-    }
+    const int rc = rest(s, n_steps - 2 * pairs);
+    if (rc) return rc;
     dft_flush(pl, s);
     HIPCHK(hipGetLastError());
     if (n_samples) return collect_timing(pl, n_samples);
@@ -5605,21 +5616,17 @@ static int run_tb(rfxh_plan* pl, hipStream_t s, int64_t n_steps, int use_graph) 
   HIPCHK(hipEventRecord(pl->ev_in, s));
   HIPCHK(hipStreamWaitEvent(pl->cap_stream, pl->ev_in, 0));
   int64_t done = 0;
-  while (n_steps - done >= 2 * sweeps) {
+  while (2 * pairs - done >= 2 * sweeps) {
     HIPCHK(hipGraphLaunch(pl->graph_exec[g], pl->cap_stream));
     done += 2 * sweeps;
   }
-  for (; n_steps - done >= 2; done += 2) {
+  for (; done < 2 * pairs; done += 2) {
     const int rc = launch_tb(pl, pl->cap_stream, nullptr, pl->cur);
     if (rc) return rc;
     pl->cur ^= 1;
   }
-  if (done < n_steps) {
-    advance(pl, pl->cap_stream, -1);
-    const int rc = launch_step(pl, pl->cap_stream, nullptr, pl->cur);
-    if (rc) return rc;
-    advance(pl, pl->cap_stream, 1);
-  }
+  const int rc = rest(pl->cap_stream, n_steps - done);
+  if (rc) return rc;
   dft_flush(pl, pl->cap_stream);
   HIPCHK(hipGetLastError());
   HIPCHK(hipEventRecord(pl->ev_out, pl->cap_stream));
@@ -5642,10 +5649,12 @@ int rfxh_run(rfxh_plan* pl, int64_t step0, int64_t n_steps, void* stream, int us
     if (rc == 0) return run_resident(pl, s, step0, n_steps);
     pl->rp.ok = pl->res = false;
   }
-  if (pl->tb) return run_tb(pl, s, n_steps, use_graph);
+  // (timing samples of a default plan are of single steps, as they were)
+  if (pl->tb && !(pl->tb_auto && pl->timing)) return run_tb(pl, s, n_steps, use_graph);
   const int flip = pl->fused ? 1 : 0;
   if (!pl->fused) advance(pl, s, -1);
-  if (!use_graph || pl->timing || n_steps < pl->graph_chunk) {
+  // (the captured graphs of a plan with the sweep are the sweep's)
+  if (!use_graph || pl->timing || pl->tb || n_steps < pl->graph_chunk) {
     // timing: sample up to kTimingSamples evenly spaced steps; the host does
     // not wait inside the loop, so the queue stays full and each event pair
     // brackets only its kernels
@@ -5749,6 +5758,27 @@ static PsiIO psi_io(const rfxh_plan* pl, int set) {
   return ps;
 }
 
+// The default of very large grids: two steps a sweep move the state once
+// where two-pass steps move it four times (1636 against 2340 us a step at
+// 533^3, 1034 against 1368 at 450x440x430, 643 against 784 at 400x400x301, 481
+// against 536 at 320^3, 659 against 825 at 161x541x541, 922 against 1129 at
+// 1021x257x257).  It loses where rows or planes are short (521 against 257 at
+// 325x325x145), where the z slabs do not fit its edge tiles so that every tile
+// runs their code (1028 against 847 at 363^3 with 16 layers, 979 against 817 at
+// 364^3 with 12, 689 against 795 with 10), and on graded grids (1092 against
+// 829 at 405x405x285, 1560 against 1545 at 457^3).  A plan that the sweep
+// refuses keeps the two-pass step.
+static void tb_choose(rfxh_plan* pl, bool free_choice) {
+  const KParams& kp = pl->kp;
+  const int z = std::max(kp.cn[4], kp.cn[5]);
+  if (!free_choice || pl->res || !pl->set[1][0] || kp.graded ||
+      (long long)kp.nx * kp.plane < 40000000LL || kp.ny < 256 || kp.nz < 256 ||
+      (z > 0 && (std::min(kp.cn[4], kp.cn[5]) == 0 || z + kTBHalo > kTBEdgeC - 2 * kTBHalo)))
+    return;
+  pl->tb_auto = rfxh_set_variant(pl, 8, 0) == RFXH_OK;
+  if (!pl->tb_auto) (void)hipGetLastError();   // (no memory for the sweep's scratch)
+}
+
 int rfxh_set_variant(rfxh_plan* pl, int kernel, int param) {
   if (!pl || kernel < 0 || kernel > 9) return fail(RFXH_EINVAL, "bad variant");
   if (kernel == 9) {
@@ -5760,6 +5790,7 @@ int rfxh_set_variant(rfxh_plan* pl, int kernel, int param) {
     return RFXH_OK;
   }
   if (kernel == 8) {
+    pl->tb_auto = false;
     if (param < 0) return fail(RFXH_EINVAL, "bad segment count");
     if (!pl->set[1][0]) return fail(RFXH_EINVAL, "the temporal-blocked march needs a second field set");
     if (pl->n_pole > 0 || pl->aniso)
