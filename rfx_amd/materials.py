@@ -52,6 +52,25 @@ def lorentz_pole(delta_eps: float, omega_0: float, delta: float) -> LorentzPole:
     return LorentzPole(omega_0=omega_0, delta=delta, kappa=delta_eps * omega_0 ** 2)
 
 
+def _ranks(a):
+    """np.unique with inverse of a 1-D array, by one sort of (value, index)
+    words where the value has 32 bits."""
+    n = a.size
+    if a.dtype != np.uint32 or n >= 1 << 32:
+        v, inv = np.unique(a, return_inverse=True)
+        return v, inv.ravel().astype(np.int64, copy=False)
+    w = a.astype(np.uint64) << np.uint64(32)
+    w |= np.arange(n, dtype=np.uint64)
+    w.sort()
+    s = (w >> np.uint64(32)).astype(np.uint32)
+    first = np.empty(n, bool)
+    first[:1] = True
+    np.not_equal(s[1:], s[:-1], out=first[1:])
+    inv = np.empty(n, np.int64)
+    inv[(w & np.uint64(0xFFFFFFFF)).astype(np.int64)] = np.cumsum(first) - 1
+    return s[first], inv
+
+
 class MaterialMap:
     def __init__(self, shape):
         self.shape = tuple(shape)
@@ -221,22 +240,46 @@ class MaterialMap:
     def override(self, eps_r=None, sigma=None, mu_r=None):
         """Replace per-cell material values wholesale (forward(eps_override=...),
         rfx/api/_execute.py:2800-2805), keeping each cell's flags."""
-        eps, sig, mu, flg = self.props()
-        cur = self.ids
-        E = eps[cur] if eps_r is None else np.asarray(eps_r, F32).reshape(self.shape)
-        S = sig[cur] if sigma is None else np.asarray(sigma, F32).reshape(self.shape)
-        M = mu[cur] if mu_r is None else np.asarray(mu_r, F32).reshape(self.shape)
-        Fl = flg[cur]
-        # distinct (eps, sigma, mu, flags) tuples: one 1-D unique per
-        # property (bit patterns), then one over the combined int64 key
-        parts = [np.unique(a.view(np.uint32).ravel() if a.dtype == F32 else a.ravel(),
-                           return_inverse=True) for a in (E, S, M, Fl)]
-        if max(len(v) for v, _ in parts[:3]) > MAX_IDS or len(parts[3][0]) > 256:
+        table = [a.view(np.uint32) for a in self.props()]     # eps, sigma, mu, flags
+        cur = self.ids.ravel()
+        given = [None if v is None else
+                 np.ascontiguousarray(np.asarray(v, F32).reshape(self.shape)).view(np.uint32).ravel()
+                 for v in (eps_r, sigma, mu_r)]
+        # Distinct (eps, sigma, mu, flags) tuples, ordered by bit patterns.  A
+        # cell's rank in a property comes from its id where the property is
+        # kept (the table is short), from one sort of the cells where it is
+        # given; a unique with inverse of every property and of the combined
+        # key took 80 ms of a 109 ms gradient call at 113x89x62, this 25.
+        vals, ranks, taken = [], [], []
+        used = np.flatnonzero(np.bincount(cur, minlength=len(self.table)))
+        for a, tab in zip(given + [None], table):
+            if a is None:
+                v, inv = np.unique(tab[used], return_inverse=True)
+                r = np.zeros(len(tab), np.int64)
+                r[used] = inv.ravel()
+            else:
+                v, r = _ranks(a)
+            vals.append(v)
+            ranks.append(r)
+            taken.append(a is None)
+        if max(len(v) for v in vals[:3]) > MAX_IDS or len(vals[3]) > 256:
             raise ValueError(f"override produces more than {MAX_IDS} distinct materials")
-        key = np.zeros(E.size, np.int64)       # < 65536^3 * 256 < 2^63
-        for vals, inv in parts:
-            key = key * len(vals) + inv.ravel()
-        ukey, inv = np.unique(key, return_inverse=True)
+        weight = [1] * 4                       # key < 65536^3 * 256 < 2^63
+        for q in (2, 1, 0):
+            weight[q] = weight[q + 1] * len(vals[q + 1])
+        kept = sum(r * w for r, w, k in zip(ranks, weight, taken) if k)   # per id
+        key = kept[cur]
+        for r, w, k in zip(ranks, weight, taken):
+            if not k:
+                key += r * w
+        n_key = weight[0] * len(vals[0])
+        if n_key <= 4 * key.size + 65536:      # few enough to mark instead of sort
+            seen = np.zeros(n_key, bool)
+            seen[key] = True
+            ukey = np.flatnonzero(seen)
+            inv = (np.cumsum(seen) - 1)[key]
+        else:
+            ukey, inv = _ranks(key)
         if len(ukey) > MAX_IDS:
             raise ValueError(
                 f"override produces {len(ukey)} distinct materials (max {MAX_IDS})")
@@ -244,16 +287,13 @@ class MaterialMap:
             raise NotImplementedError("overrides of subpixel-smoothed materials")
         self.table, self._lookup = [], {}
         self.get_id(1.0, 0.0, 1.0, 0)
-        new = np.empty(len(ukey), np.uint16)
-        for q, kv in enumerate(ukey):
-            idx = []
-            for vals, _ in reversed(parts):
-                kv, r = divmod(int(kv), len(vals))
-                idx.append(vals[r])
-            fl, m, s, e = idx
-            new[q] = self.get_id(np.uint32(e).view(F32), np.uint32(s).view(F32),
-                                 np.uint32(m).view(F32), int(fl))
-        self.ids = new[inv.ravel()].reshape(self.shape)
+        col, rest = [], ukey
+        for v in reversed(vals):
+            col.append(v[rest % len(v)])
+            rest = rest // len(v)
+        flags, rows = col[0].tolist(), [c.view(F32) for c in col[:0:-1]]
+        new = np.array([self.get_id(*t) for t in zip(*rows, flags)], np.uint16)
+        self.ids = new[inv].reshape(self.shape)
 
     def cell_arrays(self):
         """Dense float32 eps_r, sigma, mu_r (for small grids and tests)."""
