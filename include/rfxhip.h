@@ -228,6 +228,11 @@ int rfxh_kernel_time_ms(rfxh_plan* plan, int which, double* avg_ms, int64_t* cou
  * first run allocates its workspace (up to 100 MB, kept by the plan).  Such
  * launches run one at a time on a device, in the order of the calls; while
  * another process holds the device for them, runs take the two-pass step.
+ * Without a call to this function a plan that does not fit takes 8 where it
+ * has a second field set, one spacing, 40 million cells, rows and planes of
+ * 256 and z slabs of at most 10 layers on both faces or none (each run an even
+ * number of sweeps, its last steps two-pass, so the state stays in its field
+ * set; timed runs two-pass), else kernel 0 in flat order.
  * Kernels 1-3, 7 and 8 need the second field set.
  * Variants compute the same step; they differ in speed only (9 is 4 and 0
  * bit for bit).  The

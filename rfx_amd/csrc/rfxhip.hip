@@ -9,7 +9,7 @@
 //   injection, probes -> DFT planes.
 //
 // Two kernel designs (no MFMA: ~33 flops per cell-step):
-//   two-pass (default): an H launch and an E launch per step, in place; 12
+//   two-pass (the default of most grids): an H launch and an E launch per step, in place; 12
 //     components read + 6 written per cell-step.
 //   fused (RFXH_KERNEL=fused, needs two field sets): one launch per step.  Fields and CPML memory are
 //     double-buffered (read set A, write set B, swap), so a thread can
@@ -26,8 +26,8 @@
 // slightly slower).
 // Material coefficients come through a uint16 id per cell and a small
 // cache-resident table.  The step index lives in device memory and is
-// advanced by a one-thread kernel at the end of each step, so one captured
-// hipGraph of a chunk of steps is replayed for every chunk.
+// counted by the H pass (by a one-thread kernel after a single-launch step),
+// so one captured hipGraph of a chunk of steps is replayed for every chunk.
 
 #include <hip/hip_runtime.h>
 #include <sys/socket.h>
@@ -3136,7 +3136,7 @@ __device__ __forceinline__ void record_cell(const KParams& p, const PsiIO& ps,
 // The dispersive part of the E update at one cell and step n, from the state
 // before the E pass (E^n, P_d^n, P_l^n, P_l^{n-1}): K = sum_d cc_d P_d^n -
 // cc_L sum_l (P_l^{n+1} - P_l^n), P_l^{n+1} = a P_l^n + b P_l^{n-1} + c E^n
-// (dispersion_cell's terms); zero for a cell without poles.  Every cc is
+// (poles_step's terms); zero for a cell without poles.  Every cc is
 // 1/gamma times a constant, so d K / d(eps_r or sigma) = -(gamma'/gamma) K.
 __device__ void disp_k_cell(const KParams& p, const PsiIO& ps, int i, int j, int k, unsigned c,
                             float* out, long long stride) {
@@ -3972,7 +3972,7 @@ __global__ __launch_bounds__(kWG) void k_adj_e(KParams p, AdjParams a, SlabIO cm
       }
     }
     if (DISP) {
-      // transpose of the ADE (dispersion_cell) at this cell: with e-bar the
+      // transpose of the ADE (poles_step) at this cell: with e-bar the
       // adjoint of the new E before the CPML term, P-bar / Q-bar those of
       // the new polarisation: Debye P' = alpha P + beta (E' + E) and E' +=
       // cc P give E-bar += beta P-bar', P-bar = alpha P-bar' + cc e-bar;
