@@ -596,7 +596,7 @@ __device__ __forceinline__ float3 h_cell(const KParams& p, const float* const Eo
 // past the first of a kind (rare) are read where they are used.  What bounds
 // a dispersive cell is that wait: with every pole read after the curl, in a
 // function call that held 99 registers, the E pass of 181x149x117 cells with
-// a Debye and a Lorentz pole took 57 us; now 29.
+// a Debye and a Lorentz pole took 57 us; now 27.
 struct Poles {
   bool on;
   unsigned r;          // cell of the state box
