@@ -4857,37 +4857,38 @@ void res_choose(rfxh_plan* pl, const std::vector<rfxh_point_op>& ops,
   r.ok = true;
 }
 
-// Allocates the mailboxes and staging rings; 1: the device has no room or
-// another process holds it (the caller takes the other step kernels).
+// Allocates the mailboxes, the tables and the staging rings, one block; 1: the device
+// has no room or another process holds it (the run takes the other step
+// kernels).  The plan sees the workspace (r.box) only when all of it is there.
 int res_setup(rfxh_plan* pl, hipStream_t s) {
   ResPlan& r = pl->rp;
-  const long long n_box = 4LL * r.ntx * r.nty * r.ntz * res_words(r.nx);
+  const size_t n_box = 4 * (size_t)r.ntx * r.nty * r.ntz * res_words(r.nx) * sizeof(u64);
   long long per_step = 0;
   for (const PlaneParams& q : pl->planes) per_step += 4LL * q.n1 * q.n2;
   for (const FluxParams& q : pl->fluxes) per_step += 16LL * q.n1 * q.n2;
   // rings of about 64 MiB in all: a launch's fixed cost (about 10 us) is
   // then a few percent of its steps
-  r.chunk = per_step ? std::min<long long>(4096, std::max<long long>(16, (64LL << 20) / per_step))
-                     : (1LL << 20);
-  const long long rows = std::min<long long>(r.chunk, std::max<long long>(1, pl->max_steps));
-  const long long ring = per_step / 4 * rows;
+  const long long chunk = per_step ? std::min<long long>(4096, std::max<long long>(16, (64LL << 20) / per_step))
+                                   : (1LL << 20);
+  const long long rows = std::min<long long>(chunk, std::max<long long>(1, pl->max_steps));
   const size_t n_snap = pl->planes.size() + pl->fluxes.size();
+  // after the mailboxes: the stop word, the parameters, the snapshots, the rings
+  auto up = [](size_t n) { return (n + 255) / 256 * 256; };
+  const size_t at_kp = 256, at_snap = at_kp + up(sizeof(KParams));
+  const size_t n_head = at_snap + up(n_snap * sizeof(ResSnap));
   int dev = 0;
   HIPCHK(hipGetDevice(&dev));
   if (!res_hold(dev)) return 1;
-  r.dev = dev;
   char* base = nullptr;
-  const size_t bytes = n_box * sizeof(u64) + 256 + ring * sizeof(float);
-  if (hipMalloc(&base, bytes) != hipSuccess) {
+  if (hipMalloc(&base, n_box + n_head + (size_t)(per_step * rows)) != hipSuccess) {
     (void)hipGetLastError();
+    res_release(dev);
     return 1;
   }
-  pl->owned.push_back(base);
-  HIPCHK(hipMemsetAsync(base, 0, n_box * sizeof(u64) + 256, s));
-  r.box = reinterpret_cast<u64*>(base);
-  r.stop = reinterpret_cast<unsigned*>(base + n_box * sizeof(u64));
-  float* at = reinterpret_cast<float*>(base + n_box * sizeof(u64) + 256);
-  std::vector<ResSnap> snaps;
+  std::vector<char> head(n_head, 0);
+  std::memcpy(head.data() + at_kp, &pl->kp, sizeof(KParams));
+  std::vector<float*> rings;
+  float* at = reinterpret_cast<float*>(base + n_box + n_head);
   for (size_t q = 0; q < n_snap; ++q) {
     ResSnap sn;
     std::memset(&sn, 0, sizeof(sn));
@@ -4917,16 +4918,25 @@ int res_setup(rfxh_plan* pl, hipStream_t s) {
       sn.npts = (long long)fp.n1 * fp.n2;
     }
     sn.out = at;
-    r.rings.push_back(at);
+    rings.push_back(at);
     at += sn.npts * sn.ncomp * rows;
-    snaps.push_back(sn);
+    std::memcpy(head.data() + at_snap + q * sizeof(ResSnap), &sn, sizeof(sn));
   }
+  // (from pageable memory the copy returns once `head` has been read)
+  if (hipMemsetAsync(base, 0, n_box, s) != hipSuccess ||
+      hipMemcpyAsync(base + n_box, head.data(), n_head, hipMemcpyHostToDevice, s) != hipSuccess) {
+    (void)hipFree(base);
+    res_release(dev);
+    return fail(RFXH_EHIP, "resident step: workspace upload");
+  }
+  pl->owned.push_back(base);
+  r.dev = dev;
   r.chunk = rows;
-  if (int rc = dev_copy(pl, &pl->kp, 1, &r.kp)) return rc;
-  if (n_snap) {
-    const int rc = dev_copy(pl, snaps.data(), snaps.size(), &r.snaps);
-    if (rc) return rc;
-  }
+  r.rings.swap(rings);
+  r.stop = reinterpret_cast<unsigned*>(base + n_box);
+  r.kp = reinterpret_cast<KParams*>(base + n_box + at_kp);
+  r.snaps = n_snap ? reinterpret_cast<ResSnap*>(base + n_box + at_snap) : nullptr;
+  r.box = reinterpret_cast<u64*>(base);
   return 0;
 }
 

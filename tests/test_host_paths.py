@@ -1,0 +1,141 @@
+"""Host paths of the C ABI library that need a device to fail: run on the CPU
+against a HIP runtime of its own (fake_hip.c), which keeps device memory on
+the host, logs the launches instead of running them, and fails allocations on
+request.  Each case runs in a process of its own that loads nothing else of
+HIP."""
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+LIB = os.path.join(ROOT, "rfx_amd", "librfxhip.so")
+
+PRELUDE = """
+import ctypes as C, importlib.util, os, sys, types
+import numpy as np
+F = C.CDLL(os.environ["FAKE_HIP_SO"], mode=C.RTLD_GLOBAL)
+F.fake_log.restype = C.c_char_p
+F.fake_limit.argtypes = [C.c_longlong]
+F.fake_live.restype = F.fake_peak.restype = C.c_longlong
+F.fake_pinned.restype = C.POINTER(C.c_uint32)
+sys.modules["torch"] = types.ModuleType("torch")     # (_lib imports it to share its runtime)
+spec = importlib.util.spec_from_file_location("_lib", os.path.join(os.environ["ROOT"], "rfx_amd/_lib.py"))
+L = importlib.util.module_from_spec(spec)
+spec.loader.exec_module(L)
+lib = L.load()
+keep = []
+
+def f32(a):
+    a = np.ascontiguousarray(a, np.float32)
+    keep.append(a)
+    return a.ctypes.data_as(C.POINTER(C.c_float))
+
+def buf(n, dt=np.float32):
+    a = np.zeros(n, dt)
+    keep.append(a)
+    return a.ctypes.data
+
+def desc(n, steps=100, two=True, cpml=(0,) * 6, planes=0, mem=None):
+    # mem: cells that exist (grids whose kernels the fake runtime does not run)
+    d = L.Desc()
+    d.nx, d.ny, d.nz = n
+    cells = mem or int(np.prod(n))
+    for a in range(3):
+        d.inv_e[a] = f32(np.full(n[a], 1e3))
+        d.inv_h[a] = f32(np.full(n[a], 1e3))
+    d.dt = 1e-12
+    d.d_mat, d.n_mat = buf(cells, np.uint16), 1
+    d.mat_coef = f32([1.0, 0.5, 0.5, 0.5])
+    fl = np.zeros(1, np.uint32)
+    keep.append(fl)
+    d.mat_flags = fl.ctypes.data_as(C.POINTER(C.c_uint32))
+    for c in range(6):
+        d.d_f[c] = buf(cells)
+        if two:
+            d.d_f2[c] = buf(cells)
+    for f in range(6):
+        d.cpml_n[f] = cpml[f]
+        if cpml[f]:
+            for t in (d.cpml_b, d.cpml_c, d.cpml_km1):
+                t[f] = f32(np.zeros(cpml[f]))
+            d.cpml_inv_d[f] = 1e3
+    if any(cpml):
+        npsi = cells if mem else lib.rfxh_psi_floats(C.byref(d))
+        d.d_psi, d.d_psi2 = buf(npsi), buf(npsi)
+    d.max_steps = steps
+    if planes:
+        fr = np.array([1e9])
+        keep.append(fr)
+        pl = (L.Plane * planes)()
+        for q in range(planes):
+            pl[q].axis, pl[q].index, pl[q].comp, pl[q].n_freq = 0, q, 2, 1
+            pl[q].freqs = fr.ctypes.data_as(C.POINTER(C.c_double))
+            pl[q].d_acc = buf(2 * n[1] * n[2], np.float64)
+        keep.append(pl)
+        d.n_plane, d.planes = planes, pl
+    return d
+
+def create(d):
+    p = C.c_void_p()
+    L.check(lib.rfxh_plan_create(C.byref(d), C.byref(p)))
+    return p
+
+def variant(p):
+    k, q = C.c_int(), C.c_int()
+    L.check(lib.rfxh_get_variant(p, C.byref(k), C.byref(q)))
+    return k.value
+
+def run(p, lo=0, n=20):
+    F.fake_clear()
+    rc = lib.rfxh_run(p, lo, n, None, 1)
+    return rc, [l.split() for l in F.fake_log().decode().splitlines()]
+
+def resident(log):
+    return [l for l in log if "k_resident" in l[0]]
+
+def two_pass(log):
+    return [l for l in log if "k_update_h" in l[0] or l[0] == "graph"]
+"""
+
+
+@pytest.fixture(scope="module")
+def fake(tmp_path_factory):
+    if not os.path.exists(LIB):
+        pytest.skip("librfxhip.so not built")
+    out = str(tmp_path_factory.mktemp("fake") / "fake_hip.so")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-O1", "-o", out, os.path.join(HERE, "fake_hip.c")],
+                   check=True)
+
+    def case(body, **env):
+        e = dict(os.environ, FAKE_HIP_SO=out, ROOT=ROOT, FAKE_HIP_BUS=f"test-{os.getpid()}", **env)
+        r = subprocess.run([sys.executable, "-c", PRELUDE + textwrap.dedent(body)], env=e,
+                           capture_output=True, text=True, timeout=100)
+        assert r.returncode == 0, r.stdout + r.stderr
+    return case
+
+
+def test_resident_workspace_is_whole_or_absent(fake):
+    """Whichever allocation of a resident run's set-up fails, the run takes
+    the two-pass step, no launch ever gets a missing parameter block, and
+    nothing is left over."""
+    fake("""
+    start = F.fake_live()
+    for nth in range(4):
+        p = create(desc((12, 13, 14), planes=3))
+        assert variant(p) == 9
+        F.fake_fail_at(nth)
+        for _ in range(2):
+            rc, log = run(p)
+            assert rc == 0, (nth, lib.rfxh_last_error())
+            assert all(l[4] != "(nil)" for l in resident(log)), (nth, log)
+            assert bool(resident(log)) != bool(two_pass(log)), (nth, log)
+            if nth == 0 and _ == 0:
+                assert two_pass(log)
+        F.fake_fail_at(-1)
+        L.check(lib.rfxh_plan_destroy(p))
+        assert F.fake_live() == start
+    """)
