@@ -192,6 +192,18 @@ int rfxh_plan_destroy(rfxh_plan* plan);
  * from a captured hipGraph. */
 int rfxh_run(rfxh_plan* plan, int64_t step0, int64_t n_steps, void* stream, int use_graph);
 
+/* Whether the plan's runs went through, as far as the host can see: call it
+ * when the run's stream has been synchronised.  Only a resident run
+ * (rfxh_set_variant, kernel 9) can fail on the device: its workgroups wait for one
+ * another, and where the device does not run them all together (it is shared
+ * with a process that the guard below does not see) they give up after a few
+ * seconds.  The run's fields, probe and port rows and accumulators are then NaN,
+ * this call or the plan's next run (whichever comes first) returns RFXH_EHIP
+ * once, and the plan takes the two-pass step until kernel 9 is set again.
+ * RFXH_RESIDENT_DEAF in the environment of rfxh_plan_create makes every such wait
+ * of the plan run out after some milliseconds (to test a caller's handling). */
+int rfxh_status(rfxh_plan* plan);
+
 /* With two field sets: which set (0 = d_f/d_psi, 1 = d_f2/d_psi2) holds the
  * current state; rfxh_set_state_set tells the plan after the caller wrote a
  * state (initial conditions, a restored checkpoint) into a set. */
@@ -228,6 +240,8 @@ int rfxh_kernel_time_ms(rfxh_plan* plan, int which, double* avg_ms, int64_t* cou
  * first run allocates its workspace (up to 100 MB, kept by the plan).  Such
  * launches run one at a time on a device, in the order of the calls; while
  * another process holds the device for them, runs take the two-pass step.
+ * (The guard is an abstract socket name: processes in separate network
+ * namespaces do not see each other's, and rfxh_status reports what comes of it.)
  * Without a call to this function a plan that does not fit takes 8 where it
  * has a second field set, one spacing, 40 million cells, rows and planes of
  * 256 and z slabs of at most 10 layers on both faces or none (each run an even

@@ -112,7 +112,7 @@ class AsmBox(C.Structure):
 _lib = None
 
 EXPORTS = ("rfxh_psi_floats", "rfxh_plan_create", "rfxh_plan_destroy", "rfxh_run",
-           "rfxh_state_set", "rfxh_set_state_set", "rfxh_set_timing", "rfxh_kernel_time_ms",
+           "rfxh_status", "rfxh_state_set", "rfxh_set_state_set", "rfxh_set_timing", "rfxh_kernel_time_ms",
            "rfxh_run_record", "rfxh_run_record_h", "rfxh_run_record_ex", "rfxh_adjoint", "rfxh_batch_create",
            "rfxh_batch_destroy",
            "rfxh_batch_run", "rfxh_batch_run_record", "rfxh_batch_adjoint", "rfxh_set_variant",
@@ -144,6 +144,8 @@ def load():
     lib.rfxh_plan_destroy.restype = C.c_int
     lib.rfxh_run.argtypes = [_P, C.c_int64, C.c_int64, _P, C.c_int]
     lib.rfxh_run.restype = C.c_int
+    lib.rfxh_status.argtypes = [_P]
+    lib.rfxh_status.restype = C.c_int
     lib.rfxh_state_set.argtypes = [_P]
     lib.rfxh_state_set.restype = C.c_int
     lib.rfxh_set_state_set.argtypes = [_P, C.c_int]

@@ -275,7 +275,7 @@ class AdjointRunner:
             with torch.cuda.device(self.dr.device):
                 _lib.check(self.lib.rfxh_adjoint(self.dr.plan, C.byref(d), lo, hi,
                                                  self.dr.stream_ptr()))
-        torch.cuda.synchronize(self.dr.device)
+        self.dr.check()
         if self.dcoef_sigma is not None:
             self.grad_sigma = st.full_gradient(self.box, sigma=True)
         if self.dcoef_mu is not None:

@@ -765,7 +765,7 @@ class Simulation:
             from .autotune import autotune as _tune
             _tune(dr, trial_steps=min(32, int(n_steps)))
         dr.run(0, int(n_steps), use_graph=use_graph)
-        torch.cuda.synchronize(dr.device)
+        dr.check()
         ts = dr.time_series().cpu().numpy().astype(np.float32)
         s_params = None
         if ports:
@@ -853,6 +853,7 @@ class Simulation:
             dr = DeviceRun(prob, n_steps, self._device)
             dr.run(0, n_steps)
             ts = dr.time_series().clone()
+            dr.check()
         s_params = freqs = None
         if ports and port_t is not None:
             # differentiable S11: the same DFT and extraction in torch (complex128)
@@ -862,7 +863,6 @@ class Simulation:
             s_params = s_list[0] if len(s_list) == 1 else torch.stack(s_list)
             freqs = s11
         elif ports:
-            torch.cuda.synchronize(dr.device)
             samp = dr.port_samples().cpu().numpy().astype(np.float64)
             s_list = []
             for q, p in enumerate(ports):

@@ -22,8 +22,10 @@
 //
 // All workgroups must run together: there is at most one per compute unit, and
 // the host lets one resident launch at a time onto a device.  Every wait is
-// bounded all the same, and a workgroup that gives up fills its cells with
-// NaN.
+// bounded all the same.  A workgroup that gives up leaves the loop within 32
+// steps and sets `stop`, which ends the others' waits; what such a run computed is
+// worth nothing, so k_res_check, the last kernel of every run, then makes
+// all of its outputs NaN and tells the host.
 //
 // Measured (one step, two-pass column step -> resident): 87 x 47 x 42 cells
 // 15.5 -> 4.65 us, 41^3 without CPML 14 -> 3.05, 114 x 97 x 80 with a DFT plane
@@ -47,7 +49,8 @@ constexpr int kResWave = 4096;      // source values staged at once (steps x ope
 constexpr int kResWords = 3;        // y/z halo words a thread fetches per exchange
 constexpr int kResEdge = 192;       // most rows plus columns of a block
 constexpr int kResSnaps = 32;       // DFT planes, flux monitors and NTFF faces
-constexpr int kResSpin = 1 << 22;   // polls before a wait gives up (seconds)
+constexpr int kResLook = 1 << 12;   // polls between a wait's looks at whether to give up
+constexpr int kResSpin = 1 << 22;   // polls before it does so by itself (seconds)
 
 typedef unsigned long long u64;
 
@@ -71,6 +74,8 @@ struct ResIO {
   int n_src, n_probe, n_port;
   u64* box;                         // mailboxes [phase][parity][workgroup][words]
   unsigned* stop;                   // set by a workgroup that gave up
+  int spin;                         // polls before a wait gives up
+  unsigned skew;                    // 0 (tests: every other workgroup's tags are off by it)
   const ResSnap* snaps;
   int n_snap;
   int ty, tz, ntx, nty, ntz;        // tile rows, columns; tiles per axis
@@ -97,7 +102,7 @@ struct ResShared {
   float w[kResWave];                // their source values of the next steps [step][operation]
   float gx[2][NX];                  // graded: the planes' inverse spacings (H, E)
   ResSnap snap[kResSnaps];
-  int n_ops, bad;
+  int n_ops, bad, spin;             // bad: a wait gave up
   int wcnt[kResThreads / 64];
 };
 
@@ -219,6 +224,7 @@ __global__ __launch_bounds__(kResThreads) void k_resident(const KParams* __restr
   if (tid == 0) {
     sh.n_ops = 0;
     sh.bad = 0;
+    sh.spin = io.spin;
   }
   __syncthreads();
   int op_lo = 0, op_n = 0;          // this thread's operations
@@ -328,7 +334,7 @@ __global__ __launch_bounds__(kResThreads) void k_resident(const KParams* __restr
     }
   }
   // The state and the memory to or from registers (out = false, true).
-  auto state = [&](bool out, bool bad, const int i0, const int j, const int k) {
+  auto state = [&](bool out, const int i0, const int j, const int k) {
     const KParams& p = *pp;
     const bool live = in_tile && j < p.ny && k < p.nz;
     const unsigned P = (unsigned)p.plane;
@@ -366,7 +372,6 @@ __global__ __launch_bounds__(kResThreads) void k_resident(const KParams* __restr
         gez = gld(p.inv_e[2], k);
       }
     }
-    const float nan = __uint_as_float(0x7fc00000u);
 #pragma unroll
     for (int q = 0; q < NX; ++q) {
       if (!out) {
@@ -389,12 +394,12 @@ __global__ __launch_bounds__(kResThreads) void k_resident(const KParams* __restr
                             (unsigned)k;
       const unsigned x_t = xlo ? io.fs[0] : io.fs[1];
       if (out) {
-        stf(io.f[0], c, bad ? nan : ex[q]);
-        stf(io.f[1], c, bad ? nan : ey[q]);
-        stf(io.f[2], c, bad ? nan : ez[q]);
-        stf(io.f[3], c, bad ? nan : hx[q]);
-        stf(io.f[4], c, bad ? nan : hy[q]);
-        stf(io.f[5], c, bad ? nan : hz[q]);
+        stf(io.f[0], c, ex[q]);
+        stf(io.f[1], c, ey[q]);
+        stf(io.f[2], c, ez[q]);
+        stf(io.f[3], c, hx[q]);
+        stf(io.f[4], c, hy[q]);
+        stf(io.f[5], c, hz[q]);
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
           if (ix) stf(io.psi, x_at + t * x_t, px[t][q]);
@@ -434,7 +439,7 @@ __global__ __launch_bounds__(kResThreads) void k_resident(const KParams* __restr
     }
   };
   // (after the set-up above, whose temporaries would not fit beside it)
-  state(false, false, i0, j, k);
+  state(false, i0, j, k);
 #pragma unroll
   for (int q = 0; q < NX; ++q)
     if (in_tile) {
@@ -475,8 +480,11 @@ __global__ __launch_bounds__(kResThreads) void k_resident(const KParams* __restr
       for (int m = 0; m < kResWords; ++m)
         off |= ((unsigned)(v[m] >> 32) ^ tag) & (unsigned)~(dst[m] >> 31);
       if (off == 0u) break;
-      if (++n >= kResSpin || ((n & 4095) == 0 &&
-                              __hip_atomic_load(io.stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
+      // (the limit from LDS and only at a look: a kernel argument in this loop
+      // cost 2 % of a 28^3 step, a store to `stop` 1.6 %)
+      if (++n % kResLook == 0 &&
+          (sh.bad || n >= sh.spin ||
+           __hip_atomic_load(io.stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
         sh.bad = 1;
         break;
       }
@@ -512,7 +520,7 @@ __global__ __launch_bounds__(kResThreads) void k_resident(const KParams* __restr
   __syncthreads();
 
   bool bad = false;
-  unsigned tag = io.tag0;
+  unsigned tag = io.tag0 + ((wg & 1) ? io.skew : 0u);
   int w_base = 0, w_next = 0;           // first step of the staged source values, of the next ones
   for (int n = 0; n < n_steps; ++n) {
     const int par = n & 1;
@@ -798,7 +806,10 @@ __global__ __launch_bounds__(kResThreads) void k_resident(const KParams* __restr
     fetch(box_e, tag_e, lds_e, src_e, &sh.e[0][0][0], need_e, xs_e, xey, xez);
     lds_barrier();
     if ((n & 31) == 31) {
+      // (the second barrier: no wavefront is at its next wait, which may set
+      // `bad`, before all have read it, so all leave at the same step)
       bad = sh.bad;
+      lds_barrier();
       if (bad) break;
     }
   }
@@ -808,7 +819,7 @@ __global__ __launch_bounds__(kResThreads) void k_resident(const KParams* __restr
   // (opaque positions: the addresses of the way in would stay in registers)
   int oi = i0, oj = j, ok = k;
   __asm__ volatile("" : "+v"(oj), "+v"(ok), "+s"(oi) : : "memory");
-  state(true, bad, oi, oj, ok);
+  state(true, oi, oj, ok);
 }
 
 // Adds the staged steps [0, cnt) of a launch that started at step n0 to the
@@ -840,4 +851,34 @@ __global__ __launch_bounds__(256) void k_res_fold(const float* ring, int ncomp, 
 #pragma unroll
   for (int u = 0; u < kFoldF; ++u)
     if (f0 + u < nf) a[(long long)(f0 + u) * npts] = cur[u];
+}
+
+// After a run whose launches gave up somewhere: its fields, probe and port rows
+// and the accumulators become NaN, and the host's word is set.
+struct ResOut {
+  const unsigned* stop;
+  unsigned* status;                 // pinned host memory
+  float* f[6];
+  long long cells;
+  float *probe, *port;              // first row of the run
+  long long n_probe, n_port;        // floats of its rows
+  const MonEntry* mon;
+  int n_mon;
+};
+
+__global__ __launch_bounds__(256) void k_res_check(ResOut o) {
+  if (__hip_atomic_load(o.stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u) return;
+  const long long t0 = (long long)blockIdx.x * 256 + threadIdx.x, T = (long long)gridDim.x * 256;
+  const float nan = __uint_as_float(0x7fc00000u);
+  for (long long t = t0; t < o.cells; t += T)
+    for (int c = 0; c < 6; ++c) o.f[c][t] = nan;
+  for (long long t = t0; t < o.n_probe; t += T) o.probe[t] = nan;
+  for (long long t = t0; t < o.n_port; t += T) o.port[t] = nan;
+  for (int e = 0; e < o.n_mon; ++e) {
+    const MonEntry& m = o.mon[e];
+    const long long n = m.flux ? 4LL * m.f.nf * m.f.n1 * m.f.n2 : (long long)m.p.nf * m.p.n1 * m.p.n2;
+    double2* const acc = m.flux ? m.f.acc : m.p.acc;
+    for (long long t = t0; t < n; t += T) acc[t] = make_double2((double)nan, (double)nan);
+  }
+  if (t0 == 0) __hip_atomic_store(o.status, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }

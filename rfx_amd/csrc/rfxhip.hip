@@ -4236,6 +4236,9 @@ struct ResPlan {
   int dev = -1;                   // the device its workspace is on (-1: none yet)
   u64* box = nullptr;
   unsigned* stop = nullptr;
+  bool deaf = false;              // (tests: no workgroup hears another, every wait runs out)
+  unsigned* status = nullptr;     // pinned: set when a run gave up (k_res_check)
+  bool clear = false;             // `stop` is still set from a run that gave up
   ResSnap* snaps = nullptr;
   KParams* kp = nullptr;          // device copy of the plan's parameters
   std::vector<float*> rings;      // staging ring of each DFT plane, then of each flux entry
@@ -4783,6 +4786,40 @@ bool res_hold(int dev) {
   return true;
 }
 
+// Words of pinned host memory in which k_res_check leaves a run's failure: one
+// block for the process (an allocation and a free for every plan took 100 us of
+// a 5 ms call), a word for each plan with a workspace.
+struct ResWords {
+  std::mutex mu;
+  unsigned* base = nullptr;
+  std::vector<unsigned*> spare;
+};
+constexpr int kResWordsN = 1024;
+ResWords g_res_words;
+
+unsigned* res_word() {
+  std::lock_guard<std::mutex> lock(g_res_words.mu);
+  if (!g_res_words.base) {
+    if (hipHostMalloc(&g_res_words.base, kResWordsN * sizeof(unsigned), hipHostMallocPortable) !=
+        hipSuccess) {
+      (void)hipGetLastError();
+      g_res_words.base = nullptr;
+      return nullptr;
+    }
+    for (int w = kResWordsN; w-- > 0;) g_res_words.spare.push_back(g_res_words.base + w);
+  }
+  if (g_res_words.spare.empty()) return nullptr;
+  unsigned* const w = g_res_words.spare.back();
+  g_res_words.spare.pop_back();
+  *w = 0;
+  return w;
+}
+
+void res_word_back(unsigned* w) {
+  std::lock_guard<std::mutex> lock(g_res_words.mu);
+  g_res_words.spare.push_back(w);
+}
+
 void res_release(int dev) {
   ResDevice& d = g_res_dev[dev];
   std::lock_guard<std::mutex> lock(d.mu);
@@ -4880,7 +4917,8 @@ int res_setup(rfxh_plan* pl, hipStream_t s) {
   HIPCHK(hipGetDevice(&dev));
   if (!res_hold(dev)) return 1;
   char* base = nullptr;
-  if (hipMalloc(&base, n_box + n_head + (size_t)(per_step * rows)) != hipSuccess) {
+  if (!r.status) r.status = res_word();
+  if (!r.status || hipMalloc(&base, n_box + n_head + (size_t)(per_step * rows)) != hipSuccess) {
     (void)hipGetLastError();
     res_release(dev);
     return 1;
@@ -4961,6 +4999,8 @@ int run_resident(rfxh_plan* pl, hipStream_t s, int64_t step0, int64_t n_steps) {
   io.n_port = kp.n_port;
   io.box = r.box;
   io.stop = r.stop;
+  io.spin = r.deaf ? kResLook : kResSpin;
+  io.skew = r.deaf ? 1u << 31 : 0u;
   io.snaps = r.snaps;
   io.n_snap = (int)r.rings.size();
   io.ty = r.ty;
@@ -4969,6 +5009,8 @@ int run_resident(rfxh_plan* pl, hipStream_t s, int64_t step0, int64_t n_steps) {
   io.nty = r.nty;
   io.ntz = r.ntz;
   const dim3 grid((unsigned)(r.ntx * r.nty * r.ntz)), blk((unsigned)r.threads);
+  if (r.clear) HIPCHK(hipMemsetAsync(r.stop, 0, sizeof(unsigned), s));
+  r.clear = false;
   for (int64_t done = 0; done < n_steps;) {
     const int cnt = (int)std::min<int64_t>(r.chunk, n_steps - done);
     io.n_steps = cnt;
@@ -5008,8 +5050,33 @@ int run_resident(rfxh_plan* pl, hipStream_t s, int64_t step0, int64_t n_steps) {
     }
     done += cnt;
   }
+  ResOut out;
+  std::memset(&out, 0, sizeof(out));
+  out.stop = r.stop;
+  out.status = r.status;
+  for (int c = 0; c < 6; ++c) out.f[c] = io.f[c];
+  out.cells = (long long)kp.nx * kp.plane;
+  out.probe = kp.probe_out ? kp.probe_out + step0 * kp.n_probe : nullptr;
+  out.port = kp.port_out ? kp.port_out + 2 * step0 * kp.n_port : nullptr;
+  out.n_probe = out.probe ? n_steps * kp.n_probe : 0;
+  out.n_port = out.port ? 2 * n_steps * kp.n_port : 0;
+  out.mon = pl->mon;
+  out.n_mon = (int)r.rings.size();
+  hipLaunchKernelGGL(k_res_check, dim3(256), dim3(256), 0, s, out);
   HIPCHK(hipGetLastError());
   return 0;
+}
+
+// Error of a resident run that gave up, once the host can see it; the plan
+// then takes the two-pass step, which waits for nobody.
+int res_status(rfxh_plan* pl) {
+  ResPlan& r = pl->rp;
+  if (!r.status || __atomic_load_n(r.status, __ATOMIC_ACQUIRE) == 0u) return 0;
+  __atomic_store_n(r.status, 0u, __ATOMIC_RELAXED);
+  r.clear = true;
+  pl->res = false;
+  return fail(RFXH_EHIP, "a resident run gave up waiting for its workgroups (the device does not "
+                         "run them all together); its outputs are NaN");
 }
 
 // Whether a run of n_steps takes the resident step: not while its stream is
@@ -5513,6 +5580,7 @@ int rfxh_plan_create(const rfxh_desc* d, rfxh_plan** out) {
   res_choose(pl, ops, km1);
   // the default of every grid that fits: 3-6 times the two-pass step's speed
   pl->res = pl->rp.ok && kname.empty();
+  pl->rp.deaf = std::getenv("RFXH_RESIDENT_DEAF") != nullptr;
   pl->tev.resize(4 * kTimingSamples);
   for (auto& e : pl->tev) {
     if (hipEventCreate(&e) != hipSuccess) return bail(fail(RFXH_EHIP, "hipEventCreate"));
@@ -5532,9 +5600,15 @@ int rfxh_plan_destroy(rfxh_plan* pl) {
   for (auto e : pl->tev)
     if (e) (void)hipEventDestroy(e);
   for (void* p : pl->owned) (void)hipFree(p);
+  if (pl->rp.status) res_word_back(pl->rp.status);
   if (pl->rp.dev >= 0) res_release(pl->rp.dev);
   delete pl;
   return RFXH_OK;
+}
+
+int rfxh_status(rfxh_plan* pl) {
+  if (!pl) return fail(RFXH_EINVAL, "null plan");
+  return res_status(pl);
 }
 
 int rfxh_state_set(rfxh_plan* pl) {
@@ -5648,6 +5722,7 @@ int rfxh_run(rfxh_plan* pl, int64_t step0, int64_t n_steps, void* stream, int us
   if (!pl) return fail(RFXH_EINVAL, "null plan");
   if (step0 < 0 || n_steps < 0 || step0 + n_steps > pl->max_steps)
     return fail(RFXH_EINVAL, "steps outside the source/probe tables (max_steps)");
+  if (int rc = res_status(pl)) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
   hipLaunchKernelGGL(k_set_step, dim3(1), dim3(64), 0, s, pl->kp.step, (long long)step0);
   dft_begin(pl, s, step0);
@@ -5919,6 +5994,7 @@ int rfxh_run_record_ex(rfxh_plan* pl, int64_t step0, int64_t n_steps, const rfxh
   int rc = check_region(pl, region);
   if (rc) return rc;
   if (!d_rec) return fail(RFXH_EINVAL, "record buffer missing");
+  if ((rc = res_status(pl))) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const RegionParams rp = region_params(region);
   hipLaunchKernelGGL(k_set_step, dim3(1), dim3(64), 0, s, pl->kp.step, (long long)step0 - 1);
@@ -6332,9 +6408,10 @@ int rfxh_batch_run(rfxh_batch* b, const int64_t* step0, const int64_t* n_steps, 
   if (!b || !step0 || !n_steps) return fail(RFXH_EINVAL, "bad batch arguments");
   const int n = (int)b->plans.size();
   for (int q = 0; q < n; ++q) {
-    const rfxh_plan* pl = b->plans[q];
+    rfxh_plan* pl = b->plans[q];
     if (step0[q] < 0 || n_steps[q] < 0 || step0[q] + n_steps[q] > pl->max_steps)
       return fail(RFXH_EINVAL, "batch instance steps outside its tables (max_steps)");
+    if (int rc = res_status(pl)) return rc;
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
   // run order: most steps first, so the active instances are always a prefix
@@ -6438,7 +6515,8 @@ int rfxh_batch_run_record(rfxh_batch* b, const int64_t* step0, const int64_t* n_
     if (pl->n_pole > 0 || pl->aniso)
       return fail(RFXH_EINVAL, "dispersive or subpixel-smoothed materials: the reverse mode "
                                "covers plain isotropic plans only");
-    const int rc = check_region(pl, &regions[q]);
+    int rc = check_region(pl, &regions[q]);
+    if (rc == 0) rc = res_status(pl);
     if (rc) return rc;
     if (!d_rec[q]) return fail(RFXH_EINVAL, "record buffer missing");
     order.push_back(q);

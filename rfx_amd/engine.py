@@ -266,6 +266,11 @@ class DeviceRun:
             _lib.check(self.lib.rfxh_run(self.plan, int(step0), n, self.stream_ptr(),
                                          1 if use_graph else 0))
 
+    def check(self):
+        """Wait for the runs and raise if one of them failed on the device."""
+        torch.cuda.synchronize(self.device)
+        _lib.check(self.lib.rfxh_status(self.plan))
+
     def state_set(self) -> int:
         return int(self.lib.rfxh_state_set(self.plan))
 

@@ -139,3 +139,35 @@ def test_resident_workspace_is_whole_or_absent(fake):
         L.check(lib.rfxh_plan_destroy(p))
         assert F.fake_live() == start
     """)
+
+
+def test_a_resident_run_that_gave_up_is_reported(fake):
+    """Every resident run ends with the kernel that looks at its stop word, and
+    the word that kernel leaves for the host becomes an error of whichever
+    call comes first; after it the plan takes the two-pass step until it is
+    told otherwise."""
+    fake("""
+    for first in ("status", "run", "record", "batch"):
+        p = create(desc((12, 13, 14), planes=2))
+        b = C.c_void_p()
+        L.check(lib.rfxh_batch_create(C.byref(p), 1, C.byref(b)))
+        rc, log = run(p)
+        assert rc == 0 and resident(log) and "k_res_check" in log[-1][0], log
+        assert lib.rfxh_status(p) == 0
+        F.fake_pinned()[0] = 1                       # as k_res_check does
+        region = L.Region(0, 0, 0, 2, 2, 2)
+        rec = buf(9 * 8 * 20)
+        one, n = (C.c_int64 * 1)(0), (C.c_int64 * 1)(20)
+        rc = {"status": lambda: lib.rfxh_status(p), "run": lambda: run(p)[0],
+              "record": lambda: lib.rfxh_run_record(p, 0, 20, C.byref(region), rec, None),
+              "batch": lambda: lib.rfxh_batch_run(b, one, n, None, 0)}[first]()
+        assert rc < 0 and b"gave up" in lib.rfxh_last_error(), (first, rc)
+        assert lib.rfxh_status(p) == 0 and variant(p) != 9
+        rc, log = run(p)
+        assert rc == 0 and two_pass(log) and not resident(log), log
+        L.check(lib.rfxh_set_variant(p, 9, 0))
+        rc, log = run(p)
+        assert rc == 0 and resident(log), log
+        L.check(lib.rfxh_batch_destroy(b))
+        L.check(lib.rfxh_plan_destroy(p))
+    """)
