@@ -236,7 +236,8 @@ int rfxh_kernel_time_ms(rfxh_plan* plan, int which, double* avg_ms, int64_t* cou
  * eps, at most 32 planes, monitors
  * and NTFF faces in all and 256 point operations a block).  It is the
  * default of every plan that fits; runs of fewer than 4 steps, timed runs
- * and runs on a stream under capture take the two-pass step instead.  Its
+ * and runs on a stream under capture, or with a mask of fewer compute units than
+ * there are blocks, take the two-pass step instead.  Its
  * first run allocates its workspace (up to 100 MB, kept by the plan).  Such
  * launches run one at a time on a device, in the order of the calls; while
  * another process holds the device for them, runs take the two-pass step.

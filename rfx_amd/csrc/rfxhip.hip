@@ -4755,6 +4755,7 @@ struct ResDevice {
   int sock = -1;
 };
 constexpr int kResDevices = 64;
+constexpr int kResCUs = 512;   // most compute units of a device's mask
 ResDevice g_res_dev[kResDevices];
 
 bool res_hold(int dev) {
@@ -5079,11 +5080,26 @@ int res_status(rfxh_plan* pl) {
                          "run them all together); its outputs are NaN");
 }
 
+// Compute units that kernels on a stream may use (a stream or a process can
+// have a mask; HSA_CU_MASK acts below what the runtime reports).
+int stream_cus(hipStream_t s) {
+  const char* below = std::getenv("HSA_CU_MASK");
+  uint32_t mask[kResCUs / 32] = {};
+  if ((below && *below) || hipExtStreamGetCUMask(s, kResCUs / 32, mask) != hipSuccess) {
+    (void)hipGetLastError();
+    return 0;
+  }
+  int n = 0;
+  for (uint32_t w : mask) n += __builtin_popcount(w);
+  return n;
+}
+
 // Whether a run of n_steps takes the resident step: not while its stream is
 // being captured (the launch's order with other streams and a first
 // run's allocation do not belong in a graph) or single steps are being timed, and not for a handful
 // of steps, which the launch's fixed cost (the state's way in and out)
-// outweighs.
+// outweighs.  Nor on a stream with fewer compute units than the grid has
+// blocks: LDS holds one block a unit, so the last ones would never start.
 bool res_takes(rfxh_plan* pl, hipStream_t s, int64_t n_steps) {
   if (!pl->res || !pl->rp.ok || pl->timing || n_steps < 4) return false;
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
@@ -5091,7 +5107,8 @@ bool res_takes(rfxh_plan* pl, hipStream_t s, int64_t n_steps) {
     (void)hipGetLastError();
     return false;
   }
-  return st == hipStreamCaptureStatusNone;
+  return st == hipStreamCaptureStatusNone &&
+         stream_cus(s) >= pl->rp.ntx * pl->rp.nty * pl->rp.ntz;
 }
 
 // Launch grid of the plan's workgroup order.

@@ -171,3 +171,25 @@ def test_a_resident_run_that_gave_up_is_reported(fake):
         L.check(lib.rfxh_batch_destroy(b))
         L.check(lib.rfxh_plan_destroy(p))
     """)
+
+
+def test_resident_step_needs_a_unit_for_every_block(fake):
+    """On a stream (or in a process) whose compute-unit mask has fewer units
+    than the grid has blocks a run takes the two-pass step; on the next
+    stream without one it is resident again."""
+    body = """
+    p = create(desc((40, 41, 42)))
+    rc, log = run(p)
+    assert rc == 0
+    if os.environ.get("HSA_CU_MASK"):
+        assert two_pass(log) and not resident(log)
+        sys.exit(0)
+    blocks = int(resident(log)[0][1])
+    for units, res in ((blocks - 1, False), (blocks, True), (8, False), (-1, True)):
+        F.fake_mask(units)
+        rc, log = run(p)
+        assert rc == 0 and bool(resident(log)) == res and bool(two_pass(log)) != res, (units, log)
+        assert variant(p) == 9
+    """
+    fake(body)
+    fake(body, HSA_CU_MASK="0:0-15")
