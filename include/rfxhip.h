@@ -240,7 +240,8 @@ int rfxh_kernel_time_ms(rfxh_plan* plan, int which, double* avg_ms, int64_t* cou
  * there are blocks, take the two-pass step instead.  Its
  * first run allocates its workspace (up to 100 MB, kept by the plan).  Such
  * launches run one at a time on a device, in the order of the calls; while
- * another process holds the device for them, runs take the two-pass step.
+ * another process holds the device for them, runs take the two-pass step
+ * (which rfxh_get_variant then names; each run tries again).
  * (The guard is an abstract socket name: processes in separate network
  * namespaces do not see each other's, and rfxh_status reports what comes of it.)
  * Without a call to this function a plan that does not fit takes 8 where it

@@ -4269,6 +4269,7 @@ struct rfxh_plan {
   int tb_ops_max = 0;           // most point operations in one of its tile columns
   ResPlan rp;                   // the resident step's blocks (rp.ok: the plan can take it)
   bool res = false;             // runs take the resident step where they can
+  bool res_out = false;         // the latest one could not have its workspace
   float* psi_base = nullptr;    // CPML memory of set 0 (set 1 at + psi_set)
   float* psi_mid = nullptr;     // the sweep's memory after its first step (owned, same layout)
   long long psi_floats = 0;
@@ -5748,8 +5749,11 @@ int rfxh_run(rfxh_plan* pl, int64_t step0, int64_t n_steps, void* stream, int us
   if (res_takes(pl, s, n_steps)) {
     const int rc = pl->rp.box ? 0 : res_setup(pl, s);
     if (rc < 0) return rc;
-    if (rc == 0) return run_resident(pl, s, step0, n_steps);
-    pl->rp.ok = pl->res = false;
+    if (rc == 0) {
+      pl->res_out = false;
+      return run_resident(pl, s, step0, n_steps);
+    }
+    pl->res_out = true;   // (this run alone: the holder may be gone at the next)
   }
   // (timing samples of a default plan are of single steps, as they were)
   if (pl->tb && !(pl->tb_auto && pl->timing)) return run_tb(pl, s, n_steps, use_graph);
@@ -5889,6 +5893,7 @@ int rfxh_set_variant(rfxh_plan* pl, int kernel, int param) {
       return fail(RFXH_EINVAL, "the resident step covers grids of one block per compute unit, "
                                "without poles, per-component eps or several mu_r");
     pl->res = true;
+    pl->res_out = false;
     return RFXH_OK;
   }
   if (kernel == 8) {
@@ -5976,13 +5981,14 @@ int rfxh_set_variant(rfxh_plan* pl, int kernel, int param) {
 
 int rfxh_get_variant(rfxh_plan* pl, int* kernel, int* param) {
   if (!pl || !kernel || !param) return fail(RFXH_EINVAL, "bad arguments");
-  *kernel = pl->res ? 9
+  const bool res = pl->res && !pl->res_out;
+  *kernel = res ? 9
           : pl->tb ? 8
           : pl->wmarch ? 7
           : pl->march ? 2 + pl->march_tile
           : pl->fused ? 1
           : pl->ncol == 2 ? 4 : pl->ncol == 4 ? 5 : pl->ncol == 3 ? 6 : 0;
-  *param = pl->res ? 0
+  *param = res ? 0
          : pl->tb ? pl->tb_seg
          : pl->wmarch ? pl->wmarch_seg : pl->march ? pl->march_seg : pl->kp.order;
   return RFXH_OK;

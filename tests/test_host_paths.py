@@ -193,3 +193,26 @@ def test_resident_step_needs_a_unit_for_every_block(fake):
     """
     fake(body)
     fake(body, HSA_CU_MASK="0:0-15")
+
+
+def test_a_momentary_holder_costs_the_resident_step_for_its_time_only(fake):
+    """Runs take the two-pass step while somebody else holds the device (or its
+    memory), say so, and the resident step again when it is free."""
+    fake("""
+    import socket
+    p = create(desc((12, 13, 14)))
+    for _ in range(2):
+        with socket.socket(socket.AF_UNIX, socket.SOCK_DGRAM) as s:
+            s.bind("\\0rfxhip-resident-" + os.environ["FAKE_HIP_BUS"])
+            rc, log = run(p)
+            assert rc == 0 and two_pass(log) and not resident(log) and variant(p) != 9, log
+        if _ == 0:
+            L.check(lib.rfxh_set_variant(p, 9, 0))     # accepted, and what the plan is set to
+            assert variant(p) == 9
+    F.fake_limit(1)
+    rc, log = run(p)
+    assert rc == 0 and two_pass(log) and variant(p) != 9
+    F.fake_limit(-1)
+    rc, log = run(p)
+    assert rc == 0 and resident(log) and variant(p) == 9, log
+    """)
