@@ -4896,6 +4896,15 @@ void res_choose(rfxh_plan* pl, const std::vector<rfxh_point_op>& ops,
   r.ok = true;
 }
 
+// For the lifetime of one, this thread's allocations and copies leave alone a
+// stream capture that is under way elsewhere: in the default mode they would
+// end a global one (torch's is).
+struct RelaxedCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
 // Allocates the mailboxes, the tables and the staging rings, one block; 1: the device
 // has no room or another process holds it (the run takes the other step
 // kernels).  The plan sees the workspace (r.box) only when all of it is there.
@@ -4915,6 +4924,7 @@ int res_setup(rfxh_plan* pl, hipStream_t s) {
   auto up = [](size_t n) { return (n + 255) / 256 * 256; };
   const size_t at_kp = 256, at_snap = at_kp + up(sizeof(KParams));
   const size_t n_head = at_snap + up(n_snap * sizeof(ResSnap));
+  const RelaxedCapture relaxed;   // (a run allocated nothing before it had a workspace)
   int dev = 0;
   HIPCHK(hipGetDevice(&dev));
   if (!res_hold(dev)) return 1;

@@ -216,3 +216,23 @@ def test_a_momentary_holder_costs_the_resident_step_for_its_time_only(fake):
     rc, log = run(p)
     assert rc == 0 and resident(log) and variant(p) == 9, log
     """)
+
+
+def test_a_run_allocates_nothing_that_ends_a_capture_elsewhere(fake):
+    """The first resident run's allocations are made in the relaxed capture
+    mode, and the thread's own mode is back afterwards; a run on a stream
+    under capture allocates nothing and takes the two-pass step."""
+    fake("""
+    p = create(desc((12, 13, 14), planes=2))
+    F.fake_capture(1)
+    rc, log = run(p, n=5)
+    assert rc == 0 and two_pass(log) and not resident(log)
+    F.fake_capture(0)
+    live = F.fake_live()
+    rc, log = run(p)
+    assert rc == 0 and resident(log) and F.fake_live() > live
+    assert not any(l[0].startswith("malloc") for l in log), log
+    F.fake_clear()
+    create(desc((4, 4, 4)))
+    assert "malloc-global" in F.fake_log().decode()
+    """)
