@@ -234,7 +234,7 @@ int rfxh_kernel_time_ms(rfxh_plan* plan, int which, double* avg_ms, int64_t* cou
  * set; grids cut into at most one block per compute unit, about a million
  * cells, one mu_r, kappa = 1 in the CPML, no dispersion or per-component
  * eps, at most 32 planes, monitors
- * and NTFF faces in all and 256 point operations a block).  It is the
+ * and NTFF faces in all, with samples of 16 MB a step, and 256 point operations a block).  It is the
  * default of every plan that fits; runs of fewer than 4 steps, timed runs
  * and runs on a stream under capture, or with a mask of fewer compute units than
  * there are blocks, take the two-pass step instead.  Its

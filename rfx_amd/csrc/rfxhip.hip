@@ -4831,6 +4831,18 @@ void res_release(int dev) {
   d.sock = -1;
 }
 
+// Bytes a step stages for the folds, and the rings' size in all: a launch runs
+// as many steps as they hold, so that its fixed cost (about 10 us) is a few
+// percent of its steps.
+constexpr long long kResRing = 64LL << 20;
+constexpr int kResFew = 4;      // fewer steps a launch than this are not worth one
+long long res_step_bytes(const rfxh_plan* pl) {
+  long long b = 0;
+  for (const PlaneParams& q : pl->planes) b += 4LL * q.n1 * q.n2;
+  for (const FluxParams& q : pl->fluxes) b += 16LL * q.n1 * q.n2;
+  return b;
+}
+
 // Cuts the grid into at most one block per compute unit, the cheapest cut by
 // a model of the step (microseconds): two exchanges, 0.55 + 0.65 per
 // thousand words of a workgroup, and 0.12 per plane and wavefront of a SIMD
@@ -4838,7 +4850,7 @@ void res_release(int dev) {
 // not cover keep rp.ok false: dispersive poles, per-component eps, several
 // mu_r (a load of ch in the loop would wait for the mailbox stores), CPML
 // slabs that overlap or whose kappa is not 1, more snapshots or point operations in a block than it
-// stages, grids of more blocks than compute units.
+// stages, snapshots of which the rings hold only a few steps, grids of more blocks than compute units.
 void res_choose(rfxh_plan* pl, const std::vector<rfxh_point_op>& ops,
                 const std::vector<float>& km1) {
   ResPlan& r = pl->rp;
@@ -4850,6 +4862,7 @@ void res_choose(rfxh_plan* pl, const std::vector<rfxh_point_op>& ops,
   const long long cells = (long long)kp.nx * kp.plane;
   if (pl->n_pole > 0 || pl->aniso || kp.ch_all <= 0.f || cells > (long long)cus * 8 * kResThreads) return;
   if (pl->planes.size() + pl->fluxes.size() > (size_t)kResSnaps) return;
+  if (kResFew * res_step_bytes(pl) > kResRing) return;
   const int N[3] = {kp.nx, kp.ny, kp.nz};
   for (int a = 0; a < 3; ++a)
     if (kp.cn[2 * a] + kp.cn[2 * a + 1] > N[a]) return;
@@ -4911,13 +4924,8 @@ struct RelaxedCapture {
 int res_setup(rfxh_plan* pl, hipStream_t s) {
   ResPlan& r = pl->rp;
   const size_t n_box = 4 * (size_t)r.ntx * r.nty * r.ntz * res_words(r.nx) * sizeof(u64);
-  long long per_step = 0;
-  for (const PlaneParams& q : pl->planes) per_step += 4LL * q.n1 * q.n2;
-  for (const FluxParams& q : pl->fluxes) per_step += 16LL * q.n1 * q.n2;
-  // rings of about 64 MiB in all: a launch's fixed cost (about 10 us) is
-  // then a few percent of its steps
-  const long long chunk = per_step ? std::min<long long>(4096, std::max<long long>(16, (64LL << 20) / per_step))
-                                   : (1LL << 20);
+  const long long per_step = res_step_bytes(pl);
+  const long long chunk = per_step ? std::min<long long>(4096, kResRing / per_step) : (1LL << 20);
   const long long rows = std::min<long long>(chunk, std::max<long long>(1, pl->max_steps));
   const size_t n_snap = pl->planes.size() + pl->fluxes.size();
   // after the mailboxes: the stop word, the parameters, the snapshots, the rings
@@ -5112,7 +5120,7 @@ int stream_cus(hipStream_t s) {
 // outweighs.  Nor on a stream with fewer compute units than the grid has
 // blocks: LDS holds one block a unit, so the last ones would never start.
 bool res_takes(rfxh_plan* pl, hipStream_t s, int64_t n_steps) {
-  if (!pl->res || !pl->rp.ok || pl->timing || n_steps < 4) return false;
+  if (!pl->res || !pl->rp.ok || pl->timing || n_steps < kResFew) return false;
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(s, &st) != hipSuccess) {
     (void)hipGetLastError();

@@ -236,3 +236,31 @@ def test_a_run_allocates_nothing_that_ends_a_capture_elsewhere(fake):
     create(desc((4, 4, 4)))
     assert "malloc-global" in F.fake_log().decode()
     """)
+
+
+def test_resident_workspace_is_bounded(fake):
+    """However many samples a step stages, the workspace stays within 100 MB:
+    the rings hold fewer steps, and where they would hold fewer than four the
+    plan does not take the resident step."""
+    fake("""
+    for n, faces, res in (((8, 352, 352), 32, True), ((8, 352, 352), 7, True),
+                          ((3, 352, 352), 32, True), ((8, 352, 352), 1, True),
+                          ((8, 352, 352), -32, False),
+                          ((8, 352, 352), -8, True)):
+        d = desc(n, steps=100, planes=max(faces, 0), mem=1)
+        for q in range(faces):
+            d.planes[q].index = q % n[0]
+        if faces < 0:                                # flux monitors: four samples a point
+            fr = np.array([1e9])
+            fl = (L.Flux * -faces)()
+            for f in fl:
+                f.axis, f.index, f.lo1, f.n1, f.lo2, f.n2, f.n_freq = 0, 1, 0, n[1], 0, n[2], 1
+                f.freqs, f.d_acc = fr.ctypes.data_as(C.POINTER(C.c_double)), buf(8)
+            d.n_flux, d.flux = -faces, fl
+        p = create(d)
+        assert (variant(p) == 9) == res, (n, faces)
+        F.fake_peak()
+        rc, log = run(p, n=100)
+        assert rc == 0 and bool(resident(log)) == res, (n, faces)
+        assert F.fake_peak() <= 100e6, (n, faces)
+    """)
