@@ -5903,6 +5903,14 @@ static void tb_choose(rfxh_plan* pl, bool free_choice) {
   if (!pl->tb_auto) (void)hipGetLastError();   // (no memory for the sweep's scratch)
 }
 
+static void drop_graphs(rfxh_plan* pl) {
+  for (int g = 0; g < 2; ++g)
+    if (pl->graph_exec[g]) {
+      (void)hipGraphExecDestroy(pl->graph_exec[g]);
+      pl->graph_exec[g] = nullptr;
+    }
+}
+
 int rfxh_set_variant(rfxh_plan* pl, int kernel, int param) {
   if (!pl || kernel < 0 || kernel > 9) return fail(RFXH_EINVAL, "bad variant");
   if (kernel == 9) {
@@ -5912,6 +5920,10 @@ int rfxh_set_variant(rfxh_plan* pl, int kernel, int param) {
                                "without poles, per-component eps or several mu_r");
     pl->res = true;
     pl->res_out = false;
+    if (pl->tb || pl->fused) {   // what it does not take goes to the two-pass step
+      pl->tb = pl->fused = pl->march = pl->wmarch = false;
+      drop_graphs(pl);
+    }
     return RFXH_OK;
   }
   if (kernel == 8) {
@@ -5949,11 +5961,7 @@ int rfxh_set_variant(rfxh_plan* pl, int kernel, int param) {
     pl->res = false;
     pl->tb_seg = param;
     pl->fused = pl->march = pl->wmarch = false;
-    for (int g = 0; g < 2; ++g)
-      if (pl->graph_exec[g]) {
-        (void)hipGraphExecDestroy(pl->graph_exec[g]);
-        pl->graph_exec[g] = nullptr;
-      }
+    drop_graphs(pl);
     return RFXH_OK;
   }
   const bool pingpong = kernel == 1 || kernel == 2 || kernel == 3 || kernel == 7;
@@ -5989,11 +5997,7 @@ int rfxh_set_variant(rfxh_plan* pl, int kernel, int param) {
   pl->march = kernel == 2 || kernel == 3;
   pl->wmarch = kernel == 7;
   pl->tb = pl->res = false;
-  for (int g = 0; g < 2; ++g)
-    if (pl->graph_exec[g]) {
-      (void)hipGraphExecDestroy(pl->graph_exec[g]);
-      pl->graph_exec[g] = nullptr;
-    }
+  drop_graphs(pl);
   return RFXH_OK;
 }
 

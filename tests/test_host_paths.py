@@ -264,3 +264,25 @@ def test_resident_workspace_is_bounded(fake):
         assert rc == 0 and bool(resident(log)) == res, (n, faces)
         assert F.fake_peak() <= 100e6, (n, faces)
     """)
+
+
+def test_what_the_resident_step_leaves_takes_the_two_pass_step(fake):
+    """Short and timed runs of a plan set to the resident step, whatever it was
+    set to before."""
+    fake("""
+    for before in (1, 2, 3, 4, 7, 8):
+        p = create(desc((12, 13, 14)))
+        L.check(lib.rfxh_set_variant(p, before, 0))
+        rc, log = run(p, n=3)
+        assert rc == 0
+        cur = lib.rfxh_state_set(p)
+        L.check(lib.rfxh_set_variant(p, 9, 0))
+        rc, log = run(p, n=3)
+        assert rc == 0 and len(two_pass(log)) == 3 and not resident(log), (before, log)
+        L.check(lib.rfxh_set_timing(p, 1))
+        rc, log = run(p)
+        assert rc == 0 and two_pass(log) and lib.rfxh_state_set(p) == cur, (before, log)
+        L.check(lib.rfxh_set_timing(p, 0))
+        rc, log = run(p)
+        assert rc == 0 and resident(log) and lib.rfxh_state_set(p) == cur
+    """)
