@@ -2550,6 +2550,9 @@ __global__ __launch_bounds__(256) void k_flux_flush(FluxParams q) {
 constexpr int kFFRows = 32;    // rows of a segment (their a: 32 KB of LDS)
 constexpr int kFFCol = 8;      // columns of a wavefront at a time
 constexpr int kFFW = 4;        // wavefronts of a workgroup
+// bytes of a split's partial sums: freeing a block of 128 MiB takes 250 us, of
+// 64 MiB 10 us
+constexpr long long kFFPart = 48LL << 20;
 
 struct FarFieldParams {
   const double2* acc[6];   // [4][nf][n1][n2] per face
@@ -2689,9 +2692,11 @@ __device__ __forceinline__ void ff_out(const FarFieldParams& q, int f, int d,
   q.e_phi[o] = make_double2(-g * b.y, g * b.x);     //  j g b
 }
 
-// PARTS: blockIdx.z = face * nseg + row segment, sums to part[z][f][t][n_dir];
-// otherwise the workgroup takes every face and row and writes the fields.
-template <bool PARTS>
+// PARTS: blockIdx.z = face * nseg + row segment, sums to part[z][f][t][n_dir]
+// (1: segments of at most kFFRows rows, 2: of any; the loop alone took 578 us
+// where a single pass takes 466); 0: the workgroup takes every face and row
+// and writes the fields.
+template <int PARTS>
 __global__ __launch_bounds__(kBX * kFFW) void k_far_field(FarFieldParams q, int seg_rows, int nseg,
                                                           double2* part) {
   __shared__ FFShared sh;
@@ -2714,7 +2719,11 @@ __global__ __launch_bounds__(kBX * kFFW) void k_far_field(FarFieldParams q, int 
     const int n1 = ax == 0 ? q.hi[1] - q.lo[1] : q.hi[0] - q.lo[0];
     clear();
     const int r0 = seg * seg_rows, r1 = min(n1, r0 + seg_rows);
-    if (r0 < r1) rows(ax, face & 1, r0, r1);
+    if (PARTS == 1) {
+      if (r0 < r1) rows(ax, face & 1, r0, r1);
+    } else {
+      for (int r = r0; r < r1; r += kFFRows) rows(ax, face & 1, r, min(r1, r + kFFRows));
+    }
     ff_reduce(sh, w, lane, S);
     if (w == 0 && d < q.n_dir) {
       double2* o = part + ((long long)blockIdx.z * q.nf + f) * 4 * q.n_dir + d;
@@ -6711,6 +6720,7 @@ static int far_field_setup(const rfxh_farfield_desc* dsc, int32_t n_theta, const
   for (int a = 0; a < 3; ++a) total += 2 * (size_t)dsc->n_axis[a];
   total = (total + 1) & ~(size_t)1;   // the extra space holds complex128: 16-byte aligned
   if (hipMalloc(blk, (total + extra) * sizeof(double)) != hipSuccess) {
+    (void)hipGetLastError();
     *blk = nullptr;
     return fail(RFXH_ENOMEM, "far field: device tables");
   }
@@ -6759,20 +6769,30 @@ int rfxh_ntff_far_field(const rfxh_farfield_desc* dsc, int32_t n_theta, const do
   double* extra = nullptr;
   // directions x frequencies that do not give four workgroups to each of 256
   // compute units: the faces and row segments of their own, as short as it
-  // takes (at least 4 rows, which a's sincos need)
+  // takes (at least 4 rows, which a's sincos need; at most the kFFRows that
+  // LDS holds, more where the sums of so many segments would pass kFFPart)
   const long long tiles = ((long long)n_theta * n_phi + kBX - 1) / kBX * std::max(dsc->n_freq, 0);
   int seg_rows = 0, nseg = 0;
   size_t n_part = 0;
   if (tiles < 1024) {
-    int n1 = 1;
-    for (int a = 0; a < 2; ++a) n1 = std::max(n1, dsc->hi[a] - dsc->lo[a]);
+    long long n1 = 1;
+    for (int a = 0; a < 2; ++a) n1 = std::max(n1, (long long)dsc->hi[a] - dsc->lo[a]);
     const long long want = (1024 + 6 * std::max<long long>(1, tiles) - 1) /
                            (6 * std::max<long long>(1, tiles));
-    seg_rows = (int)std::min<long long>(kFFRows, std::max<long long>(4, (n1 + want - 1) / want));
-    nseg = (n1 + seg_rows - 1) / seg_rows;
-    n_part = (size_t)6 * nseg * 4 * (size_t)std::max(dsc->n_freq, 0) * n_theta * n_phi * 2;
+    long long rows = std::min<long long>(kFFRows, std::max<long long>(4, (n1 + want - 1) / want));
+    const long long one = 6LL * 4 * std::max(dsc->n_freq, 0) * n_theta * n_phi * 2;   // of a segment
+    const long long most = std::max<long long>(1, kFFPart / 8 / std::max<long long>(1, one));
+    if ((n1 + rows - 1) / rows > most) rows = (n1 + most - 1) / most;
+    seg_rows = (int)rows;
+    nseg = (int)((n1 + rows - 1) / rows);
+    n_part = (size_t)(nseg * one);
   }
   int rc = far_field_setup(dsc, n_theta, theta, n_phi, phi, s, n_part, q, &blk, &extra);
+  if (rc == RFXH_ENOMEM && nseg) {
+    // no room for the sums: every face and row in one workgroup needs none
+    nseg = 0;
+    rc = far_field_setup(dsc, n_theta, theta, n_phi, phi, s, 0, q, &blk, nullptr);
+  }
   if (rc == RFXH_OK) {
     for (int face = 0; face < 6; ++face) q.acc[face] = reinterpret_cast<const double2*>(dsc->d_acc[face]);
     q.e_theta = reinterpret_cast<double2*>(e_theta);
@@ -6781,11 +6801,12 @@ int rfxh_ntff_far_field(const rfxh_farfield_desc* dsc, int32_t n_theta, const do
                  nseg ? 6u * (unsigned)nseg : 1u);
     if (nseg) {
       double2* part = reinterpret_cast<double2*>(extra);
-      hipLaunchKernelGGL(k_far_field<true>, g, dim3(kBX, kFFW), 0, s, q, seg_rows, nseg, part);
+      const auto kern = seg_rows > kFFRows ? k_far_field<2> : k_far_field<1>;
+      hipLaunchKernelGGL(kern, g, dim3(kBX, kFFW), 0, s, q, seg_rows, nseg, part);
       hipLaunchKernelGGL(k_far_field_sum, dim3((unsigned)((q.n_dir + 255) / 256), g.y), dim3(256),
                          0, s, q, nseg, part);
     } else {
-      hipLaunchKernelGGL(k_far_field<false>, g, dim3(kBX, kFFW), 0, s, q, 0, 0,
+      hipLaunchKernelGGL(k_far_field<0>, g, dim3(kBX, kFFW), 0, s, q, 0, 0,
                          (double2*)nullptr);
     }
     if (hipGetLastError() != hipSuccess) rc = fail(RFXH_EHIP, "far field: launch");
@@ -6814,8 +6835,7 @@ int rfxh_ntff_far_field_adjoint(const rfxh_farfield_desc* dsc, int32_t n_theta,
   double* gs = nullptr;
   // scratch: twelve complex sums per (frequency, direction), and the parts of
   // a split over the directions where the faces' tiles do not fill the device
-  // (at most 8 segments of at least 64 directions, and 48 MiB: freeing a
-  // block of 128 MiB takes 250 us, of 64 MiB 10 us)
+  // (at most 8 segments of at least 64 directions)
   const long long n_dir = (long long)n_theta * n_phi, nf = std::max(dsc->n_freq, 0);
   const size_t sums = (size_t)24 * (size_t)nf * (size_t)n_dir;
   FFAdjOut out;
@@ -6834,9 +6854,13 @@ int rfxh_ntff_far_field_adjoint(const rfxh_farfield_desc* dsc, int32_t n_theta,
   }
   long long nseg = tiles * nf > 0 ? (2048 + tiles * nf - 1) / (tiles * nf) : 1;
   nseg = std::min<long long>({nseg, 8, std::max<long long>(1, n_dir / 64),
-                              std::max<long long>(1, (48LL << 20) / (16 * std::max<long long>(1, out.total)))});
+                              std::max<long long>(1, kFFPart / (16 * std::max<long long>(1, out.total)))});
   const size_t extra = sums + (nseg > 1 ? (size_t)nseg * (size_t)out.total * 2 : 0);
   int rc = far_field_setup(dsc, n_theta, theta, n_phi, phi, s, extra, q, &blk, &gs);
+  if (rc == RFXH_ENOMEM && nseg > 1) {
+    nseg = 1;
+    rc = far_field_setup(dsc, n_theta, theta, n_phi, phi, s, sums, q, &blk, &gs);
+  }
   if (rc == RFXH_OK) {
     hipLaunchKernelGGL(k_far_field_adj_s, dim3((unsigned)((q.n_dir + 255) / 256), (unsigned)q.nf),
                        dim3(256), 0, s, q, reinterpret_cast<const double2*>(g_theta),
@@ -6957,7 +6981,7 @@ int rfxh_ntff_far_field_noalloc(const rfxh_farfield_desc* dsc, int32_t n_theta,
   q.eta0 = dsc->eta0;
   q.e_theta = reinterpret_cast<double2*>(e_theta);
   q.e_phi = reinterpret_cast<double2*>(e_phi);
-  hipLaunchKernelGGL(k_far_field<false>, dim3((unsigned)((n_dir + kBX - 1) / kBX),
+  hipLaunchKernelGGL(k_far_field<0>, dim3((unsigned)((n_dir + kBX - 1) / kBX),
                                               (unsigned)dsc->n_freq), dim3(kBX, kFFW), 0, s, q, 0,
                      0, (double2*)nullptr);
   if (hipGetLastError() != hipSuccess) return fail(RFXH_EHIP, "far field: launch");

@@ -286,3 +286,50 @@ def test_what_the_resident_step_leaves_takes_the_two_pass_step(fake):
         rc, log = run(p)
         assert rc == 0 and resident(log) and lib.rfxh_state_set(p) == cur
     """)
+
+
+@pytest.mark.parametrize("size, nf, n_theta, n_phi", [
+    ((480, 470, 300), 4, 181, 72),       # 816 direction tiles
+    ((1000, 990, 40), 4, 120, 133),
+    ((86, 85, 84), 4, 37, 72),
+    ((300, 300, 300), 1, 2, 3),
+])
+def test_far_field_scratch_is_bounded_and_dispensable(fake, size, nf, n_theta, n_phi):
+    """The transform's scratch stays within 48 MiB and the tables, forward and
+    reverse (whose own sums it cannot do without), and where the device has
+    room for those alone the transform runs without the rest."""
+    fake(f"""
+    size, nf, nt, nph = {size}, {nf}, {n_theta}, {n_phi}
+    th, ph, fr = (np.linspace(1.0, 2.0, k) for k in (nt, nph, nf))
+    ptr = lambda a: a.ctypes.data_as(C.POINTER(C.c_double))
+    tabs = [np.ones(s + 5) for s in size]
+    d = L.FarFieldDesc()
+    for a in range(3):
+        d.lo[a], d.hi[a], d.n_axis[a] = 2, 2 + size[a], size[a] + 5
+        d.pos[a] = d.width[a] = ptr(tabs[a])
+    d.n_freq, d.freqs, d.c0, d.eta0 = nf, ptr(fr), 3e8, 377.0
+    for f in range(6):
+        d.d_acc[f] = buf(1)
+    out = (C.c_void_p * 6)(*[buf(1)] * 6)
+    table = 8 * (9 * nt * nph + nf + 2 * sum(size) + 32)
+    sums = 8 * 24 * nf * nt * nph
+    def forward():
+        return lib.rfxh_ntff_far_field(C.byref(d), nt, ptr(th), nph, ptr(ph), buf(1), buf(1), None)
+    def reverse():
+        return lib.rfxh_ntff_far_field_adjoint(C.byref(d), nt, ptr(th), nph, ptr(ph), buf(1), buf(1),
+                                               C.cast(out, C.POINTER(C.c_void_p)), None)
+    for call, need, split in ((forward, table, "k_far_field_sum"),
+                              (reverse, table + sums, "k_far_field_adj_sum")):
+        F.fake_clear()
+        F.fake_peak()
+        assert call() == 0
+        log = F.fake_log().decode()
+        assert F.fake_peak() <= (48 << 20) + need, call
+        F.fake_limit(need)
+        F.fake_clear()
+        assert call() == 0, lib.rfxh_last_error()
+        assert split not in F.fake_log().decode() and "k_far_field" in F.fake_log().decode()
+        F.fake_limit(1)
+        assert call() == -3, lib.rfxh_last_error()
+        F.fake_limit(-1)
+    """)
