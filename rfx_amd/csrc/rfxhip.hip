@@ -2180,7 +2180,7 @@ __device__ __forceinline__ void col_e(const KParams& p, const PsiIO& ps, const S
   Poles pol;
   if (DISP)
     poles_load(ps, i0, j, k, m[0],
-               p.pole_ids ? ((p.pole_ids >> m[0]) & 1u) != 0
+               p.pole_ids ? m[0] < 64 && ((p.pole_ids >> m[0]) & 1u) != 0
                           : (__float_as_uint(gld(p.ecoef, (int)m[0]).w) & RFXH_POLES) != 0,
                pol);
 #pragma unroll
