@@ -5769,7 +5769,11 @@ int rfxh_run(rfxh_plan* pl, int64_t step0, int64_t n_steps, void* stream, int us
     return fail(RFXH_EINVAL, "steps outside the source/probe tables (max_steps)");
   if (int rc = res_status(pl)) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  hipLaunchKernelGGL(k_set_step, dim3(1), dim3(64), 0, s, pl->kp.step, (long long)step0);
+  // (timing samples of a default plan are of single steps, as they were)
+  const bool tb = pl->tb && !(pl->tb_auto && pl->timing);
+  const bool counts_up = n_steps > 0 && !tb && !pl->fused;   // (see advance)
+  hipLaunchKernelGGL(k_set_step, dim3(1), dim3(64), 0, s, pl->kp.step,
+                     (long long)step0 - (counts_up ? 1 : 0));
   dft_begin(pl, s, step0);
   HIPCHK(hipGetLastError());
   if (n_steps == 0) return RFXH_OK;
@@ -5782,10 +5786,8 @@ int rfxh_run(rfxh_plan* pl, int64_t step0, int64_t n_steps, void* stream, int us
     }
     pl->res_out = true;   // (this run alone: the holder may be gone at the next)
   }
-  // (timing samples of a default plan are of single steps, as they were)
-  if (pl->tb && !(pl->tb_auto && pl->timing)) return run_tb(pl, s, n_steps, use_graph);
+  if (tb) return run_tb(pl, s, n_steps, use_graph);
   const int flip = pl->fused ? 1 : 0;
-  if (!pl->fused) advance(pl, s, -1);
   // (the captured graphs of a plan with the sweep are the sweep's)
   if (!use_graph || pl->timing || pl->tb || n_steps < pl->graph_chunk) {
     // timing: sample up to kTimingSamples evenly spaced steps; the host does

@@ -333,3 +333,16 @@ def test_far_field_scratch_is_bounded_and_dispensable(fake, size, nf, n_theta, n
         assert call() == -3, lib.rfxh_last_error()
         F.fake_limit(-1)
     """)
+
+
+def test_launches_of_single_step_runs(fake):
+    """A run of one step is four launches (the step counter, H, E, the counter),
+    of n two-pass steps 2 n + 2, whatever the plan runs otherwise."""
+    fake("""
+    p = create(desc((12, 13, 14)))
+    for v in (0, 4, 9):
+        L.check(lib.rfxh_set_variant(p, v, 0))
+        for n in (1, 2, 3):
+            rc, log = run(p, n=n)
+            assert rc == 0 and len(log) == 2 * n + 2, (v, n, log)
+    """)
