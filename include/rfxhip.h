@@ -200,8 +200,9 @@ int rfxh_run(rfxh_plan* plan, int64_t step0, int64_t n_steps, void* stream, int 
  * seconds.  The run's fields, probe and port rows and accumulators are then NaN,
  * this call or the plan's next run (whichever comes first) returns RFXH_EHIP
  * once, and the plan takes the two-pass step until kernel 9 is set again.
- * RFXH_RESIDENT_DEAF in the environment of rfxh_plan_create makes every such wait
- * of the plan run out after some milliseconds (to test a caller's handling). */
+ * RFXH_RESIDENT_LACKING in the environment of rfxh_plan_create makes the plan's
+ * resident runs fail so, after some milliseconds: their last workgroup is left
+ * out (to test a caller's handling). */
 int rfxh_status(rfxh_plan* plan);
 
 /* With two field sets: which set (0 = d_f/d_psi, 1 = d_f2/d_psi2) holds the

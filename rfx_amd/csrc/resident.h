@@ -75,7 +75,6 @@ struct ResIO {
   u64* box;                         // mailboxes [phase][parity][workgroup][words]
   unsigned* stop;                   // set by a workgroup that gave up
   int spin;                         // polls before a wait gives up
-  unsigned skew;                    // 0 (tests: every other workgroup's tags are off by it)
   const ResSnap* snaps;
   int n_snap;
   int ty, tz, ntx, nty, ntz;        // tile rows, columns; tiles per axis
@@ -520,7 +519,7 @@ __global__ __launch_bounds__(kResThreads) void k_resident(const KParams* __restr
   __syncthreads();
 
   bool bad = false;
-  unsigned tag = io.tag0 + ((wg & 1) ? io.skew : 0u);
+  unsigned tag = io.tag0;
   int w_base = 0, w_next = 0;           // first step of the staged source values, of the next ones
   for (int n = 0; n < n_steps; ++n) {
     const int par = n & 1;

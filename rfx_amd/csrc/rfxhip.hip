@@ -4245,7 +4245,7 @@ struct ResPlan {
   int dev = -1;                   // the device its workspace is on (-1: none yet)
   u64* box = nullptr;
   unsigned* stop = nullptr;
-  bool deaf = false;              // (tests: no workgroup hears another, every wait runs out)
+  bool lacking = false;           // (tests: the last workgroup is not launched)
   unsigned* status = nullptr;     // pinned: set when a run gave up (k_res_check)
   bool clear = false;             // `stop` is still set from a run that gave up
   ResSnap* snaps = nullptr;
@@ -5028,8 +5028,7 @@ int run_resident(rfxh_plan* pl, hipStream_t s, int64_t step0, int64_t n_steps) {
   io.n_port = kp.n_port;
   io.box = r.box;
   io.stop = r.stop;
-  io.spin = r.deaf ? kResLook : kResSpin;
-  io.skew = r.deaf ? 1u << 31 : 0u;
+  io.spin = r.lacking ? kResLook : kResSpin;
   io.snaps = r.snaps;
   io.n_snap = (int)r.rings.size();
   io.ty = r.ty;
@@ -5037,7 +5036,10 @@ int run_resident(rfxh_plan* pl, hipStream_t s, int64_t step0, int64_t n_steps) {
   io.ntx = r.ntx;
   io.nty = r.nty;
   io.ntz = r.ntz;
-  const dim3 grid((unsigned)(r.ntx * r.nty * r.ntz)), blk((unsigned)r.threads);
+  // (a workgroup less: its neighbours' waits for its words run out; the mailboxes
+  // of the others move together by as much, so all stay within the workspace)
+  const unsigned all = (unsigned)(r.ntx * r.nty * r.ntz);
+  const dim3 grid(r.lacking && all > 1 ? all - 1 : all), blk((unsigned)r.threads);
   if (r.clear) HIPCHK(hipMemsetAsync(r.stop, 0, sizeof(unsigned), s));
   r.clear = false;
   for (int64_t done = 0; done < n_steps;) {
@@ -5046,7 +5048,7 @@ int run_resident(rfxh_plan* pl, hipStream_t s, int64_t step0, int64_t n_steps) {
     io.step0 = step0 + done;
     if (r.tag > 0xffffffffu - 2u * (unsigned)cnt - 2u) {
       // the tags are used up: start them again over cleared mailboxes
-      HIPCHK(hipMemsetAsync(r.box, 0, 4LL * grid.x * res_words(r.nx) * sizeof(u64), s));
+      HIPCHK(hipMemsetAsync(r.box, 0, 4LL * all * res_words(r.nx) * sizeof(u64), s));
       r.tag = 0;
     }
     io.tag0 = r.tag;
@@ -5625,7 +5627,7 @@ int rfxh_plan_create(const rfxh_desc* d, rfxh_plan** out) {
   res_choose(pl, ops, km1);
   // the default of every grid that fits: 3-6 times the two-pass step's speed
   pl->res = pl->rp.ok && kname.empty();
-  pl->rp.deaf = std::getenv("RFXH_RESIDENT_DEAF") != nullptr;
+  pl->rp.lacking = std::getenv("RFXH_RESIDENT_LACKING") != nullptr;
   pl->tev.resize(4 * kTimingSamples);
   for (auto& e : pl->tev) {
     if (hipEventCreate(&e) != hipSuccess) return bail(fail(RFXH_EHIP, "hipEventCreate"));

@@ -115,6 +115,7 @@ def fake(tmp_path_factory):
         r = subprocess.run([sys.executable, "-c", PRELUDE + textwrap.dedent(body)], env=e,
                            capture_output=True, text=True, timeout=100)
         assert r.returncode == 0, r.stdout + r.stderr
+        return r.stdout
     return case
 
 
@@ -346,3 +347,13 @@ def test_launches_of_single_step_runs(fake):
             rc, log = run(p, n=n)
             assert rc == 0 and len(log) == 2 * n + 2, (v, n, log)
     """)
+
+
+def test_a_lacking_launch_is_one_workgroup_short(fake):
+    body = """
+    p = create(desc((40, 41, 42)))
+    rc, log = run(p)
+    print("BLOCKS", resident(log)[0][1])
+    """
+    assert int(fake(body).split("BLOCKS ")[1].split()[0]) == 1 + int(
+        fake(body, RFXH_RESIDENT_LACKING="1").split("BLOCKS ")[1].split()[0])

@@ -1,7 +1,7 @@
-"""A resident run whose workgroups give up waiting (forced by tags that
-no neighbour waits for and a small poll limit, so that every kernel still ends) hands out nothing that could be
-taken for a result: its fields, samples and accumulators are NaN, the
-error is raised, and the plan goes on with the two-pass step."""
+"""A resident run whose workgroups give up waiting (forced by leaving out the
+last one, with a small poll limit, so that every kernel still ends) hands out
+nothing that could be taken for a result: its fields, samples and accumulators
+are NaN, the error is raised, and the plan goes on with the two-pass step."""
 import numpy as np
 import pytest
 
@@ -31,9 +31,9 @@ def test_outputs_are_nan_and_the_error_is_raised(n, cpml, faces, steps, monkeypa
         per_step = faces * 16 * 73 * 73
         assert (64 << 20) // per_step < steps
     _, prob, _ = cases.to_sim(spec)._build_problem(steps, "run")
-    monkeypatch.setenv("RFXH_RESIDENT_DEAF", "1")
+    monkeypatch.setenv("RFXH_RESIDENT_LACKING", "1")
     dr = DeviceRun(prob, steps, "cuda")
-    monkeypatch.delenv("RFXH_RESIDENT_DEAF")
+    monkeypatch.delenv("RFXH_RESIDENT_LACKING")
     ref = DeviceRun(prob, steps, "cuda")
     at.set_variant(ref, 0, 1)
     ref.run()
@@ -58,6 +58,6 @@ def test_outputs_are_nan_and_the_error_is_raised(n, cpml, faces, steps, monkeypa
     dr.close()
     ref.close()
     # through the user's call: no result is handed out
-    monkeypatch.setenv("RFXH_RESIDENT_DEAF", "1")
+    monkeypatch.setenv("RFXH_RESIDENT_LACKING", "1")
     with pytest.raises(_lib.RfxHipError, match="gave up"):
         cases.to_sim(spec).run(n_steps=steps)
