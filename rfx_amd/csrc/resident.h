@@ -2,8 +2,7 @@
 // Included by rfxhip.hip inside its anonymous namespace.
 //
 // The two-pass step of a small grid is bound by its launches: 87 x 47 x 42
-// cells take 12.5-15.5 us a step (three graph nodes of 3-6 us), although their
-// fields are 4 MB.  Here every workgroup keeps a block of the grid for the
+// cells take 9.5 us a step (two graph nodes), although their fields are 4 MB.  Here every workgroup keeps a block of the grid for the
 // whole run -- fields, CPML memory and coefficients in registers, one thread
 // per (y, z) column of NX cells along x, the fields' copies for the y and z
 // neighbours in LDS -- and only the block's faces travel: the E of its low
@@ -27,9 +26,9 @@
 // worth nothing, so k_res_check, the last kernel of every run, then makes
 // all of its outputs NaN and tells the host.
 //
-// Measured (one step, two-pass column step -> resident): 87 x 47 x 42 cells
-// 15.5 -> 4.65 us, 41^3 without CPML 14 -> 3.05, 114 x 97 x 80 with a DFT plane
-// 30.5 -> 12.2.  What is left is the two exchanges (0.9-1.5 us each) and, from
+// Measured (one step, two-pass -> resident): 28^3 cells 8.7 -> 2.85 us, 87 x 47 x
+// 42 9.5 -> 4.6, 42^3 without CPML 7.9 -> 3.1, 113 x 97 x 80 16.5 -> 10.5, with a
+// DFT plane 21.1 -> 11.9.  What is left is the two exchanges (0.9-1.5 us each) and, from
 // 3000 cells a workgroup up, the arithmetic of the blocks in a corner of the
 // CPML, which the others wait for.  What mattered in the loop: no global
 // load outside the exchange (vector memory returns in order, so any other

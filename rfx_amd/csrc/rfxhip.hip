@@ -5625,7 +5625,8 @@ int rfxh_plan_create(const rfxh_desc* d, rfxh_plan** out) {
   std::vector<float> km1;
   for (int f = 0; f < 6; ++f) km1.insert(km1.end(), d->cpml_km1[f], d->cpml_km1[f] + d->cpml_n[f]);
   res_choose(pl, ops, km1);
-  // the default of every grid that fits: 3-6 times the two-pass step's speed
+  // the default of every grid that fits: 1.6 (113x97x80) to 3.1 (28^3) times the
+  // two-pass step's speed
   pl->res = pl->rp.ok && kname.empty();
   pl->rp.lacking = std::getenv("RFXH_RESIDENT_LACKING") != nullptr;
   pl->tev.resize(4 * kTimingSamples);
@@ -5897,8 +5898,7 @@ static PsiIO psi_io(const rfxh_plan* pl, int set) {
 
 // The default of very large grids: two steps a sweep move the state once
 // where two-pass steps move it four times (1636 against 2340 us a step at
-// 533^3, 1034 against 1368 at 450x440x430, 643 against 784 at 400x400x301, 481
-// against 536 at 320^3, 659 against 825 at 161x541x541, 922 against 1129 at
+// 533^3, 1034 against 1368 at 450x440x430, 643 against 784 at 400x400x301, 659 against 825 at 161x541x541, 922 against 1129 at
 // 1021x257x257).  It loses where rows or planes are short (521 against 257 at
 // 325x325x145), where the z slabs do not fit its edge tiles so that every tile
 // runs their code (1028 against 847 at 363^3 with 16 layers, 979 against 817 at
